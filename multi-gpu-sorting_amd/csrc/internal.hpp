@@ -70,6 +70,11 @@ const char* last_stage_names();
 size_t merge_temp_bytes(mgs_key kt, mgs_val vt, size_t na, size_t nb);
 int merge_dispatch(mgs_key kt, mgs_val vt, const void* ak, const void* av, size_t na, const void* bk, const void* bv,
                    size_t nb, void* ok, void* ov, void* temp, size_t temp_bytes, hipStream_t s);
+// The k-way merge of one or two runs (nb = 0 for one), status word first in
+// temp; portions as in multiway_dispatch (0: none).
+size_t merge_two_runs_temp_bytes(size_t total);
+int merge_two_runs(mgs_key kt, const void* a, size_t na, const void* b, size_t nb, void* out, void* temp,
+                   size_t temp_bytes, hipStream_t s, size_t portions, size_t* portion_end, hipEvent_t* portion_done);
 size_t multiway_temp_bytes(mgs_key kt, size_t k, size_t total);
 int multiway_dispatch(mgs_key kt, const void* const* runs, const size_t* lens, size_t k, void* out, void* temp,
                       size_t temp_bytes, hipStream_t s, size_t portions, size_t* portion_end,

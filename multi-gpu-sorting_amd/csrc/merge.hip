@@ -13,6 +13,7 @@
 
 #include "common.hpp"
 #include "internal.hpp"
+#include "radix_sort.hpp"
 
 namespace mgs {
 
@@ -57,11 +58,13 @@ __device__ __forceinline__ uint64_t corank(const Bits* a, uint64_t na, const Bit
 }
 
 // coarse[q]: the split of tile boundary q kCoarse, for q <= num_coarse.
+// status: a status word to clear, or NULL.
 template <int KT>
 __global__ void merge_coarse_kernel(const typename Codec<KT>::Bits* a, uint64_t na,
                                     const typename Codec<KT>::Bits* b, uint64_t nb, uint64_t* coarse,
-                                    uint64_t num_coarse) {
+                                    uint64_t num_coarse, uint32_t* status) {
   const uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q == 0 && status != nullptr) *status = 0;
   if (q > num_coarse) return;
   const uint64_t diag = std::min<uint64_t>(q * kCoarse * kMergeTile, na + nb);
   coarse[q] = corank<KT>(a, na, b, nb, diag);
@@ -82,14 +85,17 @@ __global__ void merge_partition_kernel(const typename Codec<KT>::Bits* a, uint64
   splits[i] = corank<KT>(a, na, b, nb, diag, lo, std::max(lo, hi));
 }
 
-template <int KT, typename V>
+// CHECK: report splits that do not fit the tile (unsorted input).
+template <int KT, typename V, bool CHECK>
 __global__ __launch_bounds__(kMergeBlock) void merge_tile_kernel(const typename Codec<KT>::Bits* __restrict__ a,
                                                                  const V* __restrict__ av, uint64_t na,
                                                                  const typename Codec<KT>::Bits* __restrict__ b,
                                                                  const V* __restrict__ bv, uint64_t nb,
                                                                  typename Codec<KT>::Bits* __restrict__ out,
                                                                  V* __restrict__ ov,
-                                                                 const uint64_t* __restrict__ splits) {
+                                                                 const uint64_t* __restrict__ splits,
+                                                                 uint64_t first_tile,
+                                                                 uint32_t* __restrict__ status) {
   using Bits = typename Codec<KT>::Bits;
   constexpr bool HV = kHasVal<V>;
   using VS = typename std::conditional<HV, V, uint32_t>::type;
@@ -97,14 +103,18 @@ __global__ __launch_bounds__(kMergeBlock) void merge_tile_kernel(const typename 
   __shared__ VS sv[HV ? kMergeTile : 1];
 
   const int tid = threadIdx.x;
-  const uint64_t d0 = (uint64_t)blockIdx.x * kMergeTile;
+  const uint64_t tile = first_tile + blockIdx.x;
+  const uint64_t d0 = tile * kMergeTile;
   const uint64_t d1 = std::min<uint64_t>(d0 + kMergeTile, na + nb);
   // Splits are monotone for sorted inputs; the clamps only keep unsorted
   // (invalid) input from indexing outside A and B.
-  const uint64_t a0 = min(splits[blockIdx.x], na);
-  const uint64_t a1 = min(max(splits[blockIdx.x + 1], a0), na);
+  const uint64_t a0 = min(splits[tile], na);
+  uint64_t a1 = min(max(splits[tile + 1], a0), na);
+  if constexpr (CHECK) a1 = min(a1, a0 + (d1 - d0));
   const uint64_t b0 = d0 - a0;
   const int cnt = (int)(d1 - d0);
+  if (CHECK && tid == 0 && (splits[tile + 1] < a0 || splits[tile + 1] - a0 > (uint64_t)cnt))
+    atomicOr(status, kStatusUnsorted);
   const int la = (int)(a1 - a0);
   const int lb = cnt - la;
 
@@ -200,6 +210,25 @@ __global__ __launch_bounds__(kMergeBlock) void merge_tile_kernel(const typename 
   }
 }
 
+// Scratch of the co-ranks of `total` outputs.
+inline size_t merge_splits_bytes(size_t total) {
+  const size_t tiles = (total + kMergeTile - 1) / kMergeTile;
+  return (tiles + 1 + (tiles + kCoarse - 1) / kCoarse + 1) * sizeof(uint64_t);
+}
+
+// The co-ranks of every tile boundary into `splits`.
+template <int KT>
+void merge_corank(const typename Codec<KT>::Bits* a, size_t na, const typename Codec<KT>::Bits* b, size_t nb,
+                  uint64_t* splits, uint32_t* status, hipStream_t s) {
+  const uint64_t tiles = (na + nb + kMergeTile - 1) / kMergeTile;
+  const uint64_t num_coarse = (tiles + kCoarse - 1) / kCoarse;
+  uint64_t* coarse = splits + tiles + 1;
+  merge_coarse_kernel<KT><<<(unsigned)((num_coarse + 1 + 255) / 256), 256, 0, s>>>(a, na, b, nb, coarse, num_coarse,
+                                                                                  status);
+  merge_partition_kernel<KT><<<(unsigned)((tiles + 1 + 255) / 256), 256, 0, s>>>(a, na, b, nb, splits, tiles, coarse,
+                                                                                   num_coarse);
+}
+
 template <int KT, int VT>
 int merge_typed(const void* ak, const void* av, size_t na, const void* bk, const void* bv, size_t nb, void* ok,
                 void* ov, void* temp, size_t temp_bytes, hipStream_t s) {
@@ -208,19 +237,49 @@ int merge_typed(const void* ak, const void* av, size_t na, const void* bk, const
   const size_t total = na + nb;
   if (total == 0) return MGS_OK;
   const uint64_t tiles = (total + kMergeTile - 1) / kMergeTile;
-  const uint64_t num_coarse = (tiles + kCoarse - 1) / kCoarse;
-  if (temp == nullptr || temp_bytes < (tiles + 1 + num_coarse + 1) * sizeof(uint64_t)) return MGS_ERR_TEMP_TOO_SMALL;
+  if (temp == nullptr || temp_bytes < merge_splits_bytes(total)) return MGS_ERR_TEMP_TOO_SMALL;
   uint64_t* splits = static_cast<uint64_t*>(temp);
-  uint64_t* coarse = splits + tiles + 1;
   const Bits* a = static_cast<const Bits*>(ak);
   const Bits* b = static_cast<const Bits*>(bk);
-  merge_coarse_kernel<KT><<<(unsigned)((num_coarse + 1 + 255) / 256), 256, 0, s>>>(a, na, b, nb, coarse, num_coarse);
-  merge_partition_kernel<KT><<<(unsigned)((tiles + 1 + 255) / 256), 256, 0, s>>>(a, na, b, nb, splits, tiles, coarse,
-                                                                                   num_coarse);
-  merge_tile_kernel<KT, V><<<(unsigned)tiles, kMergeBlock, 0, s>>>(
+  merge_corank<KT>(a, na, b, nb, splits, nullptr, s);
+  merge_tile_kernel<KT, V, false><<<(unsigned)tiles, kMergeBlock, 0, s>>>(
       a, static_cast<const V*>(av), na, b, static_cast<const V*>(bv), nb, static_cast<Bits*>(ok),
-      static_cast<V*>(ov), splits);
+      static_cast<V*>(ov), splits, 0, nullptr);
   return check_launch();
+}
+
+// The k-way merge's one or two runs: portion p is the tiles
+// [tiles p / portions, tiles (p + 1) / portions), so its end needs no wait.
+constexpr size_t kTwoRunsStatus = 256;  // the status word's place before the splits
+template <int KT>
+int two_runs_typed(const void* ak, size_t na, const void* bk, size_t nb, void* out, void* temp, size_t temp_bytes,
+                   hipStream_t s, size_t portions, size_t* portion_end, hipEvent_t* portion_done) {
+  using Bits = typename Codec<KT>::Bits;
+  const size_t total = na + nb;
+  if (temp == nullptr || temp_bytes < kTwoRunsStatus + merge_splits_bytes(total)) return MGS_ERR_TEMP_TOO_SMALL;
+  uint64_t* splits = reinterpret_cast<uint64_t*>(static_cast<char*>(temp) + kTwoRunsStatus);
+  const Bits* a = static_cast<const Bits*>(ak);
+  const Bits* b = static_cast<const Bits*>(bk);
+  merge_corank<KT>(a, na, b, nb, splits, static_cast<uint32_t*>(temp), s);
+  const uint64_t tiles = (total + kMergeTile - 1) / kMergeTile;
+  const size_t parts = std::max<size_t>(portions, 1);
+  for (size_t p = 0; p < parts; ++p) {
+    const uint64_t first = tiles * p / parts, end = tiles * (p + 1) / parts;
+    if (end > first)
+      merge_tile_kernel<KT, NoVal, true><<<(unsigned)(end - first), kMergeBlock, 0, s>>>(
+          a, nullptr, na, b, nullptr, nb, static_cast<Bits*>(out), nullptr, splits, first,
+          static_cast<uint32_t*>(temp));
+    const int rc = check_launch();
+    if (rc != MGS_OK) return rc;
+    if (portions > 0) {
+      portion_end[p] = (size_t)std::min<uint64_t>(end * kMergeTile, total);
+      if (portion_done) {
+        const int er = record_hip(hipEventRecord(portion_done[p], s));
+        if (er != MGS_OK) return er;
+      }
+    }
+  }
+  return MGS_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -321,8 +380,7 @@ int swap_bytes(void* a, void* b, size_t n, int bytes, hipStream_t s) {
 
 size_t merge_temp_bytes(mgs_key kt, mgs_val vt, size_t na, size_t nb) {
   if (key_bytes(kt) < 0 || val_bytes(vt) < 0) return 0;
-  const size_t tiles = (na + nb + kMergeTile - 1) / kMergeTile;
-  return (tiles + 1 + (tiles + kCoarse - 1) / kCoarse + 1) * sizeof(uint64_t);
+  return merge_splits_bytes(na + nb);
 }
 
 int merge_dispatch(mgs_key kt, mgs_val vt, const void* ak, const void* av, size_t na, const void* bk, const void* bv,
@@ -343,6 +401,21 @@ int merge_dispatch(mgs_key kt, mgs_val vt, const void* ak, const void* av, size_
     case MGS_KEY_F64: MGS_MERGE_V(MGS_KEY_F64)
   }
 #undef MGS_MERGE_V
+  return MGS_ERR_BAD_TYPE;
+}
+
+size_t merge_two_runs_temp_bytes(size_t total) { return kTwoRunsStatus + merge_splits_bytes(total); }
+
+int merge_two_runs(mgs_key kt, const void* a, size_t na, const void* b, size_t nb, void* out, void* temp,
+                   size_t temp_bytes, hipStream_t s, size_t portions, size_t* portion_end, hipEvent_t* portion_done) {
+  switch (kt) {
+    case MGS_KEY_U32: return two_runs_typed<MGS_KEY_U32>(a, na, b, nb, out, temp, temp_bytes, s, portions, portion_end, portion_done);
+    case MGS_KEY_U64: return two_runs_typed<MGS_KEY_U64>(a, na, b, nb, out, temp, temp_bytes, s, portions, portion_end, portion_done);
+    case MGS_KEY_I32: return two_runs_typed<MGS_KEY_I32>(a, na, b, nb, out, temp, temp_bytes, s, portions, portion_end, portion_done);
+    case MGS_KEY_I64: return two_runs_typed<MGS_KEY_I64>(a, na, b, nb, out, temp, temp_bytes, s, portions, portion_end, portion_done);
+    case MGS_KEY_F32: return two_runs_typed<MGS_KEY_F32>(a, na, b, nb, out, temp, temp_bytes, s, portions, portion_end, portion_done);
+    case MGS_KEY_F64: return two_runs_typed<MGS_KEY_F64>(a, na, b, nb, out, temp, temp_bytes, s, portions, portion_end, portion_done);
+  }
   return MGS_ERR_BAD_TYPE;
 }
 

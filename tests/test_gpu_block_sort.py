@@ -1,0 +1,78 @@
+"""The workgroup sort in LDS (block_sort.hpp) through the entry points that
+use it: sizes at the edges of its item slots and pieces, keys whose top
+differing bits tie (neighbour fix-up, and the passes over all bits where the
+ties are long), bit for bit against the oracle."""
+import numpy as np
+import pytest
+
+import pyoracle as O
+from helpers import KEY_NAME, from_dev, random_keys, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mg():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import mgsort
+    return mgsort
+
+
+def tied_keys(kt, n, rng, dist):
+    """uniform; pairs: every key about twice; clustered: 5 far apart values
+    plus small offsets, so that the top 18 differing bits leave long groups in
+    disorder; lone: clustered with one key at the bottom of the range."""
+    if dist == "uniform":
+        return random_keys(kt, n, rng)
+    bd = O.BITS_DTYPE[kt]
+    nbits = 32 if bd == np.uint32 else 64
+    if dist == "pairs":
+        pool = random_keys(kt, max(n // 2, 1), rng, "nonneg")
+        return pool[rng.integers(0, pool.size, size=n)]
+    top = rng.integers(0, 2**16, size=5).astype(np.uint64)[rng.integers(0, 5, size=n)] << np.uint64(nbits - 20)
+    k = (top | rng.integers(0, 2**11, size=n).astype(np.uint64)).astype(bd)
+    if dist == "lone":
+        k[n // 2] = 0
+    return k
+
+
+@pytest.mark.parametrize("kt,k", [(O.K_U32, 3), (O.K_F32, 5), (O.K_I32, 40), (O.K_U64, 4), (O.K_U64, 9), (O.K_F64, 12),
+                                  (O.K_I64, 100)], ids=lambda v: str(v))
+@pytest.mark.parametrize("dist", ["uniform", "pairs", "clustered", "lone"])
+@pytest.mark.parametrize("total", [1, 511, 513, 8191, 8193, 70_001, 400_000])
+def test_multiway_pieces(mg, kt, k, dist, total):
+    import torch
+    rng = np.random.default_rng(total + 11 * k + kt)
+    cuts = np.sort(rng.integers(0, total + 1, size=k - 1))
+    lens = np.diff(np.concatenate([[0], cuts, [total]]))
+    keys = tied_keys(kt, total, rng, dist)
+    runs, at = [], 0
+    for n in lens:
+        r = keys[at:at + n]
+        runs.append(np.ascontiguousarray(r[np.argsort(O.encode(kt, r), kind="stable")]))
+        at += n
+    expect = O.sort(kt, np.concatenate(runs))[0]
+    out = torch.empty(total, dtype=to_dev(expect).dtype, device="cuda")
+    temp = mg.temp_buffer(mg.lib.mgs_multiway_merge_temp_bytes(kt, k, total), "cuda")
+    mg.multiway_merge(KEY_NAME[kt], [to_dev(r) for r in runs], out, temp=temp)
+    assert mg.temp_status(temp) == 0
+    assert np.array_equal(from_dev(out, expect.dtype), expect)
+
+
+@pytest.mark.parametrize("lens", [(1,), (3840,), (3841, 0), (0, 3839), (100_003, 77)], ids=str)
+@pytest.mark.parametrize("portions", [0, 1, 5])
+def test_one_or_two_runs(mg, lens, portions):
+    """One or two runs take the merge path, with the stretches' ends on its
+    tile boundaries."""
+    import torch
+    rng = np.random.default_rng(sum(lens))
+    runs = [np.sort(random_keys(O.K_U32, n, rng, "lowbits")) for n in lens]
+    expect = np.sort(np.concatenate(runs))
+    out = torch.empty(expect.size, dtype=torch.int32, device="cuda")
+    temp = mg.temp_buffer(mg.lib.mgs_multiway_merge_temp_bytes(O.K_U32, len(lens), expect.size), "cuda")
+    ends = mg.multiway_merge("u32", [to_dev(r) for r in runs], out, temp=temp, portions=portions)
+    assert mg.temp_status(temp) == 0
+    assert portions == 0 or (len(ends) == portions and ends[-1] == expect.size and ends == sorted(ends))
+    assert np.array_equal(from_dev(out, np.uint32), expect)
