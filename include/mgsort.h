@@ -146,9 +146,11 @@ int mgs_sort_timed(mgs_key kt, mgs_val vt,
  * `stream` and returns MGS_PATH_SMALL (one workgroup in LDS, no scratch),
  * MGS_PATH_LSD (onesweep LSD passes) or MGS_PATH_THREE_PASS (the MSD pass,
  * the bucket pass and the LDS sort of sub-buckets, tried for 4-byte keys
- * alone of 2^23 to 3 * 2^24 keys and of 2^29 keys and more; it hands over to
- * the LSD passes when the key distribution does not suit it), or a negative
- * status. */
+ * alone of 2^23 to 3 * 2^24 keys and of 2^29 keys and more, for 8-byte
+ * integer keys from 2^22 and 4-byte integer keys with payloads from 2^24
+ * records up to about 2^28; it hands over to the LSD passes when the key
+ * distribution does not suit it, and wider records take the LSD passes when
+ * temp only fits these), or a negative status. */
 enum { MGS_PATH_SMALL = 1, MGS_PATH_LSD = 2, MGS_PATH_THREE_PASS = 3 };
 int mgs_sort_path(mgs_key kt, mgs_val vt, size_t n, const void* temp, size_t temp_bytes, void* stream);
 

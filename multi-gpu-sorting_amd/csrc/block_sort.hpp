@@ -2,25 +2,44 @@
 // and LDS (shared by the kernels whose pieces fit one workgroup).
 //
 // The caller gives the smallest and largest encoded key.  Their distance says
-// how many low bits of enc(key) - smallest differ at all; the sort takes at
-// most two LSD passes of 9 bits over the top 18 of these (the window), and
-// the write-out puts the few records that share a window value in order by
-// comparing neighbours.  Two passes leave random keys in groups of one or two
-// (8192 keys, 262144 window values), so 4-byte and 8-byte keys alike cost two
-// passes whatever their width.  A group longer than kTieReach records that
-// are not all equal would make the comparisons quadratic: the workgroup then
-// takes the passes over all differing bits instead.
+// how many low bits of a key's distance to the smallest differ at all; the
+// sort takes at most three LSD passes of 9 bits over the top 27 of these (the
+// window).  Among 4096 random keys one pair in a workgroup of 16 shares a
+// window value, so 4-byte and 8-byte keys alike cost two or three passes; the
+// write-out compares neighbours, and a workgroup that finds a record above
+// its successor puts the records that share a window value in order by
+// looking around each.  A group longer than kTieReach records that are not
+// all equal would make that quadratic: the workgroup then takes the passes
+// over all differing bits instead.
+//
+// Measured in the local sort of 2^28 u64 keys (batches of 4096, two
+// workgroups of 512 threads per CU): moving the records through registers
+// alone 0.93 ms, with two passes 1.15 ms; two passes and the look around
+// every record (the window of 18 bits leaves 1.6% of them in groups) took
+// 1.75 ms.
 #pragma once
 
 #include <type_traits>
+#include <utility>
 
 #include "radix_device.hpp"
 
 namespace mgs {
 
+// f(0), ..., f(N - 1) with constant arguments.  (Item loops that the compiler
+// only unrolls late leave the item arrays as register vectors of 16 or 32,
+// which spill.)
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_each(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_each(static_cast<F&&>(f), std::make_integer_sequence<int, N>{});
+}
+
 // Records a thread looks at on each side of its own in the write-out.
 constexpr uint32_t kTieReach = 16;
-
 // LDS counter rows of the 9-bit digits, one per wavefront.  The row stride
 // puts the two threads that scan one digit's 16 rows on different banks.
 // (16-bit counters, two to a word, halve the rows but measured 4% slower:
@@ -92,7 +111,7 @@ __device__ __forceinline__ int bit_width(Bits x) {
     return x ? 32 - __builtin_clz(x) : 0;
 }
 
-// The value of the lane below (lane 0: its own) and above (lane 63: its own).
+// The value of the lane below (lane 0: its own).
 template <typename Bits>
 __device__ __forceinline__ Bits lane_below(Bits x) {
   uint32_t lo = (uint32_t)x;
@@ -104,16 +123,17 @@ __device__ __forceinline__ Bits lane_below(Bits x) {
   }
   return (Bits)lo;
 }
-template <typename Bits>
-__device__ __forceinline__ Bits lane_above(Bits x) {
-  uint32_t lo = (uint32_t)x;
-  lo = (uint32_t)__builtin_amdgcn_update_dpp((int)lo, (int)lo, 0x130, 0xf, 0xf, false);  // wave_shl:1
-  if constexpr (sizeof(Bits) == 8) {
-    uint32_t hi = (uint32_t)(x >> 32);
-    hi = (uint32_t)__builtin_amdgcn_update_dpp((int)hi, (int)hi, 0x130, 0xf, 0xf, false);
-    return ((Bits)hi << 32) | lo;
+// The padding key of block_sort: not below any key bounded by mx.  (No float
+// has the image just below +0.0's: -0.0 shares +0.0's, and dec() of it would
+// land above mx.)
+template <int KT>
+__device__ __forceinline__ typename Codec<KT>::Bits block_pad(typename Codec<KT>::Bits mx) {
+  using Bits = typename Codec<KT>::Bits;
+  if constexpr (KT == MGS_KEY_F32 || KT == MGS_KEY_F64) {
+    constexpr Bits zero = Bits(1) << (sizeof(Bits) * 8 - 1);  // enc(+0.0)
+    if (mx == zero - 1) mx = zero - 2;
   }
-  return (Bits)lo;
+  return Codec<KT>::dec(mx);
 }
 
 // Items per thread in use for m records, and the position of a thread's item
@@ -130,7 +150,7 @@ __device__ __forceinline__ uint32_t block_first(uint32_t nit) {
 
 // Sorts the block's m records (1 <= m <= BLOCK * IPT) stably by enc(key) and
 // writes them to kout[0, m) (and vout).  mn and mx bound every enc(key).
-// Item slots beyond the m records hold the key dec(mx) on entry: padding
+// Item slots beyond the m records hold block_pad(mx) on entry: padding
 // behind the last record and not below any, so every pass leaves it there
 // and the passes need no bounds checks.  The counter rows are clear on entry
 // and on return; the caller puts a barrier between two calls.
@@ -142,167 +162,177 @@ __device__ __forceinline__ void block_sort(BlockSortSmem<typename Codec<KT>::Bit
                                            typename Codec<KT>::Bits* kout, V* vout) {
   using Bits = typename Codec<KT>::Bits;
   using R = BlockRows<BLOCK>;
+  using VS = typename BlockSortSmem<Bits, V, BLOCK, IPT>::VS;
   constexpr bool HV = kHasVal<V>;
+  constexpr uint32_t TILE = (uint32_t)BLOCK * IPT;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), w = (int)readfirstlane((uint32_t)(tid / kWave));
   m = readfirstlane(m);
   const uint32_t nit = block_items<BLOCK>(m), wb = block_first<BLOCK>(nit);
+  // The window: the bits from `low` on of the distance to mn rounded down to
+  // a multiple of 2^low, so that two keys share a window value exactly if
+  // they agree from bit `low` on; at most three digits.
+  constexpr int kWin = 3 * kBlockDigitBits;
   const int bits = bit_width<Bits>(mx - mn);
+  int low = bits > kWin ? bits - kWin : 0;
+  if (low > 0 && ((mx >> low) - (mn >> low)) >> kWin) ++low;
+  const uint32_t wbase = (uint32_t)(mn >> low);
+  const int wbits = bit_width<uint32_t>((uint32_t)(mx >> low) - wbase);
   uint32_t* const ct = sm.off + w * R::kStride;
   auto reload = [&]() {
-#pragma unroll
-    for (int i = 0; i < IPT; ++i)
+    static_for<IPT>([&](auto i) {
       if ((uint32_t)i < nit) {
         k[i] = sm.keys[wb + i * kWave];
         if constexpr (HV) v[i] = sm.vals[wb + i * kWave];
       }
+    });
   };
-  // one stable pass over `width` bits; the loops are apart so that every LDS
+  // one stable pass by digit(key); the loops are apart so that every LDS
   // operation of one is issued before the first wait
-  auto pass = [&](int shift, int width) {
-    const uint32_t mask = (1u << width) - 1u;
-    auto digit = [&](Bits x) { return (uint32_t)((Codec<KT>::enc(x) - mn) >> shift) & mask; };
+  auto pass = [&](auto digit) {
     uint32_t r[IPT];
     const uint32_t d0 = digit(k[0]);
     // runs of one digit (sorted input, duplicates, padding) would put the
     // lanes on one counter in turn: such a wavefront gives the first lane's
     // digit one atomic
     if (__popcll(ballot64(d0 == readfirstlane(d0))) >= 16) {
-#pragma unroll
-      for (int i = 0; i < IPT; ++i)
+      static_for<IPT>([&](auto i) {
         if ((uint32_t)i < nit) r[i] = rank_wave_atomic<true>(digit(k[i]), ct);
+      });
     } else {
-#pragma unroll
-      for (int i = 0; i < IPT; ++i)
+      static_for<IPT>([&](auto i) {
         if ((uint32_t)i < nit) r[i] = rank_wave_atomic<false>(digit(k[i]), ct);
+      });
     }
     __syncthreads();
     block_digit_offsets<BLOCK>(sm.off, sm.wsum);
-#pragma unroll
-    for (int i = 0; i < IPT; ++i)
+    static_for<IPT>([&](auto i) {
       if ((uint32_t)i < nit) r[i] += ct[digit(k[i])];
-#pragma unroll
-    for (int i = 0; i < IPT; ++i)
+    });
+    static_for<IPT>([&](auto i) {
       if ((uint32_t)i < nit) {
         sm.keys[r[i]] = k[i];
         if constexpr (HV) sm.vals[r[i]] = v[i];
       }
+    });
     block_clear_row<BLOCK>(sm.off);
     __syncthreads();
   };
-  const int low = bits > 2 * kBlockDigitBits ? bits - 2 * kBlockDigitBits : 0;
+  // byte offsets from the uniform base: one address register per store
+  auto store = [&](uint32_t p, Bits x) {
+    *reinterpret_cast<Bits*>(reinterpret_cast<char*>(kout) + p * (uint32_t)sizeof(Bits)) = x;
+  };
+  auto store_val = [&](uint32_t p, VS x) {
+    if constexpr (HV) *reinterpret_cast<V*>(reinterpret_cast<char*>(vout) + p * (uint32_t)sizeof(V)) = x;
+  };
   if (bits == 0) {  // equal keys: in order already
-#pragma unroll
-    for (int i = 0; i < IPT; ++i)
-      if ((uint32_t)i < nit) {
-        sm.keys[wb + i * kWave] = k[i];
-        if constexpr (HV) sm.vals[wb + i * kWave] = v[i];
+    static_for<IPT>([&](auto i) {
+      if ((uint32_t)i < nit && wb + i * kWave < m) {
+        store(wb + i * kWave, k[i]);
+        store_val(wb + i * kWave, v[i]);
       }
-    __syncthreads();
-  } else {
-    const int first = min(bits - low, kBlockDigitBits);
-    pass(low, first);
-    if (low + first < bits) {
+    });
+    return;
+  }
+  {
+    const int passes = (wbits + kBlockDigitBits - 1) / kBlockDigitBits;
+    const int width = (wbits + passes - 1) / passes;  // even digits
+    const uint32_t mask = (1u << width) - 1u;
+    for (int shift = 0;;) {
+      pass([&](Bits x) { return (((uint32_t)(Codec<KT>::enc(x) >> low) - wbase) >> shift) & mask; });
+      shift += width;
+      if (shift >= wbits) break;
       reload();
-      pass(low + first, bits - low - first);
     }
   }
-  // write-out: thread t has the records t, t + BLOCK, ...; with bits below
-  // the window a record moves left past the larger records of its group
-  // before it, right past the smaller ones after it
-#pragma unroll
-  for (int j = 0; j < IPT; ++j)
-    if ((uint32_t)j < nit) k[j] = sm.keys[j * BLOCK + tid];
-  if (low > 0) {
-    bool slow = false;
-    uint32_t np[IPT];
-    auto image = [&](uint32_t p) { return Codec<KT>::enc(sm.keys[p]) - mn; };
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) {
-      const uint32_t p = (uint32_t)(j * BLOCK + tid);
-      np[j] = p;
-      if ((uint32_t)j < nit) {
-        const Bits e = Codec<KT>::enc(k[j]) - mn;
-        Bits el = lane_below(e), er = lane_above(e);
-        if (lane == 0) el = p > 0 ? image(p - 1) : ~e;
-        if (lane == kWave - 1) er = p + 1 < m ? image(p + 1) : ~e;
-        const bool sl = ((e ^ el) >> low) == 0, sr = ((e ^ er) >> low) == 0;
-        const uint64_t left = ballot64(sl), right = ballot64(sr);
-        if ((left | right) != 0) {
-          // a group of two inside the wavefront needs no further look
-          const bool head = sr && !sl && lane < kWave - 1 && ((right >> 1 >> lane) & 1u) == 0;
-          const bool tail = sl && !sr && lane > 0 && ((left << 1 >> lane) & 1u) == 0;
-          if (head) np[j] = p + (er < e ? 1u : 0u);
-          if (tail) np[j] = p - (el > e ? 1u : 0u);
-          // a larger group needs a look if it reaches across the wavefront's
-          // ends or has a record above its successor
-          bool look = (sl || sr) && !head && !tail && p < m;
-          if (ballot64(look) != 0) {
-            const uint64_t down = ballot64(sl && el > e);
-            const uint64_t upto = ~left & ((2ull << lane) - 1u), after = ~left >> 1 >> lane;
-            const int a = 63 - (int)__builtin_clzll(upto | 1u);           // the group's first lane
-            const int b = after ? lane + (int)__builtin_ctzll(after) : 63;  // and its last
-            look = look && (upto == 0 || (after == 0 && right >> 63) || (down & ((2ull << b) - 1u) & ~((2ull << a) - 1u)) != 0);
-          }
-          if (look) {
-            bool differ = false, longer = false;
-            uint32_t at = p;
-            for (uint32_t r = 1; r <= p; ++r) {
-              const Bits x = image(p - r);
-              if (((x ^ e) >> low) != 0) break;
-              if (r > kTieReach) {
-                longer = true;
-                break;
-              }
-              differ |= x != e;
-              at -= x > e ? 1u : 0u;
-            }
-            for (uint32_t r = 1; p + r < m; ++r) {
-              const Bits x = image(p + r);
-              if (((x ^ e) >> low) != 0) break;
-              if (r > kTieReach) {
-                longer = true;
-                break;
-              }
-              differ |= x != e;
-              at += x < e ? 1u : 0u;
-            }
-            // a group that reaches further is in order if its records are
-            // all equal; otherwise the first different one on either side
-            // sees both the difference and the long run before it
-            slow |= differ && longer;
-            np[j] = at;
-          }
+  // write-out: thread t has the records t, t + BLOCK, ..., U loads in flight
+  constexpr uint32_t U = sizeof(Bits) + kValBytes<V> <= 8 ? 8 : 4;
+  auto write_out = [&](auto check) -> bool {
+    bool down = false;
+#pragma unroll 1
+    for (uint32_t j = 0; j < nit; j += U) {
+      Bits x[U], edge[U];
+      VS y[U];
+      static_for<(int)U>([&](auto u) {
+        const uint32_t p = min((j + u) * BLOCK + tid, TILE - 1);
+        x[u] = sm.keys[p];
+        if constexpr (check.value) edge[u] = sm.keys[lane == 0 ? max(p, 1u) - 1 : p];
+        if constexpr (HV) y[u] = sm.vals[p];
+      });
+      static_for<(int)U>([&](auto u) {
+        const uint32_t p = (j + u) * BLOCK + tid;
+        if constexpr (check.value) {
+          // the record before: the lane below's, or for the first lane the edge
+          const Bits b = lane_below(x[u]);
+          down |= p < m && Codec<KT>::enc(lane == 0 ? edge[u] : b) > Codec<KT>::enc(x[u]);
         }
+        if (p < m) {
+          store(p, x[u]);
+          store_val(p, y[u]);
+        }
+      });
+    }
+    return down;
+  };
+  if (low == 0) {
+    write_out(std::integral_constant<bool, false>{});
+    return;
+  }
+  const bool down = write_out(std::integral_constant<bool, true>{});
+  // (the stores below may follow another thread's to the same place)
+  auto stored = [] { __builtin_amdgcn_s_waitcnt(0); };
+  if (down) stored();
+  if (!__syncthreads_or(down ? 1 : 0)) return;
+  stored();
+  __syncthreads();
+  // a record moves left past the larger records of its group before it, right
+  // past the smaller ones after it
+  bool slow = false;
+  const Bits lim = Bits(1) << low;
+  auto image = [&](uint32_t p) { return Codec<KT>::enc(sm.keys[p]); };
+#pragma unroll 1
+  for (uint32_t j = 0; j < nit; ++j) {
+    const uint32_t p = j * BLOCK + tid;
+    if (p >= m) break;
+    const Bits raw = sm.keys[p], e = Codec<KT>::enc(raw);
+    bool differ = false, longer = false;
+    int by = 0;
+    for (uint32_t r = 1; r <= p; ++r) {
+      const Bits x = image(p - r);
+      if ((x ^ e) >= lim) break;
+      if (r > kTieReach) {
+        longer = true;
+        break;
       }
+      differ |= x != e;
+      by -= x > e ? 1 : 0;
     }
-    if (!__syncthreads_or(slow ? 1 : 0)) {
-#pragma unroll
-      for (int j = 0; j < IPT; ++j)
-        if ((uint32_t)j < nit && (uint32_t)(j * BLOCK + tid) < m) {
-          kout[np[j]] = k[j];
-          if constexpr (HV) vout[np[j]] = sm.vals[j * BLOCK + tid];
-        }
-      return;
+    for (uint32_t r = 1; p + r < m; ++r) {
+      const Bits x = image(p + r);
+      if ((x ^ e) >= lim) break;
+      if (r > kTieReach) {
+        longer = true;
+        break;
+      }
+      differ |= x != e;
+      by += x < e ? 1 : 0;
     }
-    for (int shift = 0; shift < bits; shift += kBlockDigitBits) {
-      reload();
-      pass(shift, min(bits - shift, kBlockDigitBits));
+    // a group that reaches further is in order if its records are all equal;
+    // otherwise the first different one on either side sees both the
+    // difference and the long run before it
+    slow |= differ && longer;
+    if (by != 0) {
+      store(p + (uint32_t)by, raw);
+      if constexpr (HV) store_val(p + (uint32_t)by, sm.vals[p]);
     }
-#pragma unroll
-    for (int j = 0; j < IPT; ++j)
-      if ((uint32_t)j < nit) k[j] = sm.keys[j * BLOCK + tid];
   }
-  if constexpr (HV) {
-#pragma unroll
-    for (int j = 0; j < IPT; ++j)
-      if ((uint32_t)j < nit) v[j] = sm.vals[j * BLOCK + tid];
+  stored();
+  if (!__syncthreads_or(slow ? 1 : 0)) return;
+  // all differing bits, from the present order
+  for (int shift = 0; shift < bits; shift += kBlockDigitBits) {
+    reload();
+    pass([&](Bits x) { return (uint32_t)((Codec<KT>::enc(x) - mn) >> shift) & ((1u << kBlockDigitBits) - 1u); });
   }
-#pragma unroll
-  for (int j = 0; j < IPT; ++j)
-    if ((uint32_t)j < nit && (uint32_t)(j * BLOCK + tid) < m) {
-      kout[j * BLOCK + tid] = k[j];
-      if constexpr (HV) vout[j * BLOCK + tid] = v[j];
-    }
+  write_out(std::integral_constant<bool, false>{});
 }
 
 }  // namespace mgs

@@ -53,6 +53,9 @@ inline int val_bytes(mgs_val vt) {
 }
 
 size_t sort_temp_bytes(mgs_key kt, mgs_val vt, size_t n);
+// The least scratch sort_dispatch takes: without the tables of the three-pass
+// path of wider records, which then sort by the LSD passes.
+size_t sort_least_temp_bytes(mgs_key kt, mgs_val vt, size_t n);
 int sort_dispatch(mgs_key kt, mgs_val vt, const void* kin, void* kout, const void* vin, void* vout, size_t n,
                   void* temp, size_t temp_bytes, hipStream_t s, hipEvent_t* events = nullptr, int num_events = 0,
                   int* num_marks = nullptr);

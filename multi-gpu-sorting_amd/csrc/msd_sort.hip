@@ -46,6 +46,7 @@
 #include <mutex>
 
 #include "internal.hpp"
+#include "msd_pass.hpp"
 #include "msd_sort.hpp"
 #include "radix_device.hpp"
 
@@ -59,14 +60,10 @@ constexpr int kMsdTile = MsdCfg::kTile;
 constexpr int kLocalIpt = MsdCfg::kLocalIpt;
 constexpr uint32_t kLocalCap = MsdCfg::kLocalCap;
 constexpr uint32_t kBatchTarget = kLocalCap / 2;
-constexpr uint32_t kNoWork = 0xFFFFFFFFu;
 
-// Decision word bits (MsdCtl::off): any set bit turns the path off.
-// kOffSample: a bucket holds more than kSampleCrowd of the 1024 sampled keys
-// (5 times its share: far beyond the scan's limit of twice the share, which
-// uniform keys reach in the sample with a chance of about 1e-6), so the
-// upfront read is skipped and the scan and finish kernels return at once.
-enum : uint32_t { kOffOverflow = 1u, kOffSubBucket = 2u, kOffBucket = 4u, kOffSample = 8u };
+// A bucket holding more than kSampleCrowd of the 1024 sampled keys (5 times
+// its share: far beyond the scan's limit of twice the share, which uniform
+// keys reach in the sample with a chance of about 1e-6) sets kMsdOffSample.
 constexpr uint32_t kSampleCrowd = 20;
 
 
@@ -133,7 +130,7 @@ __global__ __launch_bounds__(kMsdBlock) void msd_upfront_kernel(const uint32_t* 
   if (tid < kRadix && s_bh[tid] > kSampleCrowd) s_crowd = 1u;
   __syncthreads();
   if (s_crowd) {
-    if (c == 0 && tid == 0) ctl->off = kOffSample;  // (the LSD sort clears the status word)
+    if (c == 0 && tid == 0) ctl->off = kMsdOffSample;  // (the LSD sort clears the status word)
     return;
   }
   if (c == 0 && tid == 0) {  // nothing else writes these during this kernel
@@ -260,7 +257,7 @@ __global__ __launch_bounds__(256) void msd_scan_kernel(const uint32_t* __restric
                                                        uint32_t* __restrict__ batch_cnt,
                                                        const uint32_t* __restrict__ chain_bad,
                                                        const uint32_t* __restrict__ xcd_of) {
-  if (ctl->off & kOffSample) return;
+  if (ctl->off & kMsdOffSample) return;
   __shared__ uint32_t sums[4];
   __shared__ uint32_t s_carry;
   const uint32_t b = blockIdx.x, d = threadIdx.x;
@@ -269,7 +266,7 @@ __global__ __launch_bounds__(256) void msd_scan_kernel(const uint32_t* __restric
     uint32_t m = 0, runs = 0;
     for (uint32_t c = d; c < chains; c += kRadix) {
       const uint32_t cb = chain_bad[c];
-      if (cb & 1u) atomicOr(&ctl->off, kOffOverflow);
+      if (cb & 1u) atomicOr(&ctl->off, kMsdOffOverflow);
       runs += cb >> 1;
       m |= 1u << (xcd_of[c] & 31u);
     }
@@ -293,14 +290,14 @@ __global__ __launch_bounds__(256) void msd_scan_kernel(const uint32_t* __restric
     for (; c < chains; ++c) cnt += (slices[(size_t)c * (kMsdBins / 2) + word] >> sh) & 0xFFFFu;
   }
   sub_cnt[s] = cnt;
-  if (cnt > kLocalCap) atomicOr(&ctl->off, kOffSubBucket);
+  if (cnt > kLocalCap) atomicOr(&ctl->off, kMsdOffSubBucket);
   const uint32_t excl = block_excl_scan_256(cnt, sums, (int)d);
   sub_off[s] = excl;
   if (d == kRadix - 1) {
     bucket_tot[b] = excl + cnt;
     // a bucket far above the mean would leave pass 2 to one or two
     // workgroups: the LSD sort, whose tiles any workgroup takes, does better
-    if (excl + cnt > 2 * (n / kRadix) + 2 * (uint32_t)kMsdTile) atomicOr(&ctl->off, kOffBucket);
+    if (excl + cnt > 2 * (n / kRadix) + 2 * (uint32_t)kMsdTile) atomicOr(&ctl->off, kMsdOffBucket);
   }
 
   // batches of the local sort inside this bucket: a sub-bucket starts a new
@@ -349,7 +346,7 @@ __global__ __launch_bounds__(256) void msd_finish_kernel(MsdCtl* __restrict__ ct
                                                          uint32_t* __restrict__ tile_base1,
                                                          uint32_t* __restrict__ tile_base2,
                                                          uint32_t* __restrict__ counters) {
-  if (ctl->off & kOffSample) return;
+  if (ctl->off & kMsdOffSample) return;
   __shared__ uint32_t sums[4];
   const uint32_t d = threadIdx.x;
   const uint32_t bt = bucket_tot[d];
@@ -373,239 +370,6 @@ __global__ __launch_bounds__(256) void msd_finish_kernel(MsdCtl* __restrict__ ct
   if (d < chains1) tile_base1[d] = d * tpc1;
   counters[d] = 0;  // pass 2
   if (d < kXcds) counters[kRadix + d] = 0;  // pass 1
-}
-
-// ---------------------------------------------------------------------------
-// passes 1 and 2: onesweep passes over chains of tiles with decoupled
-// look-back inside each chain (the look-back of the LSD pass kernel).
-//   pass 1  8 chains: equal ranges of the input; the digit bases of chain C
-//           are the byte-3 bucket starts plus the keys of that digit in
-//           the ranges before it (the upfront's per-range histograms)
-//   pass 2  256 chains: the byte-3 buckets; digit bases = sub-bucket starts
-// Chain c is served by the workgroups of XCD c mod 8 (when the upfront ran
-// on all eight XCDs), which start together on their XCD's first chain and
-// move on together, so at any time the 32 workgroups of an XCD work on
-// consecutive tiles of one chain: every digit run of the chain's output is
-// then written by consecutive tiles at about the same time.
-// ---------------------------------------------------------------------------
-struct MsdPassArgs {
-  const uint32_t* src;
-  uint32_t* dst;
-  uint32_t n;
-  uint32_t chains;             // 8 (pass 1) or 256 (pass 2)
-  const uint32_t* bucket_start;
-  const uint32_t* chain_pref;  // pass 1: prefix over the upfront's ranges per digit
-  uint32_t ranges_per_chain;   // pass 1: upfront ranges per chain
-  uint32_t chain_keys;         // pass 1: keys per chain
-  const uint32_t* sub_off;     // pass 2: sub-bucket offsets inside each bucket
-  const uint32_t* tile_base;   // first descriptor tile of each chain
-  uint32_t* counters;          // tiles taken per chain
-  uint32_t* desc;              // look-back descriptors, 256 per tile
-  int parity;                  // descriptor status rotation of this pass
-  const MsdCtl* ctl;
-  uint32_t* status;
-  uint32_t spin_limit;
-};
-
-__device__ __forceinline__ void msd_publish(uint32_t* p, uint32_t v, bool xcd_local) {
-  if (xcd_local)
-    st_wg(p, v);
-  else
-    st_agent(p, v);
-}
-
-template <int KT, int PASS>
-__global__ __launch_bounds__(kMsdBlock, 4) void msd_pass_kernel(MsdPassArgs a) {
-  constexpr int W = kMsdBlock / kWave;
-  constexpr int IPT = kMsdIpt;
-  constexpr int TILE = kMsdTile;
-  using D = uint32_t;
-  if (a.ctl->off) return;
-  const bool runs = a.ctl->runs != 0;
-  const int shift = (int)a.ctl->low + (PASS == 1 ? 8 : 0);  // the window's high or low byte
-
-  __shared__ uint32_t keys[TILE];
-  __shared__ uint32_t off[W][kRadix];
-  __shared__ uint32_t gbase[kRadix];
-  __shared__ uint32_t s_prefix[kRadix];
-  __shared__ uint32_t sums[4];
-  __shared__ uint32_t s_tile;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & (kWave - 1);
-  const int w = tid / kWave;
-  const bool lb_wave = tid >= kRadix && tid < 2 * kRadix;
-  const int taker = kRadix;
-  for (int i = tid; i < W * kRadix; i += kMsdBlock) (&off[0][0])[i] = 0;
-
-  auto chain_lo = [&](uint32_t c) -> uint32_t {
-    if constexpr (PASS == 1) return c * a.chain_keys;
-    else return a.bucket_start[c];
-  };
-  auto chain_hi = [&](uint32_t c) -> uint32_t {
-    if constexpr (PASS == 1) return (uint32_t)std::min<size_t>((size_t)(c + 1) * a.chain_keys, a.n);
-    else return a.bucket_start[c + 1];
-  };
-  // thread d < 256: output position of the chain's first key of digit d
-  auto digit_base = [&](uint32_t c, uint32_t d) -> uint32_t {
-    if constexpr (PASS == 1) return a.bucket_start[d] + a.chain_pref[(size_t)c * a.ranges_per_chain * kRadix + d];
-    else return a.bucket_start[c] + a.sub_off[c * kRadix + d];
-  };
-
-  const bool xcd_local = a.chains % kXcds == 0 && a.ctl->xcd_mask == (1u << kXcds) - 1;
-  uint32_t my_chain = blockIdx.x % a.chains, chains_left = a.chains, chain_step = 1;
-  if (xcd_local) {
-    my_chain = xcc_id();
-    chains_left = a.chains / kXcds;
-    chain_step = kXcds;
-  }
-  // next tile: (chain, tile inside the chain) packed as chain << 20 | tile
-  auto take = [&]() -> uint32_t {
-    while (chains_left > 0) {
-      const uint32_t t = atomicAdd(&a.counters[my_chain], 1u);
-      const uint32_t lo = chain_lo(my_chain), hi = chain_hi(my_chain);
-      if (t < (hi - lo + TILE - 1) / TILE) return (my_chain << 20) | t;
-      my_chain += chain_step;
-      if (my_chain >= a.chains) my_chain -= a.chains;
-      --chains_left;
-    }
-    return kNoWork;
-  };
-
-  if (tid == taker) s_tile = take();
-  __syncthreads();
-  uint32_t cur = s_tile;
-  uint32_t cur_chain = 0xFFFFFFFFu, cur_base = 0, clo = 0, chi = 0;
-  uint32_t kc[IPT];
-  auto load = [&](uint32_t lo, uint32_t hi, uint32_t t, uint32_t (&k)[IPT]) {
-    const uint32_t tb = lo + t * (uint32_t)TILE;
-    const uint32_t wb = tb + (uint32_t)(w * IPT * kWave + lane);
-    if (hi - tb >= (uint32_t)TILE) {
-#pragma unroll
-      for (int i = 0; i < IPT; ++i) k[i] = a.src[wb + i * kWave];
-    } else {
-#pragma unroll
-      for (int i = 0; i < IPT; ++i) {
-        const uint32_t idx = wb + i * kWave;
-        k[i] = idx < hi ? a.src[idx] : 0u;
-      }
-    }
-  };
-  if (cur != kNoWork) load(chain_lo(cur >> 20), chain_hi(cur >> 20), cur & 0xFFFFFu, kc);
-
-  while (cur != kNoWork) {
-    const uint32_t chain = cur >> 20, lt = cur & 0xFFFFFu;
-    if (chain != cur_chain) {
-      clo = chain_lo(chain);
-      chi = chain_hi(chain);
-    }
-    const uint32_t tb = clo + lt * (uint32_t)TILE;
-    const uint32_t tile_cnt = min((uint32_t)TILE, chi - tb);
-    const bool full = tile_cnt == (uint32_t)TILE;
-    const uint32_t wb = tb + (uint32_t)(w * IPT * kWave + lane);
-    uint32_t pk[IPT];
-    uint32_t* ct = off[w];
-    if (full) {
-      uint32_t dg[IPT];
-#pragma unroll
-      for (int i = 0; i < IPT; ++i) dg[i] = digit_of<KT>(kc[i], shift);
-      if (runs)
-        rank_items_full<IPT, true>(dg, ct, pk);
-      else
-        rank_items_full<IPT, false>(dg, ct, pk);
-    } else {
-#pragma unroll
-      for (int i = 0; i < IPT; ++i) {
-        const uint32_t d = digit_of<KT>(kc[i], shift);
-        pk[i] = (wb + i * kWave < chi) ? ((d << 16) | rank_wave_atomic<false>(d, ct)) : 0u;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < IPT; ++i) asm volatile("" : "+v"(kc[i]));
-    __syncthreads();
-
-    uint32_t total = 0;
-    D* chain_desc = a.desc + (size_t)a.tile_base[chain] * kRadix;
-    D win[kPassWindow];
-    uint32_t taken = kNoWork;
-    if (lb_wave) {
-      const uint32_t d = (uint32_t)tid - kRadix;
-      if (tid == taker) taken = take();
-#pragma unroll
-      for (int i = 0; i < W; ++i) total += off[i][d];
-      msd_publish(chain_desc + (size_t)lt * kRadix + d,
-                  Desc<D>::make(lt == 0 ? kStInclusive : kStAggregate, (D)total, a.parity), xcd_local);
-      if (lt > 0) lookback_load(chain_desc, (int64_t)lt - 1, d, win);
-    } else if (tid < kRadix) {
-#pragma unroll
-      for (int i = 0; i < W; ++i) total += off[i][tid];
-    }
-    const uint32_t excl = block_excl_scan_256(tid < kRadix ? total : 0u, sums, tid);
-    if (tid < kRadix) {
-      uint32_t r = excl;
-#pragma unroll
-      for (int i = 0; i < W; ++i) {
-        const uint32_t c = off[i][tid];
-        off[i][tid] = r;
-        r += c;
-      }
-      if (chain != cur_chain) cur_base = digit_base(chain, (uint32_t)tid);
-      s_prefix[tid] = cur_base - excl;
-    }
-    cur_chain = chain;
-    if (tid == taker) s_tile = taken;
-    __syncthreads();
-    int64_t lb_t = (int64_t)lt - 1;
-    uint32_t lb_prefix = 0;
-    bool lb_done = false;
-    if (lb_wave && lt > 0)
-      lb_done = lookback_step(chain_desc, lb_t, (uint32_t)tid - kRadix, a.parity, win, lb_prefix);
-    if (full) {
-      uint32_t pos[IPT];
-#pragma unroll
-      for (int i = 0; i < IPT; ++i) pos[i] = min(off[w][pk[i] >> 16] + (pk[i] & 0xFFFFu), (uint32_t)TILE - 1);
-#pragma unroll
-      for (int i = 0; i < IPT; ++i) keys[pos[i]] = kc[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < IPT; ++i) {
-        const uint32_t pos = off[w][pk[i] >> 16] + (pk[i] & 0xFFFFu);
-        if (wb + i * kWave < chi && pos < (uint32_t)TILE) keys[pos] = kc[i];
-      }
-    }
-    const uint32_t nxt = s_tile;
-    if (nxt != kNoWork) {
-      const uint32_t nc = nxt >> 20;
-      load(chain_lo(nc), chain_hi(nc), nxt & 0xFFFFFu, kc);
-    }
-    for (int i = lane; i < kRadix; i += kWave) off[w][i] = 0;
-    if (lb_wave) {
-      const uint32_t d = (uint32_t)tid - kRadix;
-      if (lt > 0) {
-        bool gave_up = false;
-        const uint32_t prefix =
-            lb_done ? lb_prefix : lookback_from(chain_desc, lb_t, d, a.parity, win, lb_prefix, a.spin_limit, gave_up);
-        if (gave_up) atomicOr(a.status, kStatusLookback);
-        msd_publish(chain_desc + (size_t)lt * kRadix + d, Desc<D>::make(kStInclusive, (D)(prefix + total), a.parity),
-                    xcd_local);
-        gbase[d] = s_prefix[d] + prefix;
-      } else {
-        gbase[d] = s_prefix[d];
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) {
-      const uint32_t i = (uint32_t)(j * kMsdBlock + tid);
-      if (full || i < tile_cnt) {
-        const uint32_t kk = keys[i];
-        const uint32_t o = min(gbase[digit_of<KT>(kk, shift)] + i, a.n - 1);
-        a.dst[o] = kk;
-      }
-    }
-    __syncthreads();
-    cur = nxt;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -813,10 +577,17 @@ uint32_t msd_resident(K kernel) {
 
 }  // namespace
 
-bool msd_eligible(size_t n) {
-  if (env_u32("MGS_MSD", 1) == 0 || n > MsdCfg::kMaxKeys) return false;
+bool msd_enabled() { return env_u32("MGS_MSD", 1) != 0; }
+
+size_t msd_min_override(size_t dflt) {
   const char* e = std::getenv("MGS_MSD_MIN");
-  if (e != nullptr && e[0] != 0) return n >= env_u32("MGS_MSD_MIN", 0);
+  return e != nullptr && e[0] != 0 ? env_u32("MGS_MSD_MIN", 0) : dflt;
+}
+
+bool msd_eligible(size_t n) {
+  if (!msd_enabled() || n > MsdCfg::kMaxKeys) return false;
+  const size_t from = msd_min_override(MGS_MAX_KEYS);
+  if (from != MGS_MAX_KEYS) return n >= from;
   return (n >= MsdCfg::kMinKeys && n < MsdCfg::kGapLo) || n >= MsdCfg::kGapHi;
 }
 
@@ -893,7 +664,7 @@ int msd_launch(const void* kin, void* kout, void* alt, size_t n, char* t, const 
   constexpr uint32_t kRangesPerChain = MsdCfg::kMaxChains / kXcds;
   const uint32_t chains1 = (ranges + kRangesPerChain - 1) / kRangesPerChain;
   // workgroups of the passes and the local sort: as many as are resident
-  uint32_t grid = msd_resident(msd_pass_kernel<KT, 1>);
+  uint32_t grid = msd_resident(msd_pass_kernel<KT, NoVal, 1, kMsdBlock, kMsdIpt, 4>);
   grid = grid ? grid : 256u;
 
   mark(s, "msd_upfront");
@@ -909,7 +680,7 @@ int msd_launch(const void* kin, void* kout, void* alt, size_t n, char* t, const 
   mark(s, "msd_finish");
   msd_finish_kernel<<<1, kRadix, 0, s>>>(ctl, bucket_tot, bucket_start, batch_cnt, batch_base, chains1,
                                          kRangesPerChain * tpr, tile_base1, tile_base2, counters);
-  MsdPassArgs a{};
+  MsdPassArgs<uint32_t, NoVal> a{};
   a.n = nn;
   a.bucket_start = bucket_start;
   a.chain_pref = chain_pref;
@@ -927,7 +698,7 @@ int msd_launch(const void* kin, void* kout, void* alt, size_t n, char* t, const 
   a.tile_base = tile_base1;
   a.counters = counters + kRadix;
   a.parity = 0;
-  msd_pass_kernel<KT, 1><<<std::min(grid, tiles), kMsdBlock, 0, s>>>(a);
+  msd_pass_kernel<KT, NoVal, 1, kMsdBlock, kMsdIpt, 4><<<std::min(grid, tiles), kMsdBlock, 0, s>>>(a);
   mark(s, "msd_pass2");
   a.src = ka;
   a.dst = ko;
@@ -935,7 +706,7 @@ int msd_launch(const void* kin, void* kout, void* alt, size_t n, char* t, const 
   a.tile_base = tile_base2;
   a.counters = counters;
   a.parity = 1;
-  msd_pass_kernel<KT, 2><<<grid, kMsdBlock, 0, s>>>(a);
+  msd_pass_kernel<KT, NoVal, 2, kMsdBlock, kMsdIpt, 4><<<grid, kMsdBlock, 0, s>>>(a);
   mark(s, "msd_batches");
   msd_batches_kernel<<<kRadix, kRadix, 0, s>>>(ctl, bucket_start, sub_off, leaders, batch_cnt, batch_base, batches);
   mark(s, "msd_local");

@@ -54,12 +54,21 @@ struct MsdCtl {
   uint32_t xcd_mask;  // XCDs the upfront kernel ran on
   uint32_t runs;
   uint32_t low;
+  uint32_t high[2];  // the shared leading bits above the window (low word first)
 };
+
+// MsdCtl::off bits.  kMsdOffSample: the sampled keys crowd, so the upfront
+// read is skipped and the scan and finish kernels return at once.
+enum : uint32_t { kMsdOffOverflow = 1u, kMsdOffSubBucket = 2u, kMsdOffBucket = 4u, kMsdOffSample = 8u };
 
 struct MsdLayout {
   size_t ctl, desc, slices, chain_hist, chain_pref, chain_bad, xcd_of, sub_cnt, sub_off, bucket_tot, bucket_start,
       leaders, batch_cnt, batch_base, batches, tile_base1, tile_base2, counters, end;
 };
+
+// MGS_MSD not set to 0, and the value of MGS_MSD_MIN (dflt without it).
+bool msd_enabled();
+size_t msd_min_override(size_t dflt);
 
 // n in the range the path is tried for (and MGS_MSD not set to 0).
 bool msd_eligible(size_t n);

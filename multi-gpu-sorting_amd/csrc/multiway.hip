@@ -406,6 +406,7 @@ __global__ __launch_bounds__(kMwBlock, MwCfg<Bits>::kWaves) void mw_piece_kernel
   const uint32_t cnt = readfirstlane(bnd[k]);
   if (cnt == 0) return;
   const uint32_t nit = block_items<kMwBlock>(cnt), wb = block_first<kMwBlock>(nit);
+  const Bits pad = block_pad<KT>(mx);
   Bits key[kIpt];
   uint32_t none[kIpt];
   // the slice of the thread's first slot (last j with bnd[j] <= wb), then on
@@ -420,10 +421,9 @@ __global__ __launch_bounds__(kMwBlock, MwCfg<Bits>::kWaves) void mw_piece_kernel
   }
   uint32_t next = bnd[lo + 1];
   const Bits* src = sptr[lo] - bnd[lo];
-#pragma unroll
-  for (int i = 0; i < kIpt; ++i) {
+  static_for<kIpt>([&](auto i) {
     const uint32_t e = wb + i * kWave;
-    key[i] = Codec<KT>::dec(mx);
+    key[i] = pad;
     if ((uint32_t)i < nit && e < cnt) {
       if (e >= next) {
         do next = bnd[++lo + 1];
@@ -432,14 +432,13 @@ __global__ __launch_bounds__(kMwBlock, MwCfg<Bits>::kWaves) void mw_piece_kernel
       }
       key[i] = src[e];
     }
-  }
+  });
   // (only unsorted runs have keys outside the samples' bounds; block_sort
   // then stays in bounds, but padding may take their place)
-#pragma unroll
-  for (int i = 0; i < kIpt; ++i) {
+  static_for<kIpt>([&](auto i) {
     const Bits x = Codec<KT>::enc(key[i]);
     bad |= x < mn || x > mx;
-  }
+  });
   if (bad) atomicOr(status, kStatusUnsorted);
   block_sort<KT, NoVal, kMwBlock, kIpt>(sm, key, none, cnt, mn, mx, out + bases[b], (NoVal*)nullptr);
 }

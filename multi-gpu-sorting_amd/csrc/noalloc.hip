@@ -49,7 +49,7 @@ size_t noalloc_scratch_bytes() { return kNoAllocScratchBytes; }
 
 int sort_noalloc(mgs_key kt, mgs_val vt, const void* kin, void* kout, const void* vin, void* vout, size_t n,
                  hipStream_t s) {
-  const size_t need = sort_temp_bytes(kt, vt, n);
+  const size_t need = sort_least_temp_bytes(kt, vt, n);
   if (need > kNoAllocScratchBytes) return MGS_ERR_TOO_LARGE;
   void* p = nullptr;
   if (need > 0) {

@@ -8,6 +8,7 @@
 
 #include "internal.hpp"
 #include "msd_sort.hpp"
+#include "msd_wide.hpp"
 #include "radix_device.hpp"
 
 namespace mgs {
@@ -861,8 +862,10 @@ SortLayout sort_layout(size_t n) {
 // Wide records switch to larger tiles (fewer descriptors) at kBigTileMin
 // keys, so just above it the small-tile layout of kBigTileMin - 1 keys can
 // be the larger one; a buffer sized for n must serve every smaller sort.
+// wide: with room for the three-pass path of wider records, which such a sort
+// takes only if it finds the room.
 template <int KB, int VB>
-size_t sort_bytes(size_t n) {
+size_t sort_bytes(size_t n, bool wide) {
   const SortLayout L = sort_layout<KB, VB>(n);
   size_t b = L.total;
   // the three-pass path's region wherever it may run, and from its lowest
@@ -870,6 +873,8 @@ size_t sort_bytes(size_t n) {
   // decrease with n
   if (KB == 4 && VB == 0 && (msd_eligible(n) || n >= MsdCfg::kMinKeys))
     b = std::max(b, msd_layout(std::min(n, MsdCfg::kMaxKeys), L.desc, L.msd_ctl).end);
+  if (KB + VB > 4 && wide && (wide_eligible(KB, VB, n) || n >= wide_min(KB)))
+    b = std::max(b, wide_layout(KB + VB, std::min(n, wide_max(KB + VB)), L.desc, L.msd_ctl).end);
   if (KB + VB > 4 && n >= kBigTileMin) b = std::max(b, sort_layout_cfg<KB, VB, false>(kBigTileMin - 1).total);
   return b;
 }
@@ -949,6 +954,18 @@ int sort_typed_cfg(const void* kin, void* kout, const void* vin, void* vout, siz
       const int rc = msd_launch<KT>(kin, kout, ka, n, t, ML, status, spin_limit, s, mark);
       if (rc != MGS_OK) return rc;
       gate = reinterpret_cast<const uint32_t*>(t + ML.ctl);  // MsdCtl::off
+    }
+  }
+  // wider records: their three-pass path first, where the scratch has room
+  // for its tables (a buffer that only fits the LSD passes is taken too)
+  if constexpr (KB + VB > 4 && !kFloatKey<KT>) {
+    if (wide_eligible(KB, VB, n)) {
+      const WideLayout WL = wide_layout(KB + VB, n, L.desc, L.msd_ctl);
+      if (temp_bytes >= WL.end) {
+        const int rc = wide_launch<KT, VT>(kin, kout, ka, vin, vout, va, n, t, WL, status, spin_limit, s, mark);
+        if (rc != MGS_OK) return rc;
+        gate = reinterpret_cast<const uint32_t*>(t + WL.ctl);  // MsdCtl::off
+      }
     }
   }
 
@@ -1061,7 +1078,8 @@ int sort_by_val(mgs_val vt, const void* kin, void* kout, const void* vin, void* 
 
 }  // namespace
 
-size_t sort_temp_bytes(mgs_key kt, mgs_val vt, size_t n) {
+namespace {
+size_t temp_bytes_of(mgs_key kt, mgs_val vt, size_t n, bool wide) {
   const int kb = key_bytes(kt), vb = val_bytes(vt);
   if (kb <= 0 || vb < 0) return 0;
   size_t small_tile;
@@ -1070,28 +1088,33 @@ size_t sort_temp_bytes(mgs_key kt, mgs_val vt, size_t n) {
   else small_tile = SmallCfg<8, 8>::kTile;
   if (n <= small_tile) return 0;
   if (kb == 4) {
-    if (vb == 0) return sort_bytes<4, 0>(n);
-    if (vb == 4) return sort_bytes<4, 4>(n);
-    return sort_bytes<4, 8>(n);
+    if (vb == 0) return sort_bytes<4, 0>(n, wide);
+    if (vb == 4) return sort_bytes<4, 4>(n, wide);
+    return sort_bytes<4, 8>(n, wide);
   }
-  if (vb == 0) return sort_bytes<8, 0>(n);
-  if (vb == 4) return sort_bytes<8, 4>(n);
-  return sort_bytes<8, 8>(n);
+  if (vb == 0) return sort_bytes<8, 0>(n, wide);
+  if (vb == 4) return sort_bytes<8, 4>(n, wide);
+  return sort_bytes<8, 8>(n, wide);
 }
+}  // namespace
+
+size_t sort_temp_bytes(mgs_key kt, mgs_val vt, size_t n) { return temp_bytes_of(kt, vt, n, true); }
+size_t sort_least_temp_bytes(mgs_key kt, mgs_val vt, size_t n) { return temp_bytes_of(kt, vt, n, false); }
 
 namespace {
 thread_local std::string g_stage_names;
 
 template <int KB, int VB>
-int path_of(size_t n, const void* temp, size_t temp_bytes, hipStream_t s) {
+int path_of(bool floats, size_t n, const void* temp, size_t temp_bytes, hipStream_t s) {
   using SCfg = SmallCfg<KB, VB>;
   if (n <= (size_t)SCfg::kTile) return MGS_PATH_SMALL;
-  if (!(KB == 4 && VB == 0 && msd_eligible(n))) return MGS_PATH_LSD;
+  constexpr bool kAlone4 = KB == 4 && VB == 0;
+  if (!(kAlone4 ? msd_eligible(n) : !floats && wide_eligible(KB, VB, n))) return MGS_PATH_LSD;
   const SortLayout L = sort_layout<KB, VB>(n);
-  const MsdLayout ML = msd_layout(n, L.desc, L.msd_ctl);
-  if (temp == nullptr || temp_bytes < ML.end) return MGS_ERR_TEMP_TOO_SMALL;
+  const size_t need = kAlone4 ? msd_layout(n, L.desc, L.msd_ctl).end : wide_layout(KB + VB, n, L.desc, L.msd_ctl).end;
+  if (temp == nullptr || temp_bytes < need) return kAlone4 || temp == nullptr ? MGS_ERR_TEMP_TOO_SMALL : MGS_PATH_LSD;
   uint32_t off = 0;
-  hipError_t e = hipMemcpyAsync(&off, static_cast<const char*>(temp) + ML.ctl, sizeof(off), hipMemcpyDeviceToHost, s);
+  hipError_t e = hipMemcpyAsync(&off, static_cast<const char*>(temp) + L.msd_ctl, sizeof(off), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return record_hip(e);
   return off == 0 ? MGS_PATH_THREE_PASS : MGS_PATH_LSD;
@@ -1099,16 +1122,17 @@ int path_of(size_t n, const void* temp, size_t temp_bytes, hipStream_t s) {
 }  // namespace
 
 int sort_path(mgs_key kt, mgs_val vt, size_t n, const void* temp, size_t temp_bytes, hipStream_t s) {
+  const bool floats = kt == MGS_KEY_F32 || kt == MGS_KEY_F64;
   const int kb = key_bytes(kt), vb = val_bytes(vt);
   if (kb <= 0 || vb < 0) return MGS_ERR_BAD_TYPE;
   if (kb == 4) {
-    if (vb == 0) return path_of<4, 0>(n, temp, temp_bytes, s);
-    if (vb == 4) return path_of<4, 4>(n, temp, temp_bytes, s);
-    return path_of<4, 8>(n, temp, temp_bytes, s);
+    if (vb == 0) return path_of<4, 0>(floats, n, temp, temp_bytes, s);
+    if (vb == 4) return path_of<4, 4>(floats, n, temp, temp_bytes, s);
+    return path_of<4, 8>(floats, n, temp, temp_bytes, s);
   }
-  if (vb == 0) return path_of<8, 0>(n, temp, temp_bytes, s);
-  if (vb == 4) return path_of<8, 4>(n, temp, temp_bytes, s);
-  return path_of<8, 8>(n, temp, temp_bytes, s);
+  if (vb == 0) return path_of<8, 0>(floats, n, temp, temp_bytes, s);
+  if (vb == 4) return path_of<8, 4>(floats, n, temp, temp_bytes, s);
+  return path_of<8, 8>(floats, n, temp, temp_bytes, s);
 }
 
 const char* last_stage_names() { return g_stage_names.c_str(); }

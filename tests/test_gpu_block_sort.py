@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import pyoracle as O
-from helpers import KEY_NAME, from_dev, random_keys, to_dev
+from helpers import KEY_NAME, from_dev, random_keys, random_vals, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -76,3 +76,73 @@ def test_one_or_two_runs(mg, lens, portions):
     assert mg.temp_status(temp) == 0
     assert portions == 0 or (len(ends) == portions and ends[-1] == expect.size and ends == sorted(ends))
     assert np.array_equal(from_dev(out, np.uint32), expect)
+
+
+RECORDS = [(O.K_U64, None), (O.K_I64, np.uint32), (O.K_U64, np.uint64), (O.K_U32, np.uint32), (O.K_I32, np.uint64)]
+
+
+def run_three_pass(mg, kt, vdt, keys, rng, inplace):
+    """Sorts on the device, checks status and oracle, returns the path."""
+    import torch
+    n = keys.size
+    vals = None if vdt is None else random_vals(vdt, n, rng)
+    ek, ev = O.sort(kt, keys, vals)
+    vt = mg.VAL_NONE if vdt is None else (mg.VAL_U32 if vdt == np.uint32 else mg.VAL_U64)
+    temp = mg.temp_buffer(mg.lib.mgs_sort_temp_bytes(kt, vt, n), "cuda")
+    dk, dv = to_dev(keys), to_dev(vals)
+    ok = dk if inplace else torch.empty_like(dk)
+    ov = dv if inplace or dv is None else torch.empty_like(dv)
+    mg.sort(KEY_NAME[kt], dk, dv, keys_out=ok, vals_out=ov, temp=temp)
+    assert mg.temp_status(temp) == 0
+    path = mg.lib.mgs_sort_path(kt, vt, n, mg._ptr(temp), temp.numel(), None)
+    assert np.array_equal(from_dev(ok, keys.dtype), ek)
+    if vdt is not None:
+        assert np.array_equal(from_dev(ov, vals.dtype), ev)
+    if not inplace:
+        assert np.array_equal(from_dev(dk, keys.dtype), keys)
+    return path
+
+
+@pytest.mark.parametrize("kt,vdt", RECORDS, ids=lambda v: str(v))
+@pytest.mark.parametrize("n", [8195, 100_003, (1 << 20) + 77])
+@pytest.mark.parametrize("dist", ["uniform", "sorted", "reverse", "few", "lowbits", "runs", "nonneg", "stray",
+                                  "clustered", "pairs"])
+def test_three_pass_wide_forced(mg, kt, vdt, n, dist, monkeypatch):
+    """The three-pass path of wider records, tried at any size: uniform keys
+    take it, keys that crowd its sub-buckets or leave the sample's shared
+    bits hand over to the LSD passes; the result is the oracle's either way,
+    in place and out of place."""
+    monkeypatch.setenv("MGS_MSD_MIN", "0")
+    rng = np.random.default_rng(n + 5 * kt)
+    keys = tied_keys(kt, n, rng, dist) if dist in ("clustered", "pairs") else random_keys(kt, n, rng, dist)
+    path = run_three_pass(mg, kt, vdt, keys, rng, inplace=bool(n & 1))
+    assert path in (2, 3)
+    if dist in ("uniform", "nonneg"):
+        assert path == 3
+
+
+@pytest.mark.parametrize("kt,vdt", RECORDS, ids=lambda v: str(v))
+@pytest.mark.parametrize("dist", ["uniform", "sorted", "skewed", "nonneg"])
+def test_three_pass_wide_default(mg, kt, vdt, dist):
+    """Without environment: 8-byte keys from 2^22 records on, 4-byte keys
+    with payloads from 2^24."""
+    rng = np.random.default_rng(3 + kt)
+    keys = random_keys(kt, (1 << (22 if O.BITS_DTYPE[kt] == np.uint64 else 24)) + 4321, rng, dist)
+    path = run_three_pass(mg, kt, vdt, keys, rng, inplace=False)
+    assert path in (2, 3)
+    if dist == "uniform":
+        assert path == 3
+
+
+def test_three_pass_wide_small_scratch(mg):
+    """Scratch that only fits the LSD passes still sorts."""
+    rng = np.random.default_rng(8)
+    n = (1 << 22) + 9
+    keys = random_keys(O.K_U64, n, rng)
+    temp = mg.temp_buffer(n * 8 + (4 << 20), "cuda")
+    assert temp.numel() < mg.lib.mgs_sort_temp_bytes(O.K_U64, mg.VAL_NONE, n)
+    dk = to_dev(keys)
+    mg.sort("u64", dk, temp=temp)
+    assert mg.temp_status(temp) == 0
+    assert mg.lib.mgs_sort_path(O.K_U64, mg.VAL_NONE, n, mg._ptr(temp), temp.numel(), None) == 2
+    assert np.array_equal(from_dev(dk, np.uint64), np.sort(keys))
