@@ -78,18 +78,17 @@ enum {
 /* Tuning of the segmented sort; a zeroed struct (or NULL) selects the
  * defaults chosen by measurement on MI355X. */
 typedef struct mgs_tuning {
-  int32_t large_variant;    /* tile geometry of the large segments' passes: */
-                            /* 0 = default, 0 <= v <                        */
-                            /* mgs_segmented_variant_count(), see           */
+  int32_t large_variant;    /* tile geometry of the scatter of segments that */
+                            /* do not fit one workgroup: 0 = default, 0 <=  */
+                            /* v < mgs_segmented_variant_count(), see       */
                             /* mgs_segmented_variant(); others are          */
                             /* MGS_ERR_INVALID                              */
-  int32_t small_max;        /* segments up to this length sort inside one   */
-                            /* workgroup's LDS (0 = default)                */
-  int32_t medium_max;       /* segments up to this length sort with a single*/
-                            /* workgroup streaming HBM (0 = default)        */
+  int32_t small_max;        /* segments up to the larger of these two sort  */
+  int32_t medium_max;       /* inside one workgroup's LDS, as far as they   */
+                            /* fit (either 0 = default: as many as fit)     */
   int32_t max_segment_keys; /* longest segment the call accepts (0 = any up */
-                            /* to max_total_keys); below 2^30 the look-back */
-                            /* descriptors take 4 bytes instead of 8        */
+                            /* to max_total_keys); short ones take fewer    */
+                            /* launches                                     */
 } mgs_tuning;
 
 /* --------------------------------------------------------------------------
@@ -250,14 +249,14 @@ int mgs_fill_max(mgs_key kt, void* keys, size_t n, void* stream);
 size_t mgs_segmented_sort_temp_bytes(mgs_key kt, mgs_val vt,
                                      size_t max_total_keys, size_t nseg);
 
-/* The same for calls that pass `tuning` (its max_segment_keys shrinks the
- * look-back descriptors, and its large_variant sets the number of large
- * tiles); NULL gives mgs_segmented_sort_temp_bytes. */
+/* The same for calls that pass `tuning` (its max_segment_keys may save a
+ * split level's tables, and its large_variant sets the number of tiles); NULL
+ * gives mgs_segmented_sort_temp_bytes. */
 size_t mgs_segmented_sort_temp_bytes_tuned(mgs_key kt, mgs_val vt,
                                            size_t max_total_keys, size_t nseg,
                                            const mgs_tuning* tuning);
 
-/* Tile geometries of the large segments' passes (no reference counterpart:
+/* Tile geometries of the long segments' scatter (no reference counterpart:
  * the search space of the batching layer's autotuner).  Variants are
  * 0 .. mgs_segmented_variant_count() - 1 for every (kt, vt); variant v of
  * (kt, vt) runs workgroups of *block threads with *items_per_thread keys

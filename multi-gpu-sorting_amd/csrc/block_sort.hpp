@@ -6,11 +6,10 @@
 // sort takes at most three LSD passes of 9 bits over the top 27 of these (the
 // window).  Among 4096 random keys one pair in a workgroup of 16 shares a
 // window value, so 4-byte and 8-byte keys alike cost two or three passes; the
-// write-out compares neighbours, and a workgroup that finds a record above
-// its successor puts the records that share a window value in order by
-// looking around each.  A group longer than kTieReach records that are not
-// all equal would make that quadratic: the workgroup then takes the passes
-// over all differing bits instead.
+// write-out compares neighbours, and where a record is above its successor
+// one thread puts the records that share their window value in order.  A
+// group longer than kTieReach would make that slow: the workgroup then takes
+// the passes over all differing bits instead.
 //
 // Measured in the local sort of 2^28 u64 keys (batches of 4096, two
 // workgroups of 512 threads per CU): moving the records through registers
@@ -38,7 +37,8 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_each(static_cast<F&&>(f), std::make_integer_sequence<int, N>{});
 }
 
-// Records a thread looks at on each side of its own in the write-out.
+// Records that a thread puts in order on each side of the first one below its
+// predecessor.
 constexpr uint32_t kTieReach = 16;
 // LDS counter rows of the 9-bit digits, one per wavefront.  The row stride
 // puts the two threads that scan one digit's 16 rows on different banks.
@@ -123,6 +123,46 @@ __device__ __forceinline__ Bits lane_below(Bits x) {
   }
   return (Bits)lo;
 }
+// Smallest and largest encoded key of the block's m records (m > 0), held as
+// k[i] at position wb + 64 i, i < nit.
+template <int KT, typename V, int BLOCK, int IPT>
+__device__ __forceinline__ void block_min_max(BlockSortSmem<typename Codec<KT>::Bits, V, BLOCK, IPT>& sm,
+                                              const typename Codec<KT>::Bits (&k)[IPT], uint32_t wb, uint32_t m,
+                                              uint32_t nit, typename Codec<KT>::Bits& mn,
+                                              typename Codec<KT>::Bits& mx) {
+  using Bits = typename Codec<KT>::Bits;
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  Bits a = ~Bits(0), b = 0;
+  static_for<IPT>([&](auto i) {
+    if ((uint32_t)i < nit && wb + i * kWave < m) {
+      const Bits e = Codec<KT>::enc(k[i]);
+      a = e < a ? e : a;
+      b = e > b ? e : b;
+    }
+  });
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const Bits x = __shfl_xor(a, o, kWave), y = __shfl_xor(b, o, kWave);
+    a = x < a ? x : a;
+    b = y > b ? y : b;
+  }
+  if (lane == 0) {
+    sm.lo[w] = a;
+    sm.hi[w] = b;
+  }
+  __syncthreads();
+  a = sm.lo[0];
+  b = sm.hi[0];
+#pragma unroll
+  for (int i = 1; i < BLOCK / kWave; ++i) {
+    const Bits x = sm.lo[i], y = sm.hi[i];
+    a = x < a ? x : a;
+    b = y > b ? y : b;
+  }
+  mn = a;
+  mx = b;
+}
+
 // The padding key of block_sort: not below any key bounded by mx.  (No float
 // has the image just below +0.0's: -0.0 shares +0.0's, and dec() of it would
 // land above mx.)
@@ -246,8 +286,10 @@ __device__ __forceinline__ void block_sort(BlockSortSmem<typename Codec<KT>::Bit
   }
   // write-out: thread t has the records t, t + BLOCK, ..., U loads in flight
   constexpr uint32_t U = sizeof(Bits) + kValBytes<V> <= 8 ? 8 : 4;
-  auto write_out = [&](auto check) -> bool {
-    bool down = false;
+  // (the check's result: bit j for a j-th record below its predecessor)
+  static_assert(IPT <= 32, "a bit per record of a thread");
+  auto write_out = [&](auto check) -> uint32_t {
+    uint32_t down = 0;
 #pragma unroll 1
     for (uint32_t j = 0; j < nit; j += U) {
       Bits x[U], edge[U];
@@ -263,7 +305,7 @@ __device__ __forceinline__ void block_sort(BlockSortSmem<typename Codec<KT>::Bit
         if constexpr (check.value) {
           // the record before: the lane below's, or for the first lane the edge
           const Bits b = lane_below(x[u]);
-          down |= p < m && Codec<KT>::enc(lane == 0 ? edge[u] : b) > Codec<KT>::enc(x[u]);
+          if (p < m && Codec<KT>::enc(lane == 0 ? edge[u] : b) > Codec<KT>::enc(x[u])) down |= 1u << (j + u);
         }
         if (p < m) {
           store(p, x[u]);
@@ -277,52 +319,46 @@ __device__ __forceinline__ void block_sort(BlockSortSmem<typename Codec<KT>::Bit
     write_out(std::integral_constant<bool, false>{});
     return;
   }
-  const bool down = write_out(std::integral_constant<bool, true>{});
+  uint32_t down = write_out(std::integral_constant<bool, true>{});
   // (the stores below may follow another thread's to the same place)
   auto stored = [] { __builtin_amdgcn_s_waitcnt(0); };
-  if (down) stored();
-  if (!__syncthreads_or(down ? 1 : 0)) return;
   stored();
-  __syncthreads();
-  // a record moves left past the larger records of its group before it, right
-  // past the smaller ones after it
+  if (!__syncthreads_or(down != 0 ? 1 : 0)) return;
+  // Groups out of order: the thread that sees the first record of a group
+  // below its predecessor writes the whole group in order.  A group that
+  // reaches further than kTieReach from there is left to the passes.
   bool slow = false;
   const Bits lim = Bits(1) << low;
   auto image = [&](uint32_t p) { return Codec<KT>::enc(sm.keys[p]); };
-#pragma unroll 1
-  for (uint32_t j = 0; j < nit; ++j) {
-    const uint32_t p = j * BLOCK + tid;
-    if (p >= m) break;
-    const Bits raw = sm.keys[p], e = Codec<KT>::enc(raw);
-    bool differ = false, longer = false;
-    int by = 0;
-    for (uint32_t r = 1; r <= p; ++r) {
-      const Bits x = image(p - r);
+  while (down != 0) {
+    const uint32_t p = (uint32_t)__builtin_ctz(down) * BLOCK + tid;
+    down &= down - 1;
+    uint32_t l = p - 1, r = p;
+    Bits e = image(l);
+    bool first = true;
+    while (l > 0) {
+      const Bits x = image(l - 1);
       if ((x ^ e) >= lim) break;
-      if (r > kTieReach) {
-        longer = true;
-        break;
-      }
-      differ |= x != e;
-      by -= x > e ? 1 : 0;
+      if (x > e) first = false;
+      if (!first || p - l > kTieReach) break;
+      e = x;
+      --l;
     }
-    for (uint32_t r = 1; p + r < m; ++r) {
-      const Bits x = image(p + r);
-      if ((x ^ e) >= lim) break;
-      if (r > kTieReach) {
-        longer = true;
-        break;
-      }
-      differ |= x != e;
-      by += x < e ? 1 : 0;
+    if (!first) continue;
+    while (r + 1 < m && (image(r + 1) ^ e) < lim && r - p <= kTieReach) ++r;
+    if (p - l > kTieReach || r - p > kTieReach) {
+      slow = true;
+      continue;
     }
-    // a group that reaches further is in order if its records are all equal;
-    // otherwise the first different one on either side sees both the
-    // difference and the long run before it
-    slow |= differ && longer;
-    if (by != 0) {
-      store(p + (uint32_t)by, raw);
-      if constexpr (HV) store_val(p + (uint32_t)by, sm.vals[p]);
+    for (uint32_t q = l; q <= r; ++q) {
+      const Bits raw = sm.keys[q], x = Codec<KT>::enc(raw);
+      uint32_t to = l;
+      for (uint32_t t = l; t <= r; ++t) {
+        const Bits y = image(t);
+        to += (y < x || (y == x && t < q)) ? 1u : 0u;
+      }
+      store(to, raw);
+      if constexpr (HV) store_val(to, sm.vals[q]);
     }
   }
   stored();

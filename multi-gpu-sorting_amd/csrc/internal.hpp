@@ -87,6 +87,12 @@ int pivot_dispatch(mgs_key kt, const void* const* left, const void* const* right
 int swap_dispatch(mgs_key kt, mgs_val vt, void* ak, void* av, void* bk, void* bv, size_t n, hipStream_t s);
 int fill_max_dispatch(mgs_key kt, void* keys, size_t n, hipStream_t s);
 
+// mgs_sort by the segmented sort's splits and local sort (segmented.hip): one
+// array of n records.
+size_t split_sort_temp_bytes(mgs_key kt, mgs_val vt, size_t n);
+int split_sort(mgs_key kt, mgs_val vt, const void* kin, void* kout, const void* vin, void* vout, size_t n, void* temp,
+               size_t temp_bytes, hipStream_t s);
+
 size_t segmented_temp_bytes(mgs_key kt, mgs_val vt, size_t max_total, size_t nseg, const mgs_tuning* tuning);
 int segmented_variant(mgs_key kt, mgs_val vt, int var, int32_t* block, int32_t* ipt);
 int segmented_variant_count();

@@ -1,26 +1,41 @@
 // Batched segmented sort: thousands of independent arrays in a fixed launch
-// sequence whose grid sizes depend only on (nseg, max_total_keys), so a call
-// can be captured once in a hipGraph and replayed for new data.
+// sequence whose grid sizes depend only on (nseg, max_total_keys, tuning), so
+// a call can be captured once in a hipGraph and replayed for new data.
 //
 //   classify  one workgroup: resolves each segment's position (offsets form:
 //             [offsets[s], offsets[s+1]); ranges form: [ranges[2s],
 //             ranges[2s+1]) anywhere in the array, non-overlapping) and its
-//             place in the compact scratch buffer, then bins it by length
-//               small  (len <= small_max)  -> one workgroup sorts it in LDS
-//               medium (len <= medium_max) -> one workgroup streams it through
-//                                             HBM pass by pass, no look-back
-//               large                      -> onesweep tiles chained by
-//                                             decoupled look-back inside the
-//                                             segment
-//             and lays the large segments' tiles out back to back
-//   clear     zeroes per-segment histograms and look-back descriptors
-//   small     persistent grid over the small bin
-//   medium    persistent grid over the medium bin
-//   hist      per-tile histograms of the large segments
-//   scan      per-segment digit bases
-//   pass p    every large-segment tile of byte p in one launch
+//             place in the compact scratch buffer; a segment of at most
+//             small_max records becomes a batch of the local sort, a longer
+//             one a node of the first split level
+//   split level l (up to three): every node is scattered into at most 256
+//             children in key order, by
+//     count     per tile of every node: the digit of each key and their
+//               counts.  A node's digits are its own: 254 equal steps of the
+//               encoded key between (about) the first and the last hundredth
+//               of 256 sampled keys, and one digit for what lies below and
+//               above -- monotone in the key whatever the sample missed
+//     scan      per node: the tiles' offsets, and what becomes of the
+//               children: consecutive ones that fit one workgroup together
+//               become a batch, one that does not becomes a node of the next
+//               level, and one whose keys are all equal is done
+//     scatter   per tile: the records to their child, in input order
+//   long      children that are still too long after the last level: one
+//             workgroup each streams them through HBM byte by byte
+//   local     every batch is sorted in LDS (block_sort.hpp)
+//
+// A level moves a record once and reads its key twice, so an 8-byte key with
+// a payload takes one to two levels and the local sort instead of eight LSD
+// passes, and no key distribution needs a fallback: skewed keys only take
+// more levels.  Against LSD passes over all long segments at once and one
+// workgroup for each middle one: u64 + u32, 1024 segments of 2^8 to 2^22, 26.3
+// -> 12.3 ms; u32, 256 ranges of 2^10 to 2^18, 331 -> 166 us; f64, normal, 64
+// of 2^10 to 2^22, 2518 -> 752 us.
+#include <map>
+#include <mutex>
 #include <type_traits>
 
+#include "block_sort.hpp"
 #include "internal.hpp"
 #include "radix_device.hpp"
 
@@ -28,11 +43,28 @@ namespace mgs {
 
 namespace {
 
+constexpr int kMaxLevels = 3;
+
 struct SegCtl {
-  uint32_t status;  // the call's status word (first word of temp)
-  uint32_t n_small, n_medium, n_large, large_tiles;
+  uint32_t status;   // the call's status word (first word of temp)
   uint32_t skipped;  // segments left unsorted: malformed bounds or beyond max_total
+  uint32_t n_batches, n_long;
+  uint64_t alloc[kMaxLevels + 1];  // level's nodes << 32 | their tiles
 };
+
+// A range of a segment to be split: records [off, off + len), its tiles from
+// tile0 of the level on, and its digits (written by the count): 0 below
+// `base`, 255 above `top`, between them 1 + the step, which is the high word
+// of ((key - base) >> shift) mul (254 even steps), or key - base itself where
+// mul is 0 (every value a step).
+struct Node {
+  uint32_t seg, off, len, tile0;
+  uint64_t base, top;
+  uint32_t mul, shift;
+};
+
+// Where a batch's records are.
+enum : uint32_t { kSrcIn = 0, kSrcAlt = 1, kSrcOut = 2 };
 
 // Per-segment table written by classify: first key in the key array, first
 // payload in the payload array, first slot in the compact scratch buffer,
@@ -126,16 +158,12 @@ __global__ __launch_bounds__(kClassifyBlock) void seg_classify_kernel(const uint
                                                                       const uint64_t* __restrict__ val_begin,
                                                                       uint32_t nseg, uint64_t max_total,
                                                                       uint64_t max_seg,
-                                                                      uint32_t small_max, uint32_t medium_max,
-                                                                      uint32_t tile, SegTab tab,
-                                                                      uint32_t* small_list, uint32_t* medium_list,
-                                                                      uint32_t* large_list, uint32_t* tile_start,
-                                                                      SegCtl* ctl, uint32_t* tile_counter) {
+                                                                      uint32_t small_max, uint32_t tile, SegTab tab,
+                                                                      uint4* batches, Node* nodes, SegCtl* ctl) {
   __shared__ uint32_t sm[3][16];
   __shared__ uint64_t sm64[16];
   const int tid = threadIdx.x;
-  if (tid < kMaxPasses + 1) tile_counter[tid] = 0;
-  uint32_t run_s = 0, run_m = 0, run_l = 0, run_t = 0, skipped = 0;
+  uint32_t run_s = 0, run_l = 0, run_t = 0, skipped = 0;
   uint64_t run_alt = 0, run_max = 0;
   const uint64_t base0 = RANGES ? 0 : bounds[0];
   for (uint32_t base = 0; base < nseg; base += kClassifyBlock) {
@@ -178,70 +206,30 @@ __global__ __launch_bounds__(kClassifyBlock) void seg_classify_kernel(const uint
     }
     const uint32_t bad = (s < nseg && !ok) ? 1u : 0u;
     const uint32_t is_s = (s < nseg && len > 0 && len <= small_max) ? 1u : 0u;
-    const uint32_t is_m = (s < nseg && len > small_max && len <= medium_max) ? 1u : 0u;
-    const uint32_t is_l = (s < nseg && len > medium_max) ? 1u : 0u;
+    const uint32_t is_l = (s < nseg && len > small_max) ? 1u : 0u;
     const uint32_t nt = is_l ? (len + tile - 1) / tile : 0u;
-    uint32_t es, em, el, ts, tm, tl;
-    block_scan3(is_s, is_m, is_l, es, em, el, ts, tm, tl, sm);
-    uint32_t et, eb, e2, tt, tb, t2;
-    block_scan3(nt, bad, 0, et, eb, e2, tt, tb, t2, sm);
-    if (is_s) small_list[run_s + es] = s;
-    if (is_m) medium_list[run_m + em] = s;
-    if (is_l) {
-      large_list[run_l + el] = s;
-      tile_start[run_l + el] = run_t + et;
-    }
+    uint32_t es, el, et, eb, e1, e2, ts, tl, tt, tb, t1, t2;
+    block_scan3(is_s, is_l, nt, es, el, et, ts, tl, tt, sm);
+    block_scan3(bad, 0, 0, eb, e1, e2, tb, t1, t2, sm);
+    if (is_s) batches[run_s + es] = make_uint4(s, 0, len, kSrcIn);
+    if (is_l) nodes[run_l + el] = Node{s, 0, len, run_t + et, 0, 0, 0, 0};
     run_s += ts;
-    run_m += tm;
     run_l += tl;
     run_t += tt;
     skipped += tb;
   }
   if (tid == 0) {
-    ctl->n_small = run_s;
-    ctl->n_medium = run_m;
-    ctl->n_large = run_l;
-    ctl->large_tiles = run_t;
+    ctl->n_batches = run_s;
+    ctl->n_long = 0;
+    ctl->alloc[0] = (uint64_t)run_l << 32 | run_t;
+    for (int l = 1; l <= kMaxLevels; ++l) ctl->alloc[l] = 0;
     ctl->skipped = skipped;
     ctl->status = skipped ? kStatusSkipped : 0u;
-    tile_start[run_l] = run_t;
-  }
-}
-
-__global__ void seg_clear_kernel(uint32_t* __restrict__ hist, uint32_t hist_words_per_seg,
-                                 uint32_t* __restrict__ desc, uint32_t desc_words_per_tile,
-                                 const SegCtl* __restrict__ ctl) {
-  const size_t hw = (size_t)ctl->n_large * hist_words_per_seg;
-  const size_t dw = (size_t)ctl->large_tiles * desc_words_per_tile;
-  const size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t st = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = g; i < hw; i += st) hist[i] = 0;
-  for (size_t i = g; i < dw; i += st) desc[i] = 0;
-}
-
-template <int KT, typename V, int BLOCK, int IPT>
-__global__ __launch_bounds__(BLOCK) void seg_small_kernel(const typename Codec<KT>::Bits* k_in,
-                                                          typename Codec<KT>::Bits* k_out, const V* v_in, V* v_out,
-                                                          SegTab tab, const uint32_t* __restrict__ list,
-                                                          const SegCtl* __restrict__ ctl) {
-  const uint32_t cnt = ctl->n_small;
-  for (uint32_t i = blockIdx.x; i < cnt; i += gridDim.x) {
-    const uint32_t s = list[i];
-    const uint64_t b = tab.begin[s];
-    const uint32_t len = tab.len[s];
-    const V* vi = nullptr;
-    V* vo = nullptr;
-    if constexpr (kHasVal<V>) {
-      vi = v_in + tab.vbegin[s];
-      vo = v_out + tab.vbegin[s];
-    }
-    small_sort_block<KT, V, BLOCK, IPT>(k_in + b, k_out + b, vi, vo, len);
-    __syncthreads();
   }
 }
 
 // ---------------------------------------------------------------------------
-// Medium bin: one workgroup sorts a whole segment, pass by pass, walking its
+// Long ranges: one workgroup sorts a whole range, pass by pass, walking its
 // tiles in order and carrying the per-digit running offsets in LDS, so no
 // cross-workgroup look-back is needed.
 // ---------------------------------------------------------------------------
@@ -367,36 +355,38 @@ __device__ void medium_sort_block(const typename Codec<KT>::Bits* k_in, typename
 }
 
 template <int KT, typename V, int BLOCK, int IPT>
-__global__ __launch_bounds__(BLOCK) void seg_medium_kernel(const typename Codec<KT>::Bits* k_in,
-                                                           typename Codec<KT>::Bits* k_alt,
-                                                           typename Codec<KT>::Bits* k_out, const V* v_in, V* v_alt,
-                                                           V* v_out, SegTab tab, const uint32_t* __restrict__ list,
-                                                           const SegCtl* __restrict__ ctl) {
-  const uint32_t cnt = ctl->n_medium;
+__global__ __launch_bounds__(BLOCK) void seg_long_kernel(typename Codec<KT>::Bits* k_alt,
+                                                         typename Codec<KT>::Bits* k_out, V* v_alt, V* v_out,
+                                                         SegTab tab, const uint4* __restrict__ list,
+                                                         const SegCtl* __restrict__ ctl) {
+  const uint32_t cnt = ctl->n_long;
   for (uint32_t i = blockIdx.x; i < cnt; i += gridDim.x) {
-    const uint32_t s = list[i];
-    const uint64_t b = tab.begin[s];
-    const uint32_t len = tab.len[s];
-    const uint64_t ab = tab.alt[s];
-    const V* vi = nullptr;
+    const uint4 e = list[i];
+    const uint64_t ob = tab.begin[e.x] + e.y, ab = tab.alt[e.x] + e.y;
     V *va = nullptr, *vo = nullptr;
     if constexpr (kHasVal<V>) {
-      const uint64_t vb = tab.vbegin[s];
-      vi = v_in + vb;
       va = v_alt + ab;
-      vo = v_out + vb;
+      vo = v_out + tab.vbegin[e.x] + e.y;
     }
-    medium_sort_block<KT, V, BLOCK, IPT>(k_in + b, k_alt + ab, k_out + b, vi, va, vo, len);
+    if (e.w == kSrcAlt) {  // (the passes start from the output)
+      for (uint32_t j = threadIdx.x; j < e.z; j += BLOCK) {
+        k_out[ob + j] = k_alt[ab + j];
+        if constexpr (kHasVal<V>) vo[j] = va[j];
+      }
+      __threadfence_block();
+      __syncthreads();
+    }
+    medium_sort_block<KT, V, BLOCK, IPT>(k_out + ob, k_alt + ab, k_out + ob, vo, va, vo, e.z);
     __syncthreads();
   }
 }
 
-// Large bin: locate tile g among the large segments.
-__device__ __forceinline__ uint32_t find_large(const uint32_t* tile_start, uint32_t n_large, uint32_t g) {
-  uint32_t lo = 0, hi = n_large;  // largest li with tile_start[li] <= g
+// The node of tile g: the last one with tile0 <= g.
+__device__ __forceinline__ uint32_t find_node(const Node* __restrict__ nodes, uint32_t n, uint32_t g) {
+  uint32_t lo = 0, hi = n;
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
-    if (tile_start[mid] <= g)
+    if (nodes[mid].tile0 <= g)
       lo = mid;
     else
       hi = mid;
@@ -404,131 +394,472 @@ __device__ __forceinline__ uint32_t find_large(const uint32_t* tile_start, uint3
   return lo;
 }
 
-template <int KT, int BLOCK, int TILE>
-__global__ __launch_bounds__(BLOCK) void seg_hist_kernel(const typename Codec<KT>::Bits* __restrict__ k_in,
-                                                         SegTab tab, const uint32_t* __restrict__ large_list,
-                                                         const uint32_t* __restrict__ tile_start,
-                                                         uint32_t* __restrict__ seg_hist,
-                                                         const SegCtl* __restrict__ ctl) {
+// A node's digits, and the digit of a key.
+template <typename Bits>
+struct Steps {
+  Bits base, top;
+  uint32_t mul, shift;
+};
+template <int KT>
+__device__ __forceinline__ uint32_t step_digit(typename Codec<KT>::Bits raw, const Steps<typename Codec<KT>::Bits>& st) {
   using Bits = typename Codec<KT>::Bits;
-  constexpr int P = (int)sizeof(Bits);
-  __shared__ uint32_t h[P][kRadix];
-  const uint32_t g = blockIdx.x;
-  if (g >= ctl->large_tiles) return;
-  const int tid = threadIdx.x;
-  for (int i = tid; i < P * kRadix; i += BLOCK) (&h[0][0])[i] = 0;
-  __syncthreads();
-  const uint32_t li = find_large(tile_start, ctl->n_large, g);
-  const uint32_t s = large_list[li];
-  const uint64_t b = tab.begin[s];
-  const uint32_t len = tab.len[s];
-  const uint32_t t0 = (g - tile_start[li]) * (uint32_t)TILE;
-  const uint32_t t1 = min(len, t0 + (uint32_t)TILE);
-  for (uint32_t i = t0 + tid; i < t1; i += BLOCK) {
-    const Bits k = k_in[b + i];
-#pragma unroll
-    for (int p = 0; p < P; ++p) seg_hist_count(&h[0][0], p * kRadix + digit_of<KT>(k, 8 * p));
-  }
-  __syncthreads();
-  uint32_t* dsth = seg_hist + (size_t)li * P * kRadix;
-  for (int i = tid; i < P * kRadix; i += BLOCK) {
-    const uint32_t c = (&h[0][0])[i];
-    if (c) atomicAdd(&dsth[i], c);
-  }
+  const Bits e = Codec<KT>::enc(raw);
+  const uint32_t t = (uint32_t)((Bits)(e - st.base) >> st.shift);
+  uint32_t d = (st.mul ? __umulhi(t, st.mul) : t) + 1u;
+  d = e < st.base ? 0u : d;
+  return e > st.top ? 255u : d;
 }
 
-template <int P>
-__global__ __launch_bounds__(256) void seg_scan_kernel(const uint32_t* seg_hist, uint32_t* seg_base,
-                                                       const SegCtl* __restrict__ ctl) {
-  __shared__ uint32_t sums[4];
-  const uint32_t li = blockIdx.x;
-  if (li >= ctl->n_large) return;
-  const int tid = threadIdx.x;
-  for (int p = 0; p < P; ++p) {
-    const size_t o = ((size_t)li * P + p) * kRadix + tid;
-    const uint32_t c = seg_hist[o];
-    const uint32_t e = block_excl_scan_256(c, sums, tid);
-    __syncthreads();
-    seg_base[o] = e;  // may alias seg_hist: every read of this row is done
-  }
-}
+// ---------------------------------------------------------------------------
+// count: workgroup b takes the tiles [T b / B, T (b + 1) / B) of the level,
+// which mostly share a node; a node's digits are derived anew by every
+// workgroup that meets it (from the same samples) and kept for the scatter by
+// the one with its first tile.
+// whole > 0 (first level only): the call sorts one array of so many records,
+// and workgroup 0 writes what classify would.
+// ---------------------------------------------------------------------------
+constexpr int kCountBlock = 512;
 
-template <int KT, typename V, int BLOCK, int IPT, typename D>
-__global__ __launch_bounds__(BLOCK) void seg_pass_kernel(const typename Codec<KT>::Bits* k_in,
-                                                         typename Codec<KT>::Bits* k_alt,
-                                                         typename Codec<KT>::Bits* k_out, const V* v_in, V* v_alt,
-                                                         V* v_out, SegTab tab,
-                                                         const uint32_t* __restrict__ large_list,
-                                                         const uint32_t* __restrict__ tile_start,
-                                                         const uint32_t* __restrict__ seg_base,
-                                                         uint32_t* __restrict__ tile_counter, D* __restrict__ desc,
-                                                         const SegCtl* __restrict__ ctl, uint32_t* __restrict__ status,
-                                                         int pass) {
+template <int KT>
+__global__ __launch_bounds__(kCountBlock) void seg_count_kernel(const typename Codec<KT>::Bits* __restrict__ src,
+                                                                SegTab tab, const uint64_t* place, Node* nodes,
+                                                                uint32_t* __restrict__ rows, uint32_t tile,
+                                                                SegCtl* ctl, int level, uint32_t whole) {
   using Bits = typename Codec<KT>::Bits;
-  constexpr int P = (int)sizeof(Bits);
-  __shared__ uint32_t s_tile;
-  if (threadIdx.x == 0) s_tile = atomicAdd(&tile_counter[pass], 1u);
-  __syncthreads();
-  const uint32_t g = s_tile;
-  if (g >= ctl->large_tiles) return;
-  const uint32_t li = find_large(tile_start, ctl->n_large, g);
-  const uint32_t s = large_list[li];
-  const uint64_t b = tab.begin[s];
-  const uint64_t ab = tab.alt[s];
-  const uint32_t len = tab.len[s];
-  const Bits* src;
-  Bits* dst;
-  if (pass == 0) {
-    src = k_in + b;
-    dst = k_alt + ab;
-  } else if (pass & 1) {
-    src = k_alt + ab;
-    dst = k_out + b;
-  } else {
-    src = k_out + b;
-    dst = k_alt + ab;
+  constexpr int kSamples = 256;
+  __shared__ Bits smp[kSamples];
+  __shared__ uint32_t rank[kSamples], same[kSamples];
+  __shared__ Bits s_lo, s_hi, s_mid;
+  __shared__ uint32_t s_same;
+  __shared__ uint32_t h[kCountBlock / 128][kRadix];
+  uint32_t n_nodes = 1, n_tiles = (whole + tile - 1) / tile;
+  if (whole == 0) {
+    n_nodes = (uint32_t)(ctl->alloc[level] >> 32);
+    n_tiles = (uint32_t)ctl->alloc[level];
+  } else if (blockIdx.x == 0 && threadIdx.x == 0) {
+    tab.begin[0] = tab.vbegin[0] = tab.alt[0] = 0;
+    tab.len[0] = whole;
+    nodes[0].seg = nodes[0].off = nodes[0].tile0 = 0;
+    nodes[0].len = whole;
+    ctl->status = ctl->skipped = ctl->n_batches = ctl->n_long = 0;
+    ctl->alloc[0] = (uint64_t)1 << 32 | n_tiles;
+    for (int l = 1; l <= kMaxLevels; ++l) ctl->alloc[l] = 0;
   }
-  const V* vsrc = nullptr;
-  V* vdst = nullptr;
-  if constexpr (kHasVal<V>) {
-    const uint64_t vb = tab.vbegin[s];
-    if (pass == 0) {
-      vsrc = v_in + vb;
-      vdst = v_alt + ab;
-    } else if (pass & 1) {
-      vsrc = v_alt + ab;
-      vdst = v_out + vb;
-    } else {
-      vsrc = v_out + vb;
-      vdst = v_alt + ab;
+  const uint32_t g0 = (uint32_t)((uint64_t)n_tiles * blockIdx.x / gridDim.x);
+  const uint32_t g1 = (uint32_t)((uint64_t)n_tiles * (blockIdx.x + 1) / gridDim.x);
+  if (g0 >= g1) return;
+  const int tid = threadIdx.x;
+  uint32_t* const my = h[tid / 128];  // one histogram per two wavefronts
+  uint32_t ni = whole ? 0 : find_node(nodes, n_nodes, g0);
+  bool fresh = true;
+  Steps<Bits> st{};
+  uint32_t len = 0, tile0 = 0;
+  const Bits* keys = nullptr;
+  for (uint32_t g = g0; g < g1; ++g) {
+    if (!fresh && ni + 1 < n_nodes && nodes[ni + 1].tile0 <= g) {
+      ++ni;
+      fresh = true;
     }
+    if (fresh) {
+      fresh = false;
+      keys = src;
+      len = whole;
+      if (whole == 0) {
+        keys += place[nodes[ni].seg] + nodes[ni].off;
+        len = nodes[ni].len;
+        tile0 = nodes[ni].tile0;
+      }
+      if (tid < kSamples) {
+        smp[tid] = Codec<KT>::enc(keys[((uint64_t)tid * (len - 1)) / (kSamples - 1)]);
+        rank[tid] = 0;
+        same[tid] = 0;
+      }
+      __syncthreads();
+      // rank of every sample, half of the others per thread (ties by place)
+      {
+        const int i = tid & (kSamples - 1), from = tid / kSamples * (kSamples / 2);
+        const Bits x = smp[i];
+        uint32_t r = 0, e = 0;
+#pragma unroll 8
+        for (int j = from; j < from + kSamples / 2; ++j) {
+          const bool eq = smp[j] == x;
+          r += (smp[j] < x || (eq && j < i)) ? 1u : 0u;
+          e += eq ? 1u : 0u;
+        }
+        atomicAdd(&rank[i], r);
+        atomicAdd(&same[i], e);
+      }
+      __syncthreads();
+      if (tid < kSamples) {
+        if (rank[tid] == 2) s_lo = smp[tid];
+        if (rank[tid] == kSamples - 3) s_hi = smp[tid];
+        if (rank[tid] == kSamples / 2) {
+          s_mid = smp[tid];
+          s_same = same[tid];
+        }
+      }
+      __syncthreads();
+      // a sixty-fourth of their distance further on both sides; or, where
+      // half of the samples are one value, steps of one from that value on:
+      // its records are done, the others go below and above
+      const bool heavy = s_same >= kSamples / 2;
+      Bits lo = heavy ? s_mid : s_lo, hi = heavy ? s_mid : s_hi;
+      const Bits more = (hi - lo) / 64;
+      lo = lo > more ? lo - more : Bits(0);
+      hi = ~Bits(0) - hi > more ? hi + more : ~Bits(0);
+      st.base = lo;
+      st.top = hi;
+      const Bits range = hi - lo;
+      st.mul = 0;
+      st.shift = 0;
+      if (range > 253) {  // 254 even steps
+        st.shift = (uint32_t)max(bit_width<Bits>(range) - 32, 0);
+        st.mul = (uint32_t)((254ull << 32) / ((uint64_t)(uint32_t)(range >> st.shift) + 1u));
+      }
+      if (tid == 0 && tile0 >= g0) {
+        nodes[ni].base = (uint64_t)st.base;
+        nodes[ni].top = (uint64_t)st.top;
+        nodes[ni].mul = st.mul;
+        nodes[ni].shift = st.shift;
+      }
+    }
+    for (int i = tid; i < (kCountBlock / 128) * kRadix; i += kCountBlock) (&h[0][0])[i] = 0;
+    __syncthreads();
+    const uint32_t t0 = (g - tile0) * tile, t1 = min(len, t0 + tile);
+    uint32_t i = t0 + tid;
+    for (; i + 7 * kCountBlock < t1; i += 8 * kCountBlock) {
+      Bits k[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) k[u] = keys[i + u * kCountBlock];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) lds_count_wave(my, step_digit<KT>(k[u], st));
+    }
+    for (; i < t1; i += kCountBlock) lds_count_wave(my, step_digit<KT>(keys[i], st));
+    __syncthreads();
+    if (tid < kRadix) {
+      uint32_t s = 0;
+#pragma unroll
+      for (int q = 0; q < kCountBlock / 128; ++q) s += h[q][tid];
+      rows[(size_t)g * kRadix + tid] = s;
+    }
+    __syncthreads();
   }
-  const uint32_t t0 = tile_start[li];
-  onesweep_tile<KT, V, BLOCK, IPT, D>(src, dst, vsrc, vdst, len, len, g - t0, desc + (size_t)t0 * kRadix,
-                                      seg_base + ((size_t)li * P + pass) * kRadix, pass * 8, pass & 1, status);
+}
+
+// ---------------------------------------------------------------------------
+// scan: one workgroup of PARTS * 256 threads per node; thread (q, d) has
+// digit d of the q-th part of the node's tiles.  The rows become the offsets
+// inside the node of each tile's digits.  Then the first 256 threads dispose
+// of the children.  PARTS = 4 for the first level, whose segments have up to
+// hundreds of tiles, 1 for the later ones, whose nodes are many and short.
+// ---------------------------------------------------------------------------
+template <int PARTS>
+__global__ __launch_bounds__(PARTS * kRadix) void seg_scan_kernel(const Node* __restrict__ nodes,
+                                                                  uint32_t* __restrict__ rows, uint32_t tile,
+                                                                  uint32_t cap, uint32_t dst, int last,
+                                                                  Node* __restrict__ next, uint4* __restrict__ batches,
+                                                                  uint4* __restrict__ longs, SegCtl* __restrict__ ctl,
+                                                                  int level) {
+  __shared__ uint32_t part[PARTS][kRadix];
+  __shared__ uint32_t s_off[kRadix + 1], s_step[kRadix];
+  __shared__ uint32_t sums[4], sums2[4], sums3[4];
+  __shared__ uint64_t s_own[kRadix / kWave], s_cut[kRadix / kWave];
+  __shared__ uint32_t s_max, s_batch, s_long;
+  __shared__ uint64_t s_next;
+  const int tid = threadIdx.x, q = tid / kRadix, d = tid & (kRadix - 1), lane = tid & (kWave - 1);
+  const uint32_t n_nodes = (uint32_t)(ctl->alloc[level] >> 32);
+  for (uint32_t ni = blockIdx.x; ni < n_nodes; ni += gridDim.x) {
+    const Node nd = nodes[ni];
+    const uint32_t nt = (nd.len + tile - 1) / tile;
+    uint32_t* const col = rows + (size_t)nd.tile0 * kRadix + d;
+    const uint32_t a = (uint32_t)((uint64_t)nt * q / PARTS), b = (uint32_t)((uint64_t)nt * (q + 1) / PARTS);
+    uint32_t sum = 0, t = a;
+    for (; t + 8 <= b; t += 8) {
+      uint32_t c[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) c[u] = col[(size_t)(t + u) * kRadix];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) sum += c[u];
+    }
+    for (; t < b; ++t) sum += col[(size_t)t * kRadix];
+    part[q][d] = sum;
+    if (tid == 0) s_max = 0;
+    __syncthreads();
+    uint32_t cnt = 0;
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i) cnt += part[i][d];
+    const uint32_t excl = block_excl_scan_256(tid < kRadix ? cnt : 0u, sums, tid);
+    if (tid < kRadix) s_off[d] = excl;
+    if (tid == 0) s_off[kRadix] = nd.len;
+    // Children longer than the cap are done if every key is the same (equal: a
+    // step of one value) or split again (big).  The others are batched where
+    // floor(offset / T) agrees, T = cap - (the largest of them up to cap / 2; a
+    // longer one is a batch by itself), so that a batch fits the cap.
+    const bool child = tid < kRadix && cnt > 0;
+    const bool over = child && cnt > cap;
+    const bool equal = over && nd.mul == 0 && d >= 1 && d <= 254;
+    const bool big = over && !equal;
+    const bool own = over || (child && cnt > cap / 2);  // not batched with others
+    if (tid < kRadix) {
+      const uint64_t m = ballot64(own);
+      if (lane == 0) s_own[d / kWave] = m;
+      if (child && !own) atomicMax(&s_max, cnt);
+    }
+    __syncthreads();
+    {
+      uint32_t run = s_off[d];
+      for (int i = 0; i < q; ++i) run += part[i][d];
+      for (t = a; t + 8 <= b; t += 8) {
+        uint32_t c[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) c[u] = col[(size_t)(t + u) * kRadix];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          col[(size_t)(t + u) * kRadix] = run;
+          run += c[u];
+        }
+      }
+      for (; t < b; ++t) {
+        const uint32_t c = col[(size_t)t * kRadix];
+        col[(size_t)t * kRadix] = run;
+        run += c;
+      }
+    }
+    const uint32_t T = cap - s_max;
+    const uint32_t step = excl / T;
+    if (tid < kRadix) s_step[d] = step;
+    __syncthreads();
+    // a batch starts at every child of its own, behind it, and where the step
+    // changes; it ends where the next one starts
+    bool cut = false;
+    if (tid < kRadix) {
+      cut = d == 0 || own || ((s_own[(d - 1) / kWave] >> ((d - 1) & (kWave - 1))) & 1u) || s_step[d - 1] != step;
+      const uint64_t m = ballot64(cut);
+      if (lane == 0) s_cut[d / kWave] = m;
+    }
+    __syncthreads();
+    uint32_t end = kRadix;
+    if (cut) {
+      uint64_t m = s_cut[d / kWave] >> 1 >> lane;
+      if (m) {
+        end = d + 1 + (uint32_t)__builtin_ctzll(m);
+      } else {
+        for (int i = d / kWave + 1; i < kRadix / kWave; ++i)
+          if (s_cut[i]) {
+            end = i * kWave + (uint32_t)__builtin_ctzll(s_cut[i]);
+            break;
+          }
+      }
+    }
+    const uint32_t len = cut ? s_off[end] - excl : 0u;
+    // batches of the local sort; an equal child in the scratch is cut into
+    // caps to be copied to the output
+    uint32_t nb = cut && len > 0 && !over ? 1u : 0u;
+    if (equal && dst != kSrcOut) nb = (cnt + cap - 1) / cap;
+    const uint32_t bigs = big ? 1u : 0u, bigt = big && !last ? (cnt + tile - 1) / tile : 0u;
+    const uint32_t eb = block_excl_scan_256(nb, sums, tid);
+    const uint32_t en = block_excl_scan_256(bigs, sums2, tid);
+    const uint32_t et = block_excl_scan_256(bigt, sums3, tid);
+    if (tid == kRadix - 1) {
+      if (eb + nb) s_batch = atomicAdd(&ctl->n_batches, eb + nb);
+      if (en + bigs) {
+        if (last)
+          s_long = atomicAdd(&ctl->n_long, en + bigs);
+        else
+          s_next = atomicAdd(reinterpret_cast<unsigned long long*>(&ctl->alloc[level + 1]),
+                             (unsigned long long)(en + bigs) << 32 | (et + bigt));
+      }
+    }
+    __syncthreads();
+    if (big) {
+      if (last)
+        longs[s_long + en] = make_uint4(nd.seg, nd.off + excl, cnt, dst);
+      else
+        next[(uint32_t)(s_next >> 32) + en] = Node{nd.seg, nd.off + excl, cnt, (uint32_t)s_next + et, 0, 0, 0, 0};
+    } else if (equal) {
+      for (uint32_t i = 0; i < nb; ++i)
+        batches[s_batch + eb + i] = make_uint4(nd.seg, nd.off + excl + i * cap, min(cap, cnt - i * cap), dst);
+    } else if (nb) {
+      batches[s_batch + eb] = make_uint4(nd.seg, nd.off + excl, len, dst);
+    }
+    __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------------------
+// scatter: a workgroup takes tiles of its XCD's part of the level: ranks its
+// records by digit in LDS, stages them in digit order and writes every digit's
+// run to the tile's offset (rows).  Bound by HBM: one read and one write of
+// every record.
+// ---------------------------------------------------------------------------
+template <int KT, typename V, int BLOCK, int IPT, int WAVES>
+__global__ __launch_bounds__(BLOCK, WAVES) void seg_scatter_kernel(
+    const typename Codec<KT>::Bits* __restrict__ src, const V* __restrict__ vsrc, typename Codec<KT>::Bits* __restrict__ dst,
+    V* __restrict__ vdst, const uint64_t* __restrict__ sp, const uint64_t* __restrict__ svp,
+    const uint64_t* __restrict__ dp, const uint64_t* __restrict__ dvp, const Node* __restrict__ nodes,
+    const uint32_t* __restrict__ rows, const SegCtl* __restrict__ ctl, int level) {
+  using Bits = typename Codec<KT>::Bits;
+  constexpr int W = BLOCK / kWave;
+  constexpr int TILE = BLOCK * IPT;
+  constexpr bool HV = kHasVal<V>;
+  using VS = typename std::conditional<HV, V, uint32_t>::type;
+  __shared__ Bits keys[TILE];
+  __shared__ VS vstage[HV ? TILE : 1];
+  __shared__ uint32_t off[W][kRadix];
+  __shared__ uint32_t gbase[kRadix];
+  __shared__ uint32_t sums[4];
+  const uint32_t n_nodes = (uint32_t)(ctl->alloc[level] >> 32), n_tiles = (uint32_t)ctl->alloc[level];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), w = (int)readfirstlane((uint32_t)(tid / kWave));
+  for (int i = lane; i < kRadix; i += kWave) off[w][i] = 0;
+  // Workgroups b, b + 8, ... run on one XCD: its eighth of the tiles is one
+  // stretch, so that the ends of neighbouring tiles' runs meet in one L2.
+  const uint32_t groups = min(kXcds, gridDim.x), x = blockIdx.x % groups, j0 = blockIdx.x / groups;
+  const uint32_t stride = (gridDim.x - x + groups - 1) / groups;
+  const uint32_t first = (uint32_t)((uint64_t)n_tiles * x / groups), stop = (uint32_t)((uint64_t)n_tiles * (x + 1) / groups);
+  for (uint32_t g = first + j0; g < stop; g += stride) {
+    const Node nd = nodes[find_node(nodes, n_nodes, g)];
+    const Steps<Bits> st{(Bits)nd.base, (Bits)nd.top, nd.mul, nd.shift};
+    const uint32_t t0 = (g - nd.tile0) * (uint32_t)TILE;
+    const uint32_t cnt = min((uint32_t)TILE, nd.len - t0);
+    const bool full = cnt == (uint32_t)TILE;
+    const Bits* in = src + sp[nd.seg] + nd.off + t0;
+    const uint32_t wb = (uint32_t)(w * IPT * kWave + lane);
+    const uint32_t row = tid < kRadix ? rows[(size_t)g * kRadix + tid] : 0u;
+    Bits k[IPT];
+    VS v[IPT];
+    if (full) {
+      static_for<IPT>([&](auto i) { k[i] = in[wb + i * kWave]; });
+    } else {
+      static_for<IPT>([&](auto i) { k[i] = wb + i * kWave < cnt ? in[wb + i * kWave] : Bits(0); });
+    }
+    if constexpr (HV) {
+      const V* vin = vsrc + svp[nd.seg] + nd.off + t0;
+      if (full) {
+        static_for<IPT>([&](auto i) { v[i] = vin[wb + i * kWave]; });
+      } else {
+        static_for<IPT>([&](auto i) { v[i] = wb + i * kWave < cnt ? vin[wb + i * kWave] : VS(0); });
+      }
+    }
+    uint32_t r[IPT];
+    uint32_t* const ct = off[w];
+    if (full) {
+      const uint32_t d0 = step_digit<KT>(k[0], st);
+      if (__popcll(ballot64(d0 == readfirstlane(d0))) >= 16) {
+        static_for<IPT>([&](auto i) { r[i] = rank_wave_atomic<true>(step_digit<KT>(k[i], st), ct); });
+      } else {
+        static_for<IPT>([&](auto i) { r[i] = rank_wave_atomic<false>(step_digit<KT>(k[i], st), ct); });
+      }
+    } else {
+      static_for<IPT>([&](auto i) {
+        r[i] = 0;
+        if (wb + i * kWave < cnt) r[i] = rank_wave_atomic<true>(step_digit<KT>(k[i], st), ct);
+      });
+    }
+    __syncthreads();
+    uint32_t total = 0;
+    if (tid < kRadix) {
+#pragma unroll
+      for (int i = 0; i < W; ++i) total += off[i][tid];
+    }
+    const uint32_t excl = block_excl_scan_256(total, sums, tid);
+    if (tid < kRadix) {
+      uint32_t run = excl;
+#pragma unroll
+      for (int i = 0; i < W; ++i) {
+        const uint32_t c = off[i][tid];
+        off[i][tid] = run;
+        run += c;
+      }
+      gbase[tid] = row - excl;
+    }
+    __syncthreads();
+    static_for<IPT>([&](auto i) { r[i] += ct[step_digit<KT>(k[i], st)]; });
+    static_for<IPT>([&](auto i) {
+      if (full || wb + i * kWave < cnt) {
+        keys[r[i]] = k[i];
+        if constexpr (HV) vstage[r[i]] = v[i];
+      }
+    });
+    for (int i = lane; i < kRadix; i += kWave) off[w][i] = 0;
+    __syncthreads();
+    // a corrupted offset stays inside the node
+    const uint32_t top = nd.len - 1;
+    Bits* const ko = dst + dp[nd.seg] + nd.off;
+    V* vo = nullptr;
+    if constexpr (HV) vo = vdst + dvp[nd.seg] + nd.off;
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+      const uint32_t i = (uint32_t)(j * BLOCK + tid);
+      if (full || i < cnt) {
+        const Bits kk = keys[i];
+        const uint32_t o = min(gbase[step_digit<KT>(kk, st)] + i, top);
+        ko[o] = kk;
+        if constexpr (HV) vo[o] = vstage[i];
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// ---------------------------------------------------------------------------
+// local: workgroup b sorts the batches b, b + B, ... in LDS
+// ---------------------------------------------------------------------------
+template <int KT, typename V, int BLOCK, int IPT, int WAVES>
+__global__ __launch_bounds__(BLOCK, WAVES) void seg_local_kernel(const typename Codec<KT>::Bits* k_in,
+                                                                 const typename Codec<KT>::Bits* k_alt,
+                                                                 typename Codec<KT>::Bits* k_out, const V* v_in,
+                                                                 const V* v_alt, V* v_out, SegTab tab,
+                                                                 const uint4* __restrict__ batches,
+                                                                 const SegCtl* __restrict__ ctl) {
+  using Bits = typename Codec<KT>::Bits;
+  using Smem = BlockSortSmem<Bits, V, BLOCK, IPT>;
+  using VS = typename Smem::VS;
+  __shared__ Smem sm;
+  const uint32_t total = ctl->n_batches;
+  block_clear_row<BLOCK>(sm.off);
+  for (uint32_t bi = blockIdx.x; bi < total; bi += gridDim.x) {
+    const uint4 e = batches[bi];
+    const uint32_t m = readfirstlane(e.z);
+    if (m == 0) continue;
+    const uint64_t ob = tab.begin[e.x] + e.y;
+    const uint64_t ab = tab.alt[e.x] + e.y;
+    const Bits* kb = e.w == kSrcIn ? k_in + ob : e.w == kSrcAlt ? k_alt + ab : k_out + ob;
+    const uint32_t nit = block_items<BLOCK>(m), wb = block_first<BLOCK>(nit);
+    Bits k[IPT];
+    VS v[IPT];
+    static_for<IPT>([&](auto i) {
+      k[i] = 0;
+      if (wb + i * kWave < m && (uint32_t)i < nit) k[i] = kb[wb + i * kWave];
+    });
+    V* vo = nullptr;
+    if constexpr (kHasVal<V>) {
+      const uint64_t vb = tab.vbegin[e.x] + e.y;
+      const V* vs = e.w == kSrcIn ? v_in + vb : e.w == kSrcAlt ? v_alt + ab : v_out + vb;
+      vo = v_out + vb;
+      static_for<IPT>([&](auto i) {
+        v[i] = 0;
+        if (wb + i * kWave < m && (uint32_t)i < nit) v[i] = vs[wb + i * kWave];
+      });
+    }
+    Bits mn, mx;
+    block_min_max<KT, V, BLOCK, IPT>(sm, k, wb, m, nit, mn, mx);
+    const Bits pad = block_pad<KT>(mx);
+    static_for<IPT>([&](auto i) { k[i] = wb + i * kWave < m ? k[i] : pad; });
+    block_sort<KT, V, BLOCK, IPT>(sm, k, v, m, mn, mx, k_out + ob, vo);
+    __syncthreads();
+  }
 }
 
 constexpr size_t kAlign = 256;
 inline size_t align_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
 
 struct SegLayout {
-  size_t alt_k, alt_v, ctl, tab_begin, tab_vbegin, tab_alt, tab_len, small_list, medium_list, large_list, tile_start, seg_hist,
-      seg_base, tile_counter, desc, total;
-  uint32_t max_large, tiles_ub;
-  bool wide_desc;
+  size_t ctl, alt_k, alt_v, tab_begin, tab_vbegin, tab_alt, tab_len, nodes[kMaxLevels], batches, longs, rows, total;
+  uint32_t nodes_ub[kMaxLevels], tiles_ub[kMaxLevels], batches_ub;
+  int levels;
 };
 
-// Items per thread of the large segments' tiles for 8- and 12-byte records
-// and for 16-byte ones (one workgroup per CU; 20 and 14 measured 24% faster
-// than 8 and 4 on 4096 arrays of u64 keys with a u32 payload).
-#ifndef MGS_SEG_IPT_WIDE
-#define MGS_SEG_IPT_WIDE 20
-#endif
-#ifndef MGS_SEG_IPT_WIDE16
-#define MGS_SEG_IPT_WIDE16 14
-#endif
-
-// Tile geometries of the large segments' passes, chosen per call by
+// Tile geometries of the scatter, chosen per call by
 // mgs_tuning::large_variant (0 = the default; the autotuner times all of
 // them per record width, payload and size):
 //   record   variant 0        variant 1          variant 2
@@ -537,7 +868,7 @@ struct SegLayout {
 //   12 B     512 x 20         512 x 16           512 x 12
 //   16 B     512 x 14         512 x 12           512 x 8
 // (threads x items per thread).  Variant 0: 16 items per thread for 4-byte
-// keys (two workgroups per CU); wider records use the LDS of a whole CU, as
+// keys (four workgroups per CU); wider records use the LDS of a whole CU, as
 // the plain sort's large tiles do.  Variant 1 of the 4-byte keys is the
 // plain sort's tile; the others trade tile size for occupancy.
 constexpr int kSegVariants = 3;
@@ -546,10 +877,13 @@ struct SegLargeGeom {
   static constexpr int kRec = KB + VB;
   static constexpr int kBlock = (kRec <= 4 && VAR == 1) ? 1024 : 512;
   static constexpr int kIpt = kRec <= 4    ? (VAR == 0 ? 16 : VAR == 1 ? 18 : 8)
-                              : kRec <= 8  ? (VAR == 0 ? MGS_SEG_IPT_WIDE : VAR == 1 ? 28 : 12)
-                              : kRec <= 12 ? (VAR == 0 ? MGS_SEG_IPT_WIDE : VAR == 1 ? 16 : 12)
-                                           : (VAR == 0 ? MGS_SEG_IPT_WIDE16 : VAR == 1 ? 12 : 8);
+                              : kRec <= 8  ? (VAR == 0 ? 20 : VAR == 1 ? 28 : 12)
+                              : kRec <= 12 ? (VAR == 0 ? 20 : VAR == 1 ? 16 : 12)
+                                           : (VAR == 0 ? 14 : VAR == 1 ? 12 : 8);
   static constexpr int kTile = kBlock * kIpt;
+  // wavefronts per SIMD: 1024-thread workgroups and tiles that leave the LDS
+  // to a second workgroup run four, the others two
+  static constexpr int kWaves = kBlock == 1024 || kTile * kRec <= 66 * 1024 ? 4 : 2;
 };
 
 template <int KB, int VB>
@@ -563,56 +897,65 @@ inline int seg_large_tile(int var) {
 
 template <int KB, int VB>
 struct SegCfg {
-  // one workgroup per medium segment streams it through tiles of this size
+  // one workgroup per long range streams it through tiles of this size
   using M = TileCfg<KB, VB, 16, 8, 8, 4, 4, MGS_OS_BLOCK>;
-  using S = SmallCfg<KB, VB>;
-  static constexpr int kSmallMax = S::kTile;
-  static constexpr int kMediumMax = 1 << 17;
+  // local sort: 512 threads, three workgroups per CU for 4-byte records, two
+  // for wider ones: as many items as leave none in scratch registers at that
+  // occupancy
+  static constexpr int kRec = KB + VB;
+  static constexpr int kLocalBlock = 512;
+  static constexpr int kLocalIpt = kRec <= 4 ? 16 : kRec <= 8 ? 14 : kRec <= 12 ? 10 : 7;
+  static constexpr int kLocalWaves = kRec <= 4 ? 6 : 4;
+  static constexpr uint32_t kCap = (uint32_t)kLocalBlock * kLocalIpt;
 };
 
-// Large segments always hold more than kMinLargeExclusive keys, whatever the
-// tuning, so the scratch size depends only on (max_total, nseg).
-constexpr uint32_t kMinLargeExclusive = 256;
+// Nodes of the first level hold more than kMinSplit records, whatever the
+// tuning, so the scratch size depends only on the sizes and the variant.
+constexpr uint32_t kMinSplit = 256;
 
+// wide_range: doubles.
 template <int KB, int VB>
-SegLayout seg_layout(size_t max_total, size_t nseg, size_t max_seg, int large_tile) {
-  constexpr int P = KB;
+SegLayout seg_layout(size_t max_total, size_t nseg, size_t max_seg, int large_tile, bool wide_range) {
+  constexpr size_t cap = SegCfg<KB, VB>::kCap;
   SegLayout L{};
-  L.max_large = (uint32_t)std::min<size_t>(nseg, max_total / (kMinLargeExclusive + 1) + 1);
-  L.tiles_ub = (uint32_t)(max_total / (size_t)large_tile + L.max_large + 1);
-  // descriptor values are prefixes inside one segment: 30 bits hold them
-  // unless a segment may reach 2^30 keys
-  L.wide_desc = max_seg >= (size_t(1) << 30);
+  // Levels of splitting: two reach the cap for segments up to 2^20 records
+  // unless their keys are skewed on more than two scales (the long kernel
+  // then takes what is left); longer ones get a third, and so do doubles from
+  // 2^15 on, whose encoded range around zero spans 2000 exponents (normal
+  // doubles, 2^20: 243 us with two levels and the long kernel).
+  L.levels = max_seg > (wide_range ? size_t(1) << 15 : size_t(1) << 20) ? 3 : 2;
+  // a batch that a node's children form holds more than cap / 2 records on
+  // average but for one per node and the breaks at children above cap / 2
+  // (at most two per such child); equal children are cut into caps
+  size_t nodes = 0;
+  for (int l = 0; l < L.levels; ++l) {
+    L.nodes_ub[l] = (uint32_t)(l == 0 ? std::min<size_t>(nseg, max_total / (kMinSplit + 1) + 1) : max_total / (cap + 1) + 1);
+    L.tiles_ub[l] = (uint32_t)(max_total / (size_t)large_tile + L.nodes_ub[l] + 1);
+    nodes += L.nodes_ub[l];
+  }
+  const size_t per_level = 8 * (max_total / cap + 1);
+  L.batches_ub = (uint32_t)(nseg + 2 * nodes + L.levels * per_level);
   size_t o = 0;
-  L.ctl = o;  // first: its status word is the call's status word
-  o = align_up(o + sizeof(SegCtl));
-  L.alt_k = o;
-  o = align_up(o + max_total * KB);
-  L.alt_v = o;
-  o = align_up(o + max_total * VB);
-  L.tab_begin = o;
-  o = align_up(o + nseg * 8);
-  L.tab_vbegin = o;
-  o = align_up(o + nseg * 8);
-  L.tab_alt = o;
-  o = align_up(o + nseg * 8);
-  L.tab_len = o;
-  o = align_up(o + nseg * 4);
-  L.small_list = o;
-  o = align_up(o + nseg * 4);
-  L.medium_list = o;
-  o = align_up(o + nseg * 4);
-  L.large_list = o;
-  o = align_up(o + nseg * 4);
-  L.tile_start = o;
-  o = align_up(o + (nseg + 1) * 4);
-  L.seg_hist = o;  // histograms, scanned in place into digit bases
-  o = align_up(o + (size_t)L.max_large * P * kRadix * 4);
-  L.seg_base = L.seg_hist;
-  L.tile_counter = o;
-  o = align_up(o + (kMaxPasses + 1) * 4);
-  L.desc = o;
-  o = align_up(o + (size_t)L.tiles_ub * kRadix * (L.wide_desc ? 8 : 4));
+  auto take = [&](size_t bytes) {
+    const size_t at = o;
+    o = align_up(o + bytes);
+    return at;
+  };
+  L.ctl = take(sizeof(SegCtl));  // first: its status word is the call's status word
+  L.alt_k = take(max_total * KB);
+  L.alt_v = take(max_total * VB);
+  L.tab_begin = take(nseg * 8);
+  L.tab_vbegin = take(nseg * 8);
+  L.tab_alt = take(nseg * 8);
+  L.tab_len = take(nseg * 4);
+  uint32_t tiles = 0;
+  for (int l = 0; l < L.levels; ++l) {
+    L.nodes[l] = take((size_t)L.nodes_ub[l] * sizeof(Node));
+    tiles = std::max(tiles, L.tiles_ub[l]);
+  }
+  L.batches = take((size_t)L.batches_ub * 16);
+  L.longs = take((max_total / (cap + 1) + 1) * 16);
+  L.rows = take((size_t)tiles * kRadix * 4);
   L.total = o;
   return L;
 }
@@ -628,28 +971,22 @@ inline size_t segment_bound(size_t max_total, const mgs_tuning* tuning) {
 
 inline int large_variant_of(const mgs_tuning* tuning) { return tuning != nullptr ? tuning->large_variant : 0; }
 
-// The large segments' histogram, scan and passes with the tile geometry of
-// variant VAR.
-template <int KT, int VT, int VAR>
-void seg_large(const typename Codec<KT>::Bits* ki, typename Codec<KT>::Bits* ka, typename Codec<KT>::Bits* ko,
-               const typename ValOf<VT>::T* vi, typename ValOf<VT>::T* va, typename ValOf<VT>::T* vo,
-               const SegTab& tab, const uint32_t* large_list, const uint32_t* tile_start, uint32_t* seg_hist,
-               uint32_t* seg_base, uint32_t* tcount, void* desc, SegCtl* ctl, const SegLayout& L, hipStream_t s) {
-  using V = typename ValOf<VT>::T;
-  constexpr int KB = sizeof(typename Codec<KT>::Bits);
-  constexpr int VB = kValBytes<V>;
-  constexpr int P = KB;
-  using G = SegLargeGeom<KB, VB, VAR>;
-  seg_hist_kernel<KT, 256, G::kTile><<<L.tiles_ub, 256, 0, s>>>(ki, tab, large_list, tile_start, seg_hist, ctl);
-  seg_scan_kernel<P><<<L.max_large, 256, 0, s>>>(seg_hist, seg_base, ctl);
-  for (int p = 0; p < P; ++p) {
-    if (L.wide_desc)
-      seg_pass_kernel<KT, V, G::kBlock, G::kIpt, uint64_t><<<L.tiles_ub, G::kBlock, 0, s>>>(
-          ki, ka, ko, vi, va, vo, tab, large_list, tile_start, seg_base, tcount, (uint64_t*)desc, ctl, &ctl->status, p);
-    else
-      seg_pass_kernel<KT, V, G::kBlock, G::kIpt, uint32_t><<<L.tiles_ub, G::kBlock, 0, s>>>(
-          ki, ka, ko, vi, va, vo, tab, large_list, tile_start, seg_base, tcount, (uint32_t*)desc, ctl, &ctl->status, p);
-  }
+// Workgroups of `kernel` resident on the device; cached per (kernel, device)
+// so that graph capture issues no queries.
+template <typename K>
+uint32_t seg_resident(K kernel, int block) {
+  static std::mutex mu;
+  static std::map<std::pair<const void*, int>, uint32_t> cache;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  const auto key = std::make_pair(reinterpret_cast<const void*>(kernel), dev);
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = cache.find(key);
+  if (it != cache.end()) return it->second;
+  int cus = 0, per_cu = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 256;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, 0) != hipSuccess) return 256;
+  return cache[key] = (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, cus);
 }
 
 template <int KT, int VT>
@@ -659,69 +996,99 @@ int seg_typed(const void* kin, void* kout, const void* vin, void* vout, const ui
   using V = typename ValOf<VT>::T;
   constexpr int KB = sizeof(Bits);
   constexpr int VB = kValBytes<V>;
-  constexpr int P = KB;
   using C = SegCfg<KB, VB>;
-  using SC = typename C::S;
   using VP = typename std::conditional<kHasVal<V>, V, uint32_t>::type;
 
-  uint32_t small_max = C::kSmallMax, medium_max = C::kMediumMax;
-  if (tuning) {
-    if (tuning->small_max > 0) small_max = std::min<uint32_t>((uint32_t)tuning->small_max, C::kSmallMax);
-    if (tuning->medium_max > 0) medium_max = (uint32_t)tuning->medium_max;
-  }
-  medium_max = std::max({medium_max, small_max, kMinLargeExclusive});
+  // the longest segment that one workgroup sorts: the larger of the caller's
+  // two single-workgroup limits, as many as fit its LDS by default
+  uint32_t small_max = C::kCap;
+  if (tuning && tuning->small_max > 0 && tuning->medium_max > 0)
+    small_max = std::min<uint32_t>((uint32_t)std::max(tuning->small_max, tuning->medium_max), C::kCap);
+  small_max = std::max(small_max, kMinSplit);
   const size_t max_seg = segment_bound(max_total, tuning);
   const int var = large_variant_of(tuning);
   if (var < 0 || var >= kSegVariants) return MGS_ERR_INVALID;
-  const int large_tile = seg_large_tile<KB, VB>(var);
-  const SegLayout L = seg_layout<KB, VB>(max_total, nseg, max_seg, large_tile);
+  const uint32_t tile = (uint32_t)seg_large_tile<KB, VB>(var);
+  const SegLayout L = seg_layout<KB, VB>(max_total, nseg, max_seg, (int)tile, KT == MGS_KEY_F64);
   if (temp == nullptr || temp_bytes < L.total) return MGS_ERR_TEMP_TOO_SMALL;
   char* t = static_cast<char*>(temp);
   Bits* ka = reinterpret_cast<Bits*>(t + L.alt_k);
-  VP* va = reinterpret_cast<VP*>(t + L.alt_v);
+  V* va = reinterpret_cast<V*>(reinterpret_cast<VP*>(t + L.alt_v));
   SegCtl* ctl = reinterpret_cast<SegCtl*>(t + L.ctl);
-  uint32_t* small_list = reinterpret_cast<uint32_t*>(t + L.small_list);
-  uint32_t* medium_list = reinterpret_cast<uint32_t*>(t + L.medium_list);
-  uint32_t* large_list = reinterpret_cast<uint32_t*>(t + L.large_list);
-  uint32_t* tile_start = reinterpret_cast<uint32_t*>(t + L.tile_start);
-  uint32_t* seg_hist = reinterpret_cast<uint32_t*>(t + L.seg_hist);
-  uint32_t* seg_base = reinterpret_cast<uint32_t*>(t + L.seg_base);
-  uint32_t* tcount = reinterpret_cast<uint32_t*>(t + L.tile_counter);
-  void* desc = t + L.desc;
+  uint4* batches = reinterpret_cast<uint4*>(t + L.batches);
+  uint4* longs = reinterpret_cast<uint4*>(t + L.longs);
+  uint32_t* rows = reinterpret_cast<uint32_t*>(t + L.rows);
+  Node* nodes[kMaxLevels];
+  for (int l = 0; l < L.levels; ++l) nodes[l] = reinterpret_cast<Node*>(t + L.nodes[l]);
   const SegTab tab{reinterpret_cast<uint64_t*>(t + L.tab_begin), reinterpret_cast<uint64_t*>(t + L.tab_vbegin),
                    reinterpret_cast<uint64_t*>(t + L.tab_alt), reinterpret_cast<uint32_t*>(t + L.tab_len)};
-
   const Bits* ki = static_cast<const Bits*>(kin);
   Bits* ko = static_cast<Bits*>(kout);
   const V* vi = static_cast<const V*>(vin);
   V* vo = static_cast<V*>(vout);
 
-  if (ranges)
-    seg_classify_kernel<true><<<1, kClassifyBlock, 0, s>>>(bounds, val_begin, (uint32_t)nseg, max_total, max_seg, small_max, medium_max,
-                                                           (uint32_t)large_tile, tab, small_list, medium_list, large_list,
-                                                           tile_start, ctl, tcount);
-  else
-    seg_classify_kernel<false><<<1, kClassifyBlock, 0, s>>>(bounds, val_begin, (uint32_t)nseg, max_total, max_seg, small_max, medium_max,
-                                                            (uint32_t)large_tile, tab, small_list, medium_list, large_list,
-                                                            tile_start, ctl, tcount);
-  seg_clear_kernel<<<2048, 256, 0, s>>>(seg_hist, P * kRadix, (uint32_t*)desc, kRadix * (L.wide_desc ? 2 : 1), ctl);
-  {
-    const unsigned grid = (unsigned)std::min<size_t>(nseg, 8192);
-    seg_small_kernel<KT, V, SC::kBlock, SC::kIpt><<<grid, SC::kBlock, 0, s>>>(ki, ko, vi, vo, tab, small_list, ctl);
+  // (no bounds: one array, of more records than one workgroup sorts)
+  const uint32_t whole = bounds == nullptr ? (uint32_t)max_total : 0u;
+  if (bounds == nullptr && max_total <= small_max) return MGS_ERR_INVALID;
+  if (bounds != nullptr && ranges)
+    seg_classify_kernel<true><<<1, kClassifyBlock, 0, s>>>(bounds, val_begin, (uint32_t)nseg, max_total, max_seg,
+                                                           small_max, tile, tab, batches, nodes[0], ctl);
+  else if (bounds != nullptr)
+    seg_classify_kernel<false><<<1, kClassifyBlock, 0, s>>>(bounds, val_begin, (uint32_t)nseg, max_total, max_seg,
+                                                            small_max, tile, tab, batches, nodes[0], ctl);
+  // level l reads the input, the scratch, the output and writes the scratch,
+  // the output, the scratch
+  auto level = [&](int l, auto scatter, int block) {
+    const bool from_alt = l == 1, to_alt = l != 1;
+    const Bits* ks = l == 0 ? ki : from_alt ? ka : ko;
+    const V* vs = l == 0 ? vi : from_alt ? va : vo;
+    const uint64_t* sp = from_alt ? tab.alt : tab.begin;
+    const uint64_t* svp = from_alt ? tab.alt : tab.vbegin;
+    const uint64_t* dp = to_alt ? tab.alt : tab.begin;
+    const uint64_t* dvp = to_alt ? tab.alt : tab.vbegin;
+    auto count = seg_count_kernel<KT>;
+    count<<<std::min(L.tiles_ub[l], seg_resident(count, kCountBlock)), kCountBlock, 0, s>>>(
+        ks, tab, sp, nodes[l], rows, tile, ctl, l, l == 0 ? whole : 0u);
+    const bool last = l + 1 == L.levels;
+    const uint32_t to = to_alt ? kSrcAlt : kSrcOut;
+    if (l == 0)
+      seg_scan_kernel<4><<<std::min(L.nodes_ub[l], 512u), 4 * kRadix, 0, s>>>(nodes[l], rows, tile, C::kCap, to, last ? 1 : 0,
+                                                                             last ? nullptr : nodes[l + 1], batches,
+                                                                             longs, ctl, l);
+    else
+      seg_scan_kernel<1><<<std::min(L.nodes_ub[l], 2048u), kRadix, 0, s>>>(nodes[l], rows, tile, C::kCap, to, last ? 1 : 0,
+                                                                         last ? nullptr : nodes[l + 1], batches, longs,
+                                                                         ctl, l);
+    scatter<<<std::min(L.tiles_ub[l], seg_resident(scatter, block)), block, 0, s>>>(
+        ks, vs, to_alt ? ka : ko, to_alt ? va : vo, sp, svp, dp, dvp, nodes[l], rows, ctl, l);
+  };
+  if (max_seg > small_max) {
+    for (int l = 0; l < L.levels; ++l) {
+      switch (var) {
+        case 1: {
+          using G = SegLargeGeom<KB, VB, 1>;
+          level(l, seg_scatter_kernel<KT, V, G::kBlock, G::kIpt, G::kWaves>, G::kBlock);
+          break;
+        }
+        case 2: {
+          using G = SegLargeGeom<KB, VB, 2>;
+          level(l, seg_scatter_kernel<KT, V, G::kBlock, G::kIpt, G::kWaves>, G::kBlock);
+          break;
+        }
+        default: {
+          using G = SegLargeGeom<KB, VB, 0>;
+          level(l, seg_scatter_kernel<KT, V, G::kBlock, G::kIpt, G::kWaves>, G::kBlock);
+        }
+      }
+    }
     using MC = typename C::M;
-    seg_medium_kernel<KT, V, MC::kBlock, MC::kIpt>
-        <<<grid, MC::kBlock, 0, s>>>(ki, ka, ko, vi, (V*)va, vo, tab, medium_list, ctl);
+    auto lng = seg_long_kernel<KT, V, MC::kBlock, MC::kIpt>;
+    lng<<<std::min<uint32_t>((uint32_t)(max_total / (C::kCap + 1) + 1), seg_resident(lng, MC::kBlock)), MC::kBlock, 0, s>>>(
+        ka, ko, va, vo, tab, longs, ctl);
   }
-  switch (var) {
-    case 1:
-      seg_large<KT, VT, 1>(ki, ka, ko, vi, (V*)va, vo, tab, large_list, tile_start, seg_hist, seg_base, tcount, desc, ctl, L, s);
-      break;
-    case 2:
-      seg_large<KT, VT, 2>(ki, ka, ko, vi, (V*)va, vo, tab, large_list, tile_start, seg_hist, seg_base, tcount, desc, ctl, L, s);
-      break;
-    default:
-      seg_large<KT, VT, 0>(ki, ka, ko, vi, (V*)va, vo, tab, large_list, tile_start, seg_hist, seg_base, tcount, desc, ctl, L, s);
-  }
+  auto local = seg_local_kernel<KT, V, C::kLocalBlock, C::kLocalIpt, C::kLocalWaves>;
+  local<<<std::min(L.batches_ub, seg_resident(local, C::kLocalBlock)), C::kLocalBlock, 0, s>>>(ki, ka, ko, vi, va, vo, tab,
+                                                                                           batches, ctl);
   return check_launch();
 }
 
@@ -744,9 +1111,9 @@ int seg_by_val(mgs_val vt, const void* kin, void* kout, const void* vin, void* v
 }
 
 template <int KB, int VB>
-size_t seg_bytes(size_t max_total, size_t nseg, size_t max_seg, int var) {
+size_t seg_bytes(size_t max_total, size_t nseg, size_t max_seg, int var, bool wide_range = false) {
   if (var < 0 || var >= kSegVariants) var = 0;
-  return seg_layout<KB, VB>(max_total, nseg, max_seg, seg_large_tile<KB, VB>(var)).total;
+  return seg_layout<KB, VB>(max_total, nseg, max_seg, seg_large_tile<KB, VB>(var), wide_range).total;
 }
 
 template <int KB, int VB>
@@ -778,9 +1145,9 @@ size_t segmented_temp_bytes(mgs_key kt, mgs_val vt, size_t max_total, size_t nse
     if (vb == 4) return seg_bytes<4, 4>(max_total, nseg, ms, var);
     return seg_bytes<4, 8>(max_total, nseg, ms, var);
   }
-  if (vb == 0) return seg_bytes<8, 0>(max_total, nseg, ms, var);
-  if (vb == 4) return seg_bytes<8, 4>(max_total, nseg, ms, var);
-  return seg_bytes<8, 8>(max_total, nseg, ms, var);
+  if (vb == 0) return seg_bytes<8, 0>(max_total, nseg, ms, var, kt == MGS_KEY_F64);
+  if (vb == 4) return seg_bytes<8, 4>(max_total, nseg, ms, var, kt == MGS_KEY_F64);
+  return seg_bytes<8, 8>(max_total, nseg, ms, var, kt == MGS_KEY_F64);
 }
 
 int segmented_variant(mgs_key kt, mgs_val vt, int var, int32_t* block, int32_t* ipt) {
@@ -798,6 +1165,13 @@ int segmented_variant(mgs_key kt, mgs_val vt, int var, int32_t* block, int32_t* 
 }
 
 int segmented_variant_count() { return kSegVariants; }
+
+size_t split_sort_temp_bytes(mgs_key kt, mgs_val vt, size_t n) { return segmented_temp_bytes(kt, vt, n, 1, nullptr); }
+
+int split_sort(mgs_key kt, mgs_val vt, const void* kin, void* kout, const void* vin, void* vout, size_t n, void* temp,
+               size_t temp_bytes, hipStream_t s) {
+  return segmented_dispatch(kt, vt, kin, kout, vin, vout, nullptr, false, nullptr, 1, n, nullptr, temp, temp_bytes, s);
+}
 
 int segmented_dispatch(mgs_key kt, mgs_val vt, const void* kin, void* kout, const void* vin, void* vout,
                        const uint64_t* d_offsets, bool ranges, const uint64_t* d_val_begin, size_t nseg, size_t max_total, const mgs_tuning* tuning,

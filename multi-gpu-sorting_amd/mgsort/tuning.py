@@ -2,10 +2,11 @@
 batching layer is this library's).
 
 The search space per (key type, payload type, size bin):
-  large_variant  the tile geometry of the large segments' passes
+  large_variant  the tile geometry of the long segments' scatter
                  (mgs_segmented_variant: threads x items per thread)
-  medium_max     longest segment one workgroup streams alone
-  small_max      longest segment sorted inside one workgroup's LDS
+  small_max, medium_max  the longest segment sorted inside one workgroup's LDS
+                 is the larger of them; the default, as many records as fit,
+                 is the only point searched
 Every point is timed on a synthetic batch of that size (segment lengths
 log-uniform in [2^8, 2^22], uniform keys, u32 payload = index inside the
 segment).  The winners are written to a JSON table, which the library loads
@@ -30,8 +31,8 @@ from . import (KEY_NAMES, VAL_NAMES, Tuning, key_type, lib, segmented_sort, temp
 TABLE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "seg_tuning.json")
 KEY_STR = {v: k for k, v in KEY_NAMES.items()}
 VAL_STR = {0: "none", 1: "u32", 2: "u64"}
-MEDIUM_MAX = (0, 1 << 15, 1 << 16, 1 << 18)  # 0 = the library default (2^17)
-SMALL_MAX = (0, 1024)                          # 0 = the library default (one LDS tile)
+MEDIUM_MAX = (0,)  # 0 = the library default
+SMALL_MAX = (0,)
 
 _table: Optional[dict] = None
 
@@ -41,7 +42,7 @@ def variant_count() -> int:
 
 
 def geometry(kt, vt, variant: int) -> Tuple[int, int]:
-    """(threads per workgroup, items per thread) of a large-segment variant."""
+    """(threads per workgroup, items per thread) of a scatter variant."""
     b, i = ctypes.c_int32(0), ctypes.c_int32(0)
     st = lib.mgs_segmented_variant(key_type(kt), val_type(vt), int(variant), ctypes.byref(b), ctypes.byref(i))
     if st != 0:

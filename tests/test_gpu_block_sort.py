@@ -146,3 +146,48 @@ def test_three_pass_wide_small_scratch(mg):
     assert mg.temp_status(temp) == 0
     assert mg.lib.mgs_sort_path(O.K_U64, mg.VAL_NONE, n, mg._ptr(temp), temp.numel(), None) == 2
     assert np.array_equal(from_dev(dk, np.uint64), np.sort(keys))
+
+
+def scaled_keys(kt, n, rng, dist):
+    """heavy: one value in 60% of the places; nested: a third each uniform
+    over the whole range, over its 2^-20th and its 2^-40th (4-byte keys: 2^-10th,
+    2^-20th), which outlasts two levels of splits; edge: the range's ends and
+    254 to 256 consecutive values."""
+    bd = O.BITS_DTYPE[kt]
+    nbits = 32 if bd == np.uint32 else 64
+    k = random_keys(kt, n, rng).view(bd) if dist != "edge" else None
+    if dist == "heavy":
+        k[rng.random(n) < 0.6] = k[0]
+    elif dist == "nested":
+        if kt in (O.K_F32, O.K_F64):
+            k = random_keys(kt, n, rng, "nonneg").view(bd)
+        k = k >> (rng.integers(0, 3, size=n) * (nbits // 3 - 1)).astype(bd)
+    elif dist == "edge":
+        k = (bd(1) << bd(nbits - 3)) + rng.integers(0, 254 + n % 3, size=n).astype(bd)
+        k[n // 2], k[n // 3] = 0, bd(1) << bd(nbits - 2)
+    return k
+
+
+@pytest.mark.parametrize("kt,vdt", [(O.K_U32, None), (O.K_F32, np.uint32), (O.K_I64, None), (O.K_U64, np.uint32),
+                                    (O.K_F64, np.uint64)], ids=lambda v: str(v))
+@pytest.mark.parametrize("dist", ["uniform", "heavy", "nested", "edge", "sorted"])
+def test_splits(mg, kt, vdt, dist):
+    """Segments at the edges of what one workgroup sorts (512 x 7, 10, 14, 16
+    records), of the scatter's tiles, and long enough for two and three
+    levels of splits."""
+    import torch
+    rng = np.random.default_rng(kt + 17)
+    lens = [0, 1, 256, 257] + [512 * i + d for i in (7, 10, 14, 16, 20, 32) for d in (-1, 0, 1)]
+    lens += [70_001, 300_002] + ([1_100_003] if dist in ("uniform", "nested") else [])
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    make = scaled_keys if dist in ("heavy", "nested", "edge") else random_keys
+    parts = [make(kt, n, rng, dist).view(O.BITS_DTYPE[kt]) if n else np.zeros(0, O.BITS_DTYPE[kt]) for n in lens]
+    keys = np.concatenate(parts).view(random_keys(kt, 1, rng).dtype)
+    vals = None if vdt is None else random_vals(vdt, keys.size, rng)
+    ek, ev = O.segmented_sort(kt, keys, off, vals)
+    dk, dv = to_dev(keys), to_dev(vals)
+    mg.segmented_sort(KEY_NAME[kt], dk, torch.from_numpy(off.view(np.int64)).cuda(), dv)
+    torch.cuda.synchronize()
+    assert np.array_equal(from_dev(dk, O.BITS_DTYPE[kt]), ek.view(O.BITS_DTYPE[kt]))
+    if vdt is not None:
+        assert np.array_equal(from_dev(dv, vdt), ev)
