@@ -142,15 +142,17 @@ int mgs_sort_timed(mgs_key kt, mgs_val vt,
 
 /* Which algorithm the last mgs_sort / mgs_sort_timed call with these
  * arguments and this temp buffer used (no reference counterpart): waits for
- * `stream` and returns MGS_PATH_SMALL (one workgroup in LDS, no scratch),
- * MGS_PATH_LSD (onesweep LSD passes) or MGS_PATH_THREE_PASS (the MSD pass,
- * the bucket pass and the LDS sort of sub-buckets, tried for 4-byte keys
- * alone of 2^23 to 3 * 2^24 keys and of 2^29 keys and more, for 8-byte
- * integer keys from 2^22 and 4-byte integer keys with payloads from 2^24
- * records up to about 2^28; it hands over to the LSD passes when the key
- * distribution does not suit it, and wider records take the LSD passes when
- * temp only fits these), or a negative status. */
-enum { MGS_PATH_SMALL = 1, MGS_PATH_LSD = 2, MGS_PATH_THREE_PASS = 3 };
+ * `stream` and returns MGS_PATH_SMALL (one workgroup in LDS), MGS_PATH_SPLIT
+ * (the segmented sort's splits, for one array; below 2^23 records, 4-byte
+ * integers alone below 2^22), MGS_PATH_LSD (onesweep LSD passes) or
+ * MGS_PATH_THREE_PASS (the MSD pass, the bucket pass and the LDS sort of
+ * sub-buckets, tried for 4-byte keys alone of 2^23 to 3 * 2^24 keys and of
+ * 2^29 keys and more, for 8-byte integer keys from 2^23 and 4-byte integer
+ * keys with payloads from 2^24 records up to about 2^28; it hands over to the
+ * LSD passes when the key distribution does not suit it), or a negative
+ * status.  Where temp only fits the LSD passes, the splits and the three
+ * passes of wider records are not taken. */
+enum { MGS_PATH_SMALL = 1, MGS_PATH_LSD = 2, MGS_PATH_THREE_PASS = 3, MGS_PATH_SPLIT = 4 };
 int mgs_sort_path(mgs_key kt, mgs_val vt, size_t n, const void* temp, size_t temp_bytes, void* stream);
 
 /* Comma-separated names of the stages of this thread's last mgs_sort_timed

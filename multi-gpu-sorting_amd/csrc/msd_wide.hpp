@@ -49,11 +49,11 @@ template <int KT>
 constexpr bool kFloatKey = KT == MGS_KEY_F32 || KT == MGS_KEY_F64;
 
 // Sizes the path is tried for: up to where the sub-buckets of uniform keys
-// (n / 65536, Poisson) still fit a workgroup, and from where it gains enough
-// on uniform keys to risk its six launches (25-30 us) on keys that leave it:
-// 8-byte keys 2^22 293 -> 166 us; u32 + u32 2^22 168 -> 157 us, 2^24 366 ->
-// 317 us.
-inline size_t wide_min(int kb) { return size_t(1) << (kb == 8 ? 22 : 24); }
+// (n / 65536, Poisson) still fit a workgroup, and from where it beats the
+// splits (segmented.hip) for 8-byte keys: u64 2^22 164 us against 155 us, 2^23
+// 198 against 251, 2^24 327 against 430; and the LSD passes for 4-byte keys
+// with payloads: u32 + u32 2^24 366 -> 311 us.
+inline size_t wide_min(int kb) { return size_t(1) << (kb == 8 ? 23 : 24); }
 size_t wide_max(int rec);
 bool wide_eligible(int kb, int vb, size_t n);
 

@@ -6,6 +6,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "block_sort.hpp"
 #include "internal.hpp"
 #include "msd_sort.hpp"
 #include "msd_wide.hpp"
@@ -732,13 +733,38 @@ __global__ void fixup_kernel(const Bits* k_in, const Bits* k_alt, Bits* k_out, c
 }
 
 // ---------------------------------------------------------------------------
-// Single-workgroup sort of up to one tile, entirely in LDS.
+// Single-workgroup sort of up to one tile, entirely in LDS (block_sort.hpp).
+// Bound by latency: the load, the reductions and barriers of three passes and
+// the store, one after another.  2000 u32 keys: 10.6 us by four byte passes of
+// 256 threads, 6.9 so; 8192: 44 us by the passes over HBM, 13.7 so.  status: a status word to clear, or NULL.
 // ---------------------------------------------------------------------------
 template <int KT, typename V, int BLOCK, int IPT>
 __global__ __launch_bounds__(BLOCK) void small_sort_kernel(const typename Codec<KT>::Bits* k_in,
                                                            typename Codec<KT>::Bits* k_out, const V* v_in, V* v_out,
-                                                           uint32_t n) {
-  small_sort_block<KT, V, BLOCK, IPT>(k_in, k_out, v_in, v_out, n);
+                                                           uint32_t n, uint32_t* status) {
+  using Bits = typename Codec<KT>::Bits;
+  using Smem = BlockSortSmem<Bits, V, BLOCK, IPT>;
+  __shared__ Smem sm;
+  if (status != nullptr && threadIdx.x == 0) *status = 0;
+  block_clear_row<BLOCK>(sm.off);
+  const uint32_t nit = block_items<BLOCK>(n), wb = block_first<BLOCK>(nit);
+  Bits k[IPT];
+  typename Smem::VS v[IPT];
+  static_for<IPT>([&](auto i) {
+    k[i] = 0;
+    if ((uint32_t)i < nit && wb + i * kWave < n) k[i] = k_in[wb + i * kWave];
+  });
+  if constexpr (kHasVal<V>) {
+    static_for<IPT>([&](auto i) {
+      v[i] = 0;
+      if ((uint32_t)i < nit && wb + i * kWave < n) v[i] = v_in[wb + i * kWave];
+    });
+  }
+  Bits mn, mx;
+  block_min_max<KT, V, BLOCK, IPT>(sm, k, wb, n, nit, mn, mx);
+  const Bits pad = block_pad<KT>(mx);
+  static_for<IPT>([&](auto i) { k[i] = wb + i * kWave < n ? k[i] : pad; });
+  block_sort<KT, V, BLOCK, IPT>(sm, k, v, n, mn, mx, k_out, v_out);
 }
 
 // ---------------------------------------------------------------------------
@@ -803,6 +829,18 @@ size_t desc_budget() {
   return size_t(96) << 20;
 }
 
+// Sorts below the three-pass paths' sizes that take one workgroup or the
+// segmented sort's splits instead of the LSD passes.  The switches that force
+// a path or a variant of the passes turn it off.
+bool mid_path(int rec, bool floats, size_t n) {
+  static const char* const kForcing[] = {"MGS_MSD", "MGS_MSD_MIN", "MGS_RANK_PEERS", "MGS_SKEW_PAIR_MIN",
+                                         "MGS_XCD_LOCAL", "MGS_DESC_BUDGET", "MGS_LB_SPIN_LIMIT"};
+  if (n >= mid_max(rec, floats)) return false;
+  for (const char* name : kForcing)
+    if (std::getenv(name) != nullptr) return false;
+  return true;
+}
+
 struct SortLayout {
   size_t status, alt_k, alt_v, hist, red, counters, carry, msd_ctl, desc, total;
   uint32_t num_tiles;
@@ -862,8 +900,8 @@ SortLayout sort_layout(size_t n) {
 // Wide records switch to larger tiles (fewer descriptors) at kBigTileMin
 // keys, so just above it the small-tile layout of kBigTileMin - 1 keys can
 // be the larger one; a buffer sized for n must serve every smaller sort.
-// wide: with room for the three-pass path of wider records, which such a sort
-// takes only if it finds the room.
+// wide: with room for the three-pass path of wider records and for the
+// splits, which such a sort takes only if it finds the room.
 template <int KB, int VB>
 size_t sort_bytes(size_t n, bool wide) {
   const SortLayout L = sort_layout<KB, VB>(n);
@@ -873,6 +911,11 @@ size_t sort_bytes(size_t n, bool wide) {
   // decrease with n
   if (KB == 4 && VB == 0 && (msd_eligible(n) || n >= MsdCfg::kMinKeys))
     b = std::max(b, msd_layout(std::min(n, MsdCfg::kMaxKeys), L.desc, L.msd_ctl).end);
+  if (wide) {
+    const mgs_key kt = KB == 4 ? MGS_KEY_U32 : MGS_KEY_F64;  // (the most of its width)
+    const mgs_val vt = VB == 0 ? MGS_VAL_NONE : VB == 4 ? MGS_VAL_U32 : MGS_VAL_U64;
+    b = std::max(b, split_sort_temp_bytes(kt, vt, std::min(n, kMidMax)));
+  }
   if (KB + VB > 4 && wide && (wide_eligible(KB, VB, n) || n >= wide_min(KB)))
     b = std::max(b, wide_layout(KB + VB, std::min(n, wide_max(KB + VB)), L.desc, L.msd_ctl).end);
   if (KB + VB > 4 && n >= kBigTileMin) b = std::max(b, sort_layout_cfg<KB, VB, false>(kBigTileMin - 1).total);
@@ -922,7 +965,7 @@ int sort_typed_cfg(const void* kin, void* kout, const void* vin, void* vout, siz
 
   if (n <= (size_t)SCfg::kTile) {
     mark(s, "small_sort");
-    small_sort_kernel<KT, V, SCfg::kBlock, SCfg::kIpt><<<1, SCfg::kBlock, 0, s>>>(ki, ko, vi, vo, (uint32_t)n);
+    small_sort_kernel<KT, V, SCfg::kBlock, SCfg::kIpt><<<1, SCfg::kBlock, 0, s>>>(ki, ko, vi, vo, (uint32_t)n, nullptr);
     mark(s);
     return check_launch();
   }
@@ -934,6 +977,23 @@ int sort_typed_cfg(const void* kin, void* kout, const void* vin, void* vout, siz
   const MsdLayout ML = msd_layout(n, L.desc, L.msd_ctl);
   const size_t need = msd ? std::max(L.total, ML.end) : L.total;
   if (temp == nullptr || temp_bytes < need) return MGS_ERR_TEMP_TOO_SMALL;
+  // (a call with less scratch than the LSD passes need is refused, whatever
+  // path it would take)
+  if (mid_path(KB + VB, kFloatKey<KT>, n)) {
+    if (n <= (size_t)SCfg::kMaxTile) {
+      mark(s, "small_sort");
+      small_sort_kernel<KT, V, SCfg::kMaxBlock, SCfg::kMaxIpt>
+          <<<1, SCfg::kMaxBlock, 0, s>>>(ki, ko, vi, vo, (uint32_t)n, static_cast<uint32_t*>(temp));
+      mark(s);
+      return check_launch();
+    }
+    if (temp_bytes >= split_sort_temp_bytes((mgs_key)KT, (mgs_val)VT, n)) {
+      mark(s, "split_sort");
+      const int rc = split_sort((mgs_key)KT, (mgs_val)VT, kin, kout, vin, vout, n, temp, temp_bytes, s);
+      mark(s);
+      return rc;
+    }
+  }
   char* t = static_cast<char*>(temp);
   uint32_t* status = reinterpret_cast<uint32_t*>(t + L.status);
   Bits* ka = reinterpret_cast<Bits*>(t + L.alt_k);
@@ -1108,6 +1168,12 @@ template <int KB, int VB>
 int path_of(bool floats, size_t n, const void* temp, size_t temp_bytes, hipStream_t s) {
   using SCfg = SmallCfg<KB, VB>;
   if (n <= (size_t)SCfg::kTile) return MGS_PATH_SMALL;
+  if (mid_path(KB + VB, floats, n)) {
+    if (n <= (size_t)SCfg::kMaxTile) return MGS_PATH_SMALL;
+    const mgs_key kt = KB == 4 ? MGS_KEY_U32 : floats ? MGS_KEY_F64 : MGS_KEY_U64;
+    const mgs_val vt = VB == 0 ? MGS_VAL_NONE : VB == 4 ? MGS_VAL_U32 : MGS_VAL_U64;
+    if (temp_bytes >= split_sort_temp_bytes(kt, vt, n)) return MGS_PATH_SPLIT;
+  }
   constexpr bool kAlone4 = KB == 4 && VB == 0;
   if (!(kAlone4 ? msd_eligible(n) : !floats && wide_eligible(KB, VB, n))) return MGS_PATH_LSD;
   const SortLayout L = sort_layout<KB, VB>(n);

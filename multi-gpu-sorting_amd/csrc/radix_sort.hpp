@@ -151,12 +151,26 @@ using PassCfg = typename std::conditional<BIG || (KB + VB) <= 4, TileCfg<KB, VB>
                                           TileCfg<KB, VB, MGS_OS_IPT, 8, 8, 4, MGS_PASS_WAVES_4B>>::type;
 inline bool use_big_tiles(int kb, int vb, size_t n) { return kb + vb <= 4 || n >= kBigTileMin; }
 
-// Single-workgroup LDS sort geometry.
+// Single-workgroup LDS sort geometry: kTile records without scratch, kMaxTile
+// (as many as leave no item array in scratch registers) with a status word to
+// clear.
 template <int KB, int VB> struct SmallCfg {
-  static constexpr int kBlock = 256;
-  static constexpr int kIpt = (KB + VB) <= 8 ? 16 : 8;
+  static constexpr int kBlock = 512;
+  static constexpr int kIpt = (KB + VB) <= 8 ? 8 : 4;
   static constexpr int kTile = kBlock * kIpt;
+  static constexpr int kMaxBlock = 1024;
+  static constexpr int kMaxIpt = (KB + VB) <= 4 ? 24 : (KB + VB) <= 8 ? 15 : (KB + VB) <= 12 ? 10 : 7;
+  static constexpr int kMaxTile = kMaxBlock * kMaxIpt;
 };
+
+// Arrays below this length sort by one workgroup or by splits (mid_path).
+// LSD passes against splits: u64 2^14 85 us against 47, 2^20 166 against 83,
+// 2^22 290 against 159; f64 + u32 just below 2^23 529 against 308; f32 there
+// 231 against 193; u32 + u32 246 against 228.  u32 alone, whose four passes
+// move the least: 2^20 104 against 79, 2^22 145 against 136, but 194 against
+// 204 just below 2^23.
+inline constexpr size_t kMidMax = size_t(1) << 23;
+inline size_t mid_max(int rec, bool floats) { return rec <= 4 && !floats ? kMidMax / 2 : kMidMax; }
 
 // ---------------------------------------------------------------------------
 // Stable per-wavefront ranking of one item per lane.

@@ -26,7 +26,7 @@ KEY_BYTES = {KEY_U32: 4, KEY_I32: 4, KEY_F32: 4, KEY_U64: 8, KEY_I64: 8, KEY_F64
 VAL_BYTES = {VAL_NONE: 0, VAL_U32: 4, VAL_U64: 8}
 
 MGS_OK = 0
-PATH_SMALL, PATH_LSD, PATH_THREE_PASS = 1, 2, 3
+PATH_SMALL, PATH_LSD, PATH_THREE_PASS, PATH_SPLIT = 1, 2, 3, 4
 
 SYMBOLS = [
     "mgs_sort_temp_bytes", "mgs_sort", "mgs_sort_noalloc", "mgs_sort_timed", "mgs_sort_timed_stages", "mgs_sort_path", "mgs_merge_temp_bytes", "mgs_merge", "mgs_select_pivot",

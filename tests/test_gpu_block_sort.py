@@ -81,7 +81,7 @@ def test_one_or_two_runs(mg, lens, portions):
 RECORDS = [(O.K_U64, None), (O.K_I64, np.uint32), (O.K_U64, np.uint64), (O.K_U32, np.uint32), (O.K_I32, np.uint64)]
 
 
-def run_three_pass(mg, kt, vdt, keys, rng, inplace):
+def run_sort(mg, kt, vdt, keys, rng, inplace):
     """Sorts on the device, checks status and oracle, returns the path."""
     import torch
     n = keys.size
@@ -115,7 +115,7 @@ def test_three_pass_wide_forced(mg, kt, vdt, n, dist, monkeypatch):
     monkeypatch.setenv("MGS_MSD_MIN", "0")
     rng = np.random.default_rng(n + 5 * kt)
     keys = tied_keys(kt, n, rng, dist) if dist in ("clustered", "pairs") else random_keys(kt, n, rng, dist)
-    path = run_three_pass(mg, kt, vdt, keys, rng, inplace=bool(n & 1))
+    path = run_sort(mg, kt, vdt, keys, rng, inplace=bool(n & 1))
     assert path in (2, 3)
     if dist in ("uniform", "nonneg"):
         assert path == 3
@@ -124,11 +124,11 @@ def test_three_pass_wide_forced(mg, kt, vdt, n, dist, monkeypatch):
 @pytest.mark.parametrize("kt,vdt", RECORDS, ids=lambda v: str(v))
 @pytest.mark.parametrize("dist", ["uniform", "sorted", "skewed", "nonneg"])
 def test_three_pass_wide_default(mg, kt, vdt, dist):
-    """Without environment: 8-byte keys from 2^22 records on, 4-byte keys
+    """Without environment: 8-byte keys from 2^23 records on, 4-byte keys
     with payloads from 2^24."""
     rng = np.random.default_rng(3 + kt)
-    keys = random_keys(kt, (1 << (22 if O.BITS_DTYPE[kt] == np.uint64 else 24)) + 4321, rng, dist)
-    path = run_three_pass(mg, kt, vdt, keys, rng, inplace=False)
+    keys = random_keys(kt, (1 << (23 if O.BITS_DTYPE[kt] == np.uint64 else 24)) + 4321, rng, dist)
+    path = run_sort(mg, kt, vdt, keys, rng, inplace=False)
     assert path in (2, 3)
     if dist == "uniform":
         assert path == 3
@@ -137,7 +137,7 @@ def test_three_pass_wide_default(mg, kt, vdt, dist):
 def test_three_pass_wide_small_scratch(mg):
     """Scratch that only fits the LSD passes still sorts."""
     rng = np.random.default_rng(8)
-    n = (1 << 22) + 9
+    n = (1 << 23) + 9
     keys = random_keys(O.K_U64, n, rng)
     temp = mg.temp_buffer(n * 8 + (4 << 20), "cuda")
     assert temp.numel() < mg.lib.mgs_sort_temp_bytes(O.K_U64, mg.VAL_NONE, n)
@@ -191,3 +191,25 @@ def test_splits(mg, kt, vdt, dist):
     assert np.array_equal(from_dev(dk, O.BITS_DTYPE[kt]), ek.view(O.BITS_DTYPE[kt]))
     if vdt is not None:
         assert np.array_equal(from_dev(dv, vdt), ev)
+
+
+@pytest.mark.parametrize("kt,vdt,most", [(O.K_U32, None, 24576), (O.K_F32, np.uint32, 15360), (O.K_I64, None, 15360),
+                                         (O.K_U64, np.uint32, 10240), (O.K_F64, np.uint64, 7168)], ids=lambda v: str(v))
+@pytest.mark.parametrize("dist", ["uniform", "heavy", "nested"])
+def test_middle_sizes(mg, kt, vdt, most, dist):
+    """One array around the longest that one workgroup sorts, and by splits."""
+    rng = np.random.default_rng(kt + most)
+    for n in (2047, 2049, 4095, 4097, most - 1, most, most + 1, 200_003):
+        keys = scaled_keys(kt, n, rng, dist).view(random_keys(kt, 1, rng).dtype)
+        assert run_sort(mg, kt, vdt, keys, rng, inplace=bool(n & 1)) == (1 if n <= most else 4)
+
+
+@pytest.mark.parametrize("kt,vdt,end", [(O.K_F32, None, 23), (O.K_U32, None, 22), (O.K_U32, np.uint32, 23),
+                                        (O.K_F64, None, 23), (O.K_I64, np.uint32, 23)], ids=lambda v: str(v))
+def test_splits_end(mg, kt, vdt, end):
+    """Splits below 2^23 records (4-byte integers alone: 2^22), the passes
+    from there on."""
+    rng = np.random.default_rng(kt)
+    for n in (1 << end) - 1, 1 << end:
+        path = run_sort(mg, kt, vdt, random_keys(kt, n, rng), rng, inplace=False)
+        assert (path == 4) == (n < 1 << end)
