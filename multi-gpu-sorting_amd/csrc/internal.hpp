@@ -89,6 +89,7 @@ int fill_max_dispatch(mgs_key kt, void* keys, size_t n, hipStream_t s);
 
 // mgs_sort by the segmented sort's splits and local sort (segmented.hip): one
 // array of n records.
+uint32_t split_local_cap(int kb, int vb);  // records that its local sort takes at once
 size_t split_sort_temp_bytes(mgs_key kt, mgs_val vt, size_t n);
 int split_sort(mgs_key kt, mgs_val vt, const void* kin, void* kout, const void* vin, void* vout, size_t n, void* temp,
                size_t temp_bytes, hipStream_t s);

@@ -829,13 +829,13 @@ size_t desc_budget() {
   return size_t(96) << 20;
 }
 
-// Sorts below the three-pass paths' sizes that take one workgroup or the
-// segmented sort's splits instead of the LSD passes.  The switches that force
-// a path or a variant of the passes turn it off.
-bool mid_path(int rec, bool floats, size_t n) {
+// Sorts below mid_max records take one workgroup or the segmented sort's
+// splits instead of the LSD passes.  The switches that force a path or a
+// variant of the passes turn it off.
+bool mid_path(int kb, int vb, bool floats, size_t n) {
   static const char* const kForcing[] = {"MGS_MSD", "MGS_MSD_MIN", "MGS_RANK_PEERS", "MGS_SKEW_PAIR_MIN",
                                          "MGS_XCD_LOCAL", "MGS_DESC_BUDGET", "MGS_LB_SPIN_LIMIT"};
-  if (n >= mid_max(rec, floats)) return false;
+  if (n >= mid_max(kb, vb, floats)) return false;
   for (const char* name : kForcing)
     if (std::getenv(name) != nullptr) return false;
   return true;
@@ -914,7 +914,7 @@ size_t sort_bytes(size_t n, bool wide) {
   if (wide) {
     const mgs_key kt = KB == 4 ? MGS_KEY_U32 : MGS_KEY_F64;  // (the most of its width)
     const mgs_val vt = VB == 0 ? MGS_VAL_NONE : VB == 4 ? MGS_VAL_U32 : MGS_VAL_U64;
-    b = std::max(b, split_sort_temp_bytes(kt, vt, std::min(n, kMidMax)));
+    b = std::max(b, split_sort_temp_bytes(kt, vt, std::min(n, mid_max(KB, VB, true))));
   }
   if (KB + VB > 4 && wide && (wide_eligible(KB, VB, n) || n >= wide_min(KB)))
     b = std::max(b, wide_layout(KB + VB, std::min(n, wide_max(KB + VB)), L.desc, L.msd_ctl).end);
@@ -979,7 +979,7 @@ int sort_typed_cfg(const void* kin, void* kout, const void* vin, void* vout, siz
   if (temp == nullptr || temp_bytes < need) return MGS_ERR_TEMP_TOO_SMALL;
   // (a call with less scratch than the LSD passes need is refused, whatever
   // path it would take)
-  if (mid_path(KB + VB, kFloatKey<KT>, n)) {
+  if (mid_path(KB, VB, kFloatKey<KT>, n)) {
     if (n <= (size_t)SCfg::kMaxTile) {
       mark(s, "small_sort");
       small_sort_kernel<KT, V, SCfg::kMaxBlock, SCfg::kMaxIpt>
@@ -1168,7 +1168,7 @@ template <int KB, int VB>
 int path_of(bool floats, size_t n, const void* temp, size_t temp_bytes, hipStream_t s) {
   using SCfg = SmallCfg<KB, VB>;
   if (n <= (size_t)SCfg::kTile) return MGS_PATH_SMALL;
-  if (mid_path(KB + VB, floats, n)) {
+  if (mid_path(KB, VB, floats, n)) {
     if (n <= (size_t)SCfg::kMaxTile) return MGS_PATH_SMALL;
     const mgs_key kt = KB == 4 ? MGS_KEY_U32 : floats ? MGS_KEY_F64 : MGS_KEY_U64;
     const mgs_val vt = VB == 0 ? MGS_VAL_NONE : VB == 4 ? MGS_VAL_U32 : MGS_VAL_U64;

@@ -205,11 +205,39 @@ def test_middle_sizes(mg, kt, vdt, most, dist):
 
 
 @pytest.mark.parametrize("kt,vdt,end", [(O.K_F32, None, 23), (O.K_U32, None, 22), (O.K_U32, np.uint32, 23),
-                                        (O.K_F64, None, 23), (O.K_I64, np.uint32, 23)], ids=lambda v: str(v))
+                                        (O.K_I64, np.uint32, 23)], ids=lambda v: str(v))
 def test_splits_end(mg, kt, vdt, end):
-    """Splits below 2^23 records (4-byte integers alone: 2^22), the passes
-    from there on."""
+    """Splits below 2^23 records (4-byte integers alone: 2^22; not doubles),
+    the passes from there on."""
     rng = np.random.default_rng(kt)
     for n in (1 << end) - 1, 1 << end:
         path = run_sort(mg, kt, vdt, random_keys(kt, n, rng), rng, inplace=False)
         assert (path == 4) == (n < 1 << end)
+
+
+@pytest.mark.parametrize("kt,vdt", [(O.K_U32, None), (O.K_F64, np.uint32)], ids=lambda v: str(v))
+@pytest.mark.parametrize("dist", ["uniform", "heavy", "nested"])
+def test_splits_chunks(mg, kt, vdt, dist):
+    """Segments of more than 1024 tiles (of 4096 and 6144 records), whose
+    tiles are counted in chunks of 64, beside short ones."""
+    import torch
+    rng = np.random.default_rng(kt + 23)
+    long = 4096 * 1100 if kt == O.K_U32 else 6144 * 1100
+    lens = [9, long + 1, 70_001, long // 3, 20_000, 20_000, long - 64 * 4096 - 1]
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    keys = np.concatenate([scaled_keys(kt, n, rng, dist) for n in lens]).view(random_keys(kt, 1, rng).dtype)
+    vals = None if vdt is None else random_vals(vdt, keys.size, rng)
+    ek, ev = O.segmented_sort(kt, keys, off, vals)
+    dk, dv = to_dev(keys), to_dev(vals)
+    mg.segmented_sort(KEY_NAME[kt], dk, torch.from_numpy(off.view(np.int64)).cuda(), dv, tuning=mg.Tuning(2, 0, 0, 0))
+    torch.cuda.synchronize()
+    assert np.array_equal(from_dev(dk, O.BITS_DTYPE[kt]), ek.view(O.BITS_DTYPE[kt]))
+    if vdt is not None:
+        assert np.array_equal(from_dev(dv, vdt), ev)
+
+
+@pytest.mark.parametrize("dist", ["uniform", "sorted", "few"])
+def test_doubles_take_splits(mg, dist):
+    rng = np.random.default_rng(6)
+    keys = random_keys(O.K_F64, (1 << 24) + 77, rng, dist)
+    assert run_sort(mg, O.K_F64, None, keys, rng, inplace=True) == 4
