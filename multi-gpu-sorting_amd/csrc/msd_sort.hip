@@ -275,20 +275,9 @@ __global__ __launch_bounds__(256) void msd_scan_kernel(const uint32_t* __restric
     if (d == kRadix - 1) ctl->runs = before + runs > n / 16 ? 1u : 0u;
     __syncthreads();  // every thread has read the scan's partial sums
   }
-  // sub-bucket size: the chains' 16-bit counters of bin s
-  uint32_t cnt = 0;
-  {
-    const uint32_t word = s >> 1, sh = (s & 1u) << 4;
-    uint32_t c = 0;
-    for (; c + 4 <= chains; c += 4) {
-      const uint32_t a0 = slices[(size_t)c * (kMsdBins / 2) + word];
-      const uint32_t a1 = slices[(size_t)(c + 1) * (kMsdBins / 2) + word];
-      const uint32_t a2 = slices[(size_t)(c + 2) * (kMsdBins / 2) + word];
-      const uint32_t a3 = slices[(size_t)(c + 3) * (kMsdBins / 2) + word];
-      cnt += ((a0 >> sh) & 0xFFFFu) + ((a1 >> sh) & 0xFFFFu) + ((a2 >> sh) & 0xFFFFu) + ((a3 >> sh) & 0xFFFFu);
-    }
-    for (; c < chains; ++c) cnt += (slices[(size_t)c * (kMsdBins / 2) + word] >> sh) & 0xFFFFu;
-  }
+  __shared__ uint32_t s_cnt[kRadix];
+  sum_slices(slices, chains, b, s_cnt);
+  const uint32_t cnt = s_cnt[d];
   sub_cnt[s] = cnt;
   if (cnt > kLocalCap) atomicOr(&ctl->off, kMsdOffSubBucket);
   const uint32_t excl = block_excl_scan_256(cnt, sums, (int)d);

@@ -4,6 +4,7 @@
 #include <cmath>
 #include <cstdlib>
 
+#include "msd_pass.hpp"
 #include "msd_wide.hpp"
 #include "radix_device.hpp"
 
@@ -45,21 +46,9 @@ __global__ __launch_bounds__(256) void wide_scan_kernel(const uint32_t* __restri
     if (d == kRadix - 1) ctl->runs = before + runs > n / 16 ? 1u : 0u;
     __syncthreads();  // every thread has read the scan's partial sums
   }
-  // sub-bucket size: the ranges' 16-bit counters of window value s, eight
-  // loads in flight
-  uint32_t cnt = 0;
-  {
-    const uint32_t word = s >> 1, sh = (s & 1u) << 4;
-    uint32_t c = 0;
-    for (; c + 8 <= ranges; c += 8) {
-      uint32_t a[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) a[i] = slices[(size_t)(c + i) * (kMsdBins / 2) + word];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) cnt += (a[i] >> sh) & 0xFFFFu;
-    }
-    for (; c < ranges; ++c) cnt += (slices[(size_t)c * (kMsdBins / 2) + word] >> sh) & 0xFFFFu;
-  }
+  __shared__ uint32_t s_cnt[kRadix];
+  sum_slices(slices, ranges, b, s_cnt);
+  const uint32_t cnt = s_cnt[d];
   if (cnt > cap) atomicOr(&ctl->off, kMsdOffSubBucket);
   const uint32_t excl = block_excl_scan_256(cnt, sums, (int)d);
   sub_off[s] = excl;
