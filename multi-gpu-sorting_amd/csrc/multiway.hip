@@ -471,9 +471,8 @@ int mw_launch(const void* const* runs, const size_t* lens, size_t k, void* out, 
     return merge_two_runs((mgs_key)KT, runs[0], lens[0], k > 1 ? runs[1] : nullptr, k > 1 ? lens[1] : 0, out, temp,
                           temp_bytes, s, portions, portion_end, portion_done);
   if (ns > (uint64_t)MGS_MAX_KEYS) return MGS_ERR_TOO_LARGE;  // sample ids and the sample sort
-  const MwLayout L = mw_layout(KB, k, ns);
-  if (temp == nullptr || temp_bytes < L.total) return MGS_ERR_TEMP_TOO_SMALL;
-  if (ns == 0) {  // no keys: nothing to merge, the status word says ok
+  if (ns == 0) {  // no keys: nothing to merge and no tables, the status word says ok
+    if (temp == nullptr || temp_bytes < sizeof(uint32_t)) return MGS_ERR_TEMP_TOO_SMALL;
     hipError_t z = hipMemsetAsync(temp, 0, 4, s);
     for (size_t p = 0; z == hipSuccess && p < portions; ++p) {
       portion_end[p] = 0;
@@ -481,6 +480,8 @@ int mw_launch(const void* const* runs, const size_t* lens, size_t k, void* out, 
     }
     return record_hip(z);
   }
+  const MwLayout L = mw_layout(KB, k, ns);
+  if (temp == nullptr || temp_bytes < L.total) return MGS_ERR_TEMP_TOO_SMALL;
   char* t = static_cast<char*>(temp);
   // run table: host arrays copied into temp (pageable sources; the copy
   // has read them when hipMemcpyAsync returns)

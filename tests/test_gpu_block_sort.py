@@ -78,6 +78,18 @@ def test_one_or_two_runs(mg, lens, portions):
     assert np.array_equal(from_dev(out, np.uint32), expect)
 
 
+@pytest.mark.parametrize("kt", [O.K_U32, O.K_F64], ids=str)
+@pytest.mark.parametrize("k", [1, 2, 3, 9])
+def test_empty_runs(mg, kt, k):
+    """Runs that are all empty merge with the scratch that their size asks for."""
+    import torch
+    runs = [torch.empty(0, dtype=torch.int32 if kt == O.K_U32 else torch.int64, device="cuda") for _ in range(k)]
+    out = torch.empty(1, dtype=runs[0].dtype, device="cuda")
+    temp = mg.temp_buffer(mg.lib.mgs_multiway_merge_temp_bytes(kt, k, 0), "cuda")
+    assert mg.multiway_merge(KEY_NAME[kt], runs, out, temp=temp, portions=3) == [0, 0, 0]
+    assert mg.temp_status(temp) == 0
+
+
 RECORDS = [(O.K_U64, None), (O.K_I64, np.uint32), (O.K_U64, np.uint64), (O.K_U32, np.uint32), (O.K_I32, np.uint64)]
 
 
