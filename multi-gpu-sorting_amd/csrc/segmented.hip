@@ -13,8 +13,11 @@
 //     count     per tile of every node: the digit of each key and their
 //               counts.  A node's digits are its own: 254 equal steps of the
 //               encoded key between (about) the first and the last hundredth
-//               of 256 sampled keys, and one digit for what lies below and
-//               above -- monotone in the key whatever the sample missed
+//               of 255 sampled keys, and one digit for what lies below and
+//               above; or, where too many keys would share a step, the
+//               samples themselves as bounds, with a digit of its own for a
+//               value that several have -- monotone in the key whatever the
+//               sample missed
 //     chunk     where segments are very long: the offsets inside each 64 tiles
 //     scan      per node: the tiles' (or chunks') offsets, and what becomes of the
 //               children: consecutive ones that fit one workgroup together
@@ -27,8 +30,14 @@
 //
 // A level moves a record once and reads its key twice, so an 8-byte key with
 // a payload takes one to two levels and the local sort instead of eight LSD
-// passes, and no key distribution needs a fallback: skewed keys only take
-// more levels.  Against LSD passes over all long segments at once and one
+// passes.  Bounds from the sample divide keys of any distribution into children
+// of at most about a fortieth, so the levels bring them to what one workgroup
+// sorts in LDS up to chance: on 868 calls of 23 distributions one child in
+// thousands was left, a little above it.  (Inputs made against the sample's fixed
+// places may leave long ones: 6 to 9 ns a record of 8-byte keys each.)  With
+// equal steps alone, log-uniform u64 keys left 61% of 2^23 records to one
+// workgroup: 45.6 ms, now 0.30; 2^26 doubles 1 - eps 336 ms, now 1.9.
+// Against LSD passes over all long segments at once and one
 // workgroup for each middle one: u64 + u32, 1024 segments of 2^8 to 2^22, 26.3
 // -> 12.3 ms; u32, 256 ranges of 2^10 to 2^18, 331 -> 166 us; f64, normal, 64
 // of 2^10 to 2^22, 2518 -> 752 us.
@@ -58,11 +67,16 @@ struct SegCtl {
 // `base`, 255 above `top`, between them 1 + the step, which is the high word
 // of ((key - base) >> shift) mul (254 even steps), or key - base itself where
 // mul is 0 (every value a step).
+// shift kBySample: the sample's values are the bounds of the digits instead,
+// and the bits of `same` tell which digits hold one value only.
+// shift kDone (written by the scan): one key in all places, nothing to scatter.
 struct Node {
   uint32_t seg, off, len, tile0;
   uint64_t base, top;
   uint32_t mul, shift;
+  uint64_t same[kRadix / kWave];
 };
+enum : uint32_t { kBySample = 64, kDone = 65 };
 
 // Where a batch's records are.
 enum : uint32_t { kSrcIn = 0, kSrcAlt = 1, kSrcOut = 2 };
@@ -213,7 +227,7 @@ __global__ __launch_bounds__(kClassifyBlock) void seg_classify_kernel(const uint
     block_scan3(is_s, is_l, nt, es, el, et, ts, tl, tt, sm);
     block_scan3(bad, 0, 0, eb, e1, e2, tb, t1, t2, sm);
     if (is_s) batches[run_s + es] = make_uint4(s, 0, len, kSrcIn);
-    if (is_l) nodes[run_l + el] = Node{s, 0, len, run_t + et, 0, 0, 0, 0};
+    if (is_l) nodes[run_l + el] = Node{s, 0, len, run_t + et, 0, 0, 0, 0, {}};
     run_s += ts;
     run_l += tl;
     run_t += tt;
@@ -271,6 +285,13 @@ __device__ void medium_sort_block(const typename Codec<KT>::Bits* k_in, typename
     for (int p = 0; p < P; ++p) seg_hist_count(&hist[0][0], p * kRadix + digit_of<KT>(k, 8 * p));
   }
   __syncthreads();
+  if (k_in == k_out) {  // one key in all places: in order
+    const Bits k0 = k_in[0];
+    bool one = true;
+#pragma unroll
+    for (int p = 0; p < P; ++p) one &= hist[p][digit_of<KT>(k0, 8 * p)] == n;
+    if (one) return;
+  }
 
   for (int p = 0; p < P; ++p) {
     const int shift = 8 * p;
@@ -401,14 +422,147 @@ struct Steps {
   Bits base, top;
   uint32_t mul, shift;
 };
-template <int KT>
-__device__ __forceinline__ uint32_t step_digit(typename Codec<KT>::Bits raw, const Steps<typename Codec<KT>::Bits>& st) {
-  using Bits = typename Codec<KT>::Bits;
-  const Bits e = Codec<KT>::enc(raw);
+template <typename Bits>
+__device__ __forceinline__ uint32_t step_of(Bits e, const Steps<Bits>& st) {
   const uint32_t t = (uint32_t)((Bits)(e - st.base) >> st.shift);
   uint32_t d = (st.mul ? __umulhi(t, st.mul) : t) + 1u;
   d = e < st.base ? 0u : d;
   return e > st.top ? 255u : d;
+}
+template <int KT>
+__device__ __forceinline__ uint32_t step_digit(typename Codec<KT>::Bits raw, const Steps<typename Codec<KT>::Bits>& st) {
+  return step_of<typename Codec<KT>::Bits>(Codec<KT>::enc(raw), st);
+}
+
+// ---------------------------------------------------------------------------
+// The sample of a range: kSamples of its keys, one at a hashed place in each
+// of as many equal stretches (at even distances, keys that repeat with the
+// stride would all look alike).
+// Thread t of the first 256 gives the t-th key, encoded, and `sorted` holds
+// them in order on return; key and rank are working space.  Every thread of
+// the block calls it.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kSamples = 255;
+
+template <int KT, int BLOCK>
+__device__ __forceinline__ void sort_sample(const typename Codec<KT>::Bits* __restrict__ keys, uint32_t len,
+                                            typename Codec<KT>::Bits* key, uint32_t* rank,
+                                            typename Codec<KT>::Bits* sorted) {
+  using Bits = typename Codec<KT>::Bits;
+  const uint32_t t = threadIdx.x;
+  if (t < (uint32_t)kRadix) {
+    Bits x = ~Bits(0);  // thread 255: a place behind the sample
+    if (t < kSamples) {
+      const uint32_t a = (uint32_t)((uint64_t)len * t / kSamples), b = (uint32_t)((uint64_t)len * (t + 1) / kSamples);
+      uint32_t h = (t + 1) * 0x9E3779B9u ^ len;
+      h = (h ^ (h >> 16)) * 0x85EBCA6Bu;
+      h = (h ^ (h >> 13)) * 0xC2B2AE35u;
+      x = Codec<KT>::enc(keys[min(a + __umulhi(h ^ (h >> 16), b - a), len - 1)]);
+    }
+    key[t] = x;
+    rank[t] = 0;
+  }
+  __syncthreads();
+  {
+    // the rank of every key among a part of the others per thread (ties by place)
+    constexpr uint32_t kPart = kRadix * kRadix / BLOCK;
+    const uint32_t i = t & (kRadix - 1), from = t / kRadix * kPart;
+    const Bits x = key[i];
+    uint32_t r = 0;
+#pragma unroll 8
+    for (uint32_t j = from; j < from + kPart; ++j) r += (key[j] < x || (key[j] == x && j < i)) ? 1u : 0u;
+    atomicAdd(&rank[i], r);
+  }
+  __syncthreads();
+  if (t < (uint32_t)kRadix) sorted[rank[t]] = key[t];
+  __syncthreads();
+}
+
+// Turns the sorted sample into the bounds of the digits: digit d holds the keys
+// from bound d - 1 on and below bound d.  A value that the sample has more than
+// once is followed by the value one above it, and so has a digit of its own
+// (a sample sort with equality buckets: Sanders and Winkel, Super Scalar Sample
+// Sort, 2004).  Returns whether digit threadIdx.x (< 256) holds one value only.
+template <typename Bits>
+__device__ __forceinline__ bool sample_bounds(Bits* sorted) {
+  const uint32_t t = threadIdx.x;
+  Bits x = 0;
+  if (t < kSamples) {
+    x = sorted[t];
+    if (t > 0 && sorted[t - 1] == x && x != ~Bits(0)) ++x;
+  }
+  __syncthreads();
+  if (t < kSamples) sorted[t] = x;
+  __syncthreads();
+  if (t >= (uint32_t)kRadix) return false;
+  const Bits below = t > 0 ? sorted[t - 1] : Bits(0);
+  return t < kSamples ? sorted[t] - below == 1 : below == ~Bits(0);
+}
+
+template <int KT>
+__device__ __forceinline__ uint32_t sample_digit(typename Codec<KT>::Bits raw, const typename Codec<KT>::Bits* bounds) {
+  using Bits = typename Codec<KT>::Bits;
+  const Bits e = Codec<KT>::enc(raw);
+  // (in byte offsets: a step is a compare, a select and an add beside the load)
+  const char* const b = reinterpret_cast<const char*>(bounds);
+  uint32_t o = 0;
+#pragma unroll
+  for (uint32_t s = kRadix / 2; s > 0; s >>= 1)
+    o += *reinterpret_cast<const Bits*>(b + o + (s - 1) * sizeof(Bits)) <= e ? s * (uint32_t)sizeof(Bits) : 0u;
+  return o / (uint32_t)sizeof(Bits);
+}
+
+// Whether the sample's values bound the digits of a node with `left` levels to
+// go.  Even steps cost one multiplication per key instead of eight dependent
+// LDS reads, and leave uniform keys in children of one size, where the largest
+// of 256 digits between samples holds about 6 / 256 of the records (but that
+// whatever the keys are).  So the samples bound them only where steps would not
+// bring the children to the cap:
+// - on the last level, where a step has more samples than half the cap's share
+//   of them;
+// - before it, where one surely has more than the cap's share (two deviations;
+//   a step of uniform keys has one sample, the fullest of normal ones two), and
+//   either more than the later levels bring to the cap if each of them leaves a
+//   64th in its largest child, or the next level's steps, between the samples
+//   that share a step, would not part these: the exponents of floats fill a
+//   level's steps very unevenly, but the keys of one exponent are even.  The same
+//   value several times counts as not parted: its digit ends here.
+// Normal floats, 2^20: 85 us by steps, 114 with bounds from the sample on the first
+// level.
+// Sorted samples that share a step are neighbours, so a step has more than K of
+// them exactly if one shares it with the K-th after it: every wavefront looks at
+// all of them by itself, without a barrier.  sorted: the sample; key, low and high:
+// working space for 256 values each; every thread of the block calls it.
+template <typename Bits>
+__device__ __forceinline__ bool crowded(const Bits* sorted, const Steps<Bits>& st, uint32_t len, uint32_t cap, int left,
+                                        uint32_t* key, Bits* low, Bits* high) {
+  const uint32_t t = threadIdx.x, lane = t & (kWave - 1);
+  const float share = (float)cap * kRadix / (float)len;  // samples among cap records
+  const uint32_t may = max(4u, (uint32_t)(0.5f * share));
+  const uint32_t must = max(8u, (uint32_t)((1.0f + sqrtf(1.0f + share)) * (1.0f + sqrtf(1.0f + share))));
+  auto more_than = [&](uint32_t k, auto step) {
+    bool any = false;
+    for (uint32_t i = lane; i + k < kSamples; i += kWave) any |= step(i) == step(i + k);
+    return ballot64(any) != 0;
+  };
+  auto step = [&](uint32_t i) { return step_of<Bits>(sorted[i], st); };
+  if (left == 1) return more_than(may, step);
+  if (!more_than(must, step)) return false;
+  if (more_than(max(must, (uint32_t)min((float)kSamples, share * (left == 2 ? 64.0f : 4096.0f))), step)) return true;
+  const uint32_t d = t < kSamples ? step(t) : 0u;
+  if (t < kSamples) {
+    if (t == 0 || step(t - 1) != d) low[d] = sorted[t];
+    if (t == kSamples - 1 || step(t + 1) != d) high[d] = sorted[t];
+  }
+  __syncthreads();
+  if (t < kSamples) {
+    const Bits a = low[d], w = high[d] - a;
+    key[t] = d * kRadix + (w ? (uint32_t)(254.0 * ((double)(sorted[t] - a) / (double)w)) : 0u);
+  }
+  __syncthreads();
+  const bool both = more_than(left == 2 ? may : must, [&](uint32_t i) { return key[i]; });
+  __syncthreads();  // key, low and high are the caller's again
+  return both;
 }
 
 // ---------------------------------------------------------------------------
@@ -422,17 +576,15 @@ __device__ __forceinline__ uint32_t step_digit(typename Codec<KT>::Bits raw, con
 constexpr int kCountBlock = 512;
 
 template <int KT>
-__global__ __launch_bounds__(kCountBlock) void seg_count_kernel(const typename Codec<KT>::Bits* __restrict__ src,
+__global__ __launch_bounds__(kCountBlock, 8) void seg_count_kernel(const typename Codec<KT>::Bits* __restrict__ src,
                                                                 SegTab tab, const uint64_t* place, Node* nodes,
                                                                 uint32_t* __restrict__ rows, uint32_t tile,
-                                                                SegCtl* ctl, int level, uint32_t whole) {
+                                                                uint32_t cap, SegCtl* ctl, int level, int left,
+                                                                uint32_t whole) {
   using Bits = typename Codec<KT>::Bits;
-  constexpr int kSamples = 256;
-  __shared__ Bits smp[kSamples];
-  __shared__ uint32_t rank[kSamples], same[kSamples];
-  __shared__ Bits s_lo, s_hi, s_mid;
-  __shared__ uint32_t s_same;
-  __shared__ uint32_t h[kCountBlock / 128][kRadix];
+  __shared__ Bits smp[kRadix], bounds[kRadix];
+  __shared__ uint32_t rank[kRadix];
+  __shared__ alignas(8) uint32_t h[kCountBlock / 128][kRadix];
   uint32_t n_nodes = 1, n_tiles = (whole + tile - 1) / tile;
   if (whole == 0) {
     n_nodes = (uint32_t)(ctl->alloc[level] >> 32);
@@ -452,7 +604,7 @@ __global__ __launch_bounds__(kCountBlock) void seg_count_kernel(const typename C
   const int tid = threadIdx.x;
   uint32_t* const my = h[tid / 128];  // one histogram per two wavefronts
   uint32_t ni = whole ? 0 : find_node(nodes, n_nodes, g0);
-  bool fresh = true;
+  bool fresh = true, by_sample = false;
   Steps<Bits> st{};
   uint32_t len = 0, tile0 = 0;
   const Bits* keys = nullptr;
@@ -470,42 +622,18 @@ __global__ __launch_bounds__(kCountBlock) void seg_count_kernel(const typename C
         len = nodes[ni].len;
         tile0 = nodes[ni].tile0;
       }
-      if (tid < kSamples) {
-        smp[tid] = Codec<KT>::enc(keys[((uint64_t)tid * (len - 1)) / (kSamples - 1)]);
-        rank[tid] = 0;
-        same[tid] = 0;
+      sort_sample<KT, kCountBlock>(keys, len, smp, rank, bounds);
+      // between the third and the third last sample and a sixty-fourth of their
+      // distance further on both sides, or a thirty-second where the steps then
+      // still reach the cap (a sixty-fourth leaves more than 0.7% of uniform keys
+      // below or above in one array of ten, and 2^20 u64 keys a second level:
+      // 58 us -> 82); or a step per value around all samples where 254 cover them
+      Bits lo = bounds[0], hi = bounds[kSamples - 1], more = (253 - (hi - lo)) / 2;
+      if (hi - lo > 253) {
+        lo = bounds[2];
+        hi = bounds[kSamples - 3];
+        more = (hi - lo) / (len / 238 <= cap ? 32 : 64);
       }
-      __syncthreads();
-      // rank of every sample, half of the others per thread (ties by place)
-      {
-        const int i = tid & (kSamples - 1), from = tid / kSamples * (kSamples / 2);
-        const Bits x = smp[i];
-        uint32_t r = 0, e = 0;
-#pragma unroll 8
-        for (int j = from; j < from + kSamples / 2; ++j) {
-          const bool eq = smp[j] == x;
-          r += (smp[j] < x || (eq && j < i)) ? 1u : 0u;
-          e += eq ? 1u : 0u;
-        }
-        atomicAdd(&rank[i], r);
-        atomicAdd(&same[i], e);
-      }
-      __syncthreads();
-      if (tid < kSamples) {
-        if (rank[tid] == 2) s_lo = smp[tid];
-        if (rank[tid] == kSamples - 3) s_hi = smp[tid];
-        if (rank[tid] == kSamples / 2) {
-          s_mid = smp[tid];
-          s_same = same[tid];
-        }
-      }
-      __syncthreads();
-      // a sixty-fourth of their distance further on both sides; or, where
-      // half of the samples are one value, steps of one from that value on:
-      // its records are done, the others go below and above
-      const bool heavy = s_same >= kSamples / 2;
-      Bits lo = heavy ? s_mid : s_lo, hi = heavy ? s_mid : s_hi;
-      const Bits more = (hi - lo) / 64;
       lo = lo > more ? lo - more : Bits(0);
       hi = ~Bits(0) - hi > more ? hi + more : ~Bits(0);
       st.base = lo;
@@ -513,29 +641,43 @@ __global__ __launch_bounds__(kCountBlock) void seg_count_kernel(const typename C
       const Bits range = hi - lo;
       st.mul = 0;
       st.shift = 0;
+      by_sample = false;
       if (range > 253) {  // 254 even steps
         st.shift = (uint32_t)max(bit_width<Bits>(range) - 32, 0);
         st.mul = (uint32_t)((254ull << 32) / ((uint64_t)(uint32_t)(range >> st.shift) + 1u));
+        static_assert(sizeof(h) >= kRadix * sizeof(Bits), "working space");
+        if (len > cap) by_sample = crowded<Bits>(bounds, st, len, cap, left, rank, smp, reinterpret_cast<Bits*>(&h[0][0]));
+      }
+      if (by_sample) {
+        const uint64_t one = ballot64(sample_bounds<Bits>(bounds));
+        if (tid < kRadix && (tid & (kWave - 1)) == 0 && tile0 >= g0) nodes[ni].same[tid / kWave] = one;
       }
       if (tid == 0 && tile0 >= g0) {
         nodes[ni].base = (uint64_t)st.base;
         nodes[ni].top = (uint64_t)st.top;
         nodes[ni].mul = st.mul;
-        nodes[ni].shift = st.shift;
+        nodes[ni].shift = by_sample ? (uint32_t)kBySample : st.shift;
       }
     }
     for (int i = tid; i < (kCountBlock / 128) * kRadix; i += kCountBlock) (&h[0][0])[i] = 0;
     __syncthreads();
     const uint32_t t0 = (g - tile0) * tile, t1 = min(len, t0 + tile);
-    uint32_t i = t0 + tid;
-    for (; i + 7 * kCountBlock < t1; i += 8 * kCountBlock) {
-      Bits k[8];
+    // U keys at a time in flight
+    auto count = [&](auto U, auto digit) {
+      uint32_t i = t0 + tid;
+      for (; i + (U - 1) * kCountBlock < t1; i += U * kCountBlock) {
+        Bits k[U];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) k[u] = keys[i + u * kCountBlock];
+        for (int u = 0; u < U; ++u) k[u] = keys[i + u * kCountBlock];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) lds_count_wave(my, step_digit<KT>(k[u], st));
-    }
-    for (; i < t1; i += kCountBlock) lds_count_wave(my, step_digit<KT>(keys[i], st));
+        for (int u = 0; u < U; ++u) lds_count_wave(my, digit(k[u]));
+      }
+      for (; i < t1; i += kCountBlock) lds_count_wave(my, digit(keys[i]));
+    };
+    if (by_sample)
+      count(std::integral_constant<int, 4>{}, [&](Bits x) { return sample_digit<KT>(x, bounds); });
+    else
+      count(std::integral_constant<int, 8>{}, [&](Bits x) { return step_digit<KT>(x, st); });
     __syncthreads();
     if (tid < kRadix) {
       uint32_t s = 0;
@@ -603,17 +745,18 @@ __global__ __launch_bounds__(kRadix) void seg_chunk_kernel(const Node* __restric
 // hundreds of tiles, 1 for the later ones, whose nodes are many and short.
 // ---------------------------------------------------------------------------
 template <int PARTS>
-__global__ __launch_bounds__(PARTS * kRadix) void seg_scan_kernel(const Node* __restrict__ nodes,
+__global__ __launch_bounds__(PARTS * kRadix) void seg_scan_kernel(Node* __restrict__ nodes,
                                                                   uint32_t* __restrict__ rows,
                                                                   uint32_t* __restrict__ chunks, uint32_t tile,
-                                                                  uint32_t cap, uint32_t dst, int last,
+                                                                  uint32_t cap, uint32_t src, uint32_t dst, int last,
                                                                   Node* __restrict__ next, uint4* __restrict__ batches,
                                                                   uint4* __restrict__ longs, SegCtl* __restrict__ ctl,
                                                                   int level) {
   __shared__ uint32_t part[PARTS][kRadix];
   __shared__ uint32_t s_off[kRadix + 1], s_step[kRadix];
   __shared__ uint32_t sums[4], sums2[4], sums3[4];
-  __shared__ uint64_t s_own[kRadix / kWave], s_cut[kRadix / kWave];
+  __shared__ uint64_t s_own[kRadix / kWave], s_cut[kRadix / kWave], s_equal[kRadix / kWave];
+  __shared__ uint32_t s_first[kRadix], s_src;
   __shared__ uint32_t s_max, s_batch, s_long;
   __shared__ uint64_t s_next;
   const int tid = threadIdx.x, q = tid / kRadix, d = tid & (kRadix - 1), lane = tid & (kWave - 1);
@@ -647,12 +790,14 @@ __global__ __launch_bounds__(PARTS * kRadix) void seg_scan_kernel(const Node* __
     if (tid < kRadix) s_off[d] = excl;
     if (tid == 0) s_off[kRadix] = nd.len;
     // Children longer than the cap are done if every key is the same (equal: a
-    // step of one value) or split again (big).  The others are batched where
+    // digit of one value; one that is all of the node stays where it is and the
+    // scatter skips the node) or split again (big).  The others are batched where
     // floor(offset / T) agrees, T = cap - (the largest of them up to cap / 2; a
     // longer one is a batch by itself), so that a batch fits the cap.
     const bool child = tid < kRadix && cnt > 0;
     const bool over = child && cnt > cap;
-    const bool equal = over && nd.mul == 0 && d >= 1 && d <= 254;
+    const bool equal = over && (nd.shift == kBySample ? ((nodes[ni].same[d / kWave] >> lane) & 1u) != 0
+                                                      : nd.mul == 0 && d >= 1 && d <= 254);
     const bool big = over && !equal;
     const bool own = over || (child && cnt > cap / 2);  // not batched with others
     if (tid < kRadix) {
@@ -707,14 +852,23 @@ __global__ __launch_bounds__(PARTS * kRadix) void seg_scan_kernel(const Node* __
       }
     }
     const uint32_t len = cut ? s_off[end] - excl : 0u;
-    // batches of the local sort; an equal child in the scratch is cut into
-    // caps to be copied to the output
+    // batches of the local sort; an equal child that is not in the output is
+    // cut into caps to be copied there
+    const bool stays = equal && cnt == nd.len;
+    if (stays) nodes[ni].shift = kDone;
+    const uint32_t at = stays ? src : dst;
     uint32_t nb = cut && len > 0 && !over ? 1u : 0u;
-    if (equal && dst != kSrcOut) nb = (cnt + cap - 1) / cap;
+    if (equal && at != kSrcOut) nb = (cnt + cap - 1) / cap;
     const uint32_t bigs = big ? 1u : 0u, bigt = big && !last ? (cnt + tile - 1) / tile : 0u;
     const uint32_t eb = block_excl_scan_256(nb, sums, tid);
     const uint32_t en = block_excl_scan_256(bigs, sums2, tid);
     const uint32_t et = block_excl_scan_256(bigt, sums3, tid);
+    if (tid < kRadix) {
+      const uint64_t m = ballot64(equal && nb > 0);
+      if (lane == 0) s_equal[d / kWave] = m;
+      s_first[d] = eb;
+      if (equal && nb > 0) s_src = at;  // (one that stays is the node's only child)
+    }
     if (tid == kRadix - 1) {
       if (eb + nb) s_batch = atomicAdd(&ctl->n_batches, eb + nb);
       if (en + bigs) {
@@ -730,12 +884,16 @@ __global__ __launch_bounds__(PARTS * kRadix) void seg_scan_kernel(const Node* __
       if (last)
         longs[s_long + en] = make_uint4(nd.seg, nd.off + excl, cnt, dst);
       else
-        next[(uint32_t)(s_next >> 32) + en] = Node{nd.seg, nd.off + excl, cnt, (uint32_t)s_next + et, 0, 0, 0, 0};
-    } else if (equal) {
-      for (uint32_t i = 0; i < nb; ++i)
-        batches[s_batch + eb + i] = make_uint4(nd.seg, nd.off + excl + i * cap, min(cap, cnt - i * cap), dst);
-    } else if (nb) {
+        next[(uint32_t)(s_next >> 32) + en] = Node{nd.seg, nd.off + excl, cnt, (uint32_t)s_next + et, 0, 0, 0, 0, {}};
+    } else if (nb && !equal) {
       batches[s_batch + eb] = make_uint4(nd.seg, nd.off + excl, len, dst);
+    }
+    for (int g = 0; g < kRadix / kWave; ++g) {  // equal children may have thousands: the whole block writes each one's
+      for (uint64_t m = s_equal[g]; m != 0; m &= m - 1) {
+        const uint32_t c = g * kWave + (uint32_t)__builtin_ctzll(m), o = s_off[c], n = s_off[c + 1] - o;
+        for (uint32_t i = tid; i * cap < n; i += PARTS * kRadix)
+          batches[s_batch + s_first[c] + i] = make_uint4(nd.seg, nd.off + o + i * cap, min(cap, n - i * cap), s_src);
+      }
     }
     __syncthreads();
   }
@@ -763,6 +921,9 @@ __global__ __launch_bounds__(BLOCK, WAVES) void seg_scatter_kernel(
   __shared__ uint32_t off[W][kRadix];
   __shared__ uint32_t gbase[kRadix];
   __shared__ uint32_t sums[4];
+  __shared__ Bits bounds[kRadix];
+  __shared__ uint8_t dstage[TILE];  // digits between samples: a search is too long to repeat
+  uint32_t bounds_of = 0xFFFFFFFFu;  // the node whose sample they are
   const uint32_t n_nodes = (uint32_t)(ctl->alloc[level] >> 32), n_tiles = (uint32_t)ctl->alloc[level];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), w = (int)readfirstlane((uint32_t)(tid / kWave));
   for (int i = lane; i < kRadix; i += kWave) off[w][i] = 0;
@@ -774,7 +935,15 @@ __global__ __launch_bounds__(BLOCK, WAVES) void seg_scatter_kernel(
   for (uint32_t g = first + j0; g < stop; g += stride) {
     const uint32_t ni = find_node(nodes, n_nodes, g);
     const Node nd = nodes[ni];
-    const Steps<Bits> st{(Bits)nd.base, (Bits)nd.top, nd.mul, nd.shift};
+    if (nd.shift == kDone) continue;
+    const bool by_sample = nd.shift == kBySample;
+    const Steps<Bits> st{(Bits)nd.base, (Bits)nd.top, nd.mul, by_sample ? 0u : nd.shift};
+    if (by_sample && bounds_of != ni) {  // the sample anew (the count's would take 2 KB of scratch per node)
+      static_assert(TILE * sizeof(Bits) >= kRadix * (sizeof(Bits) + sizeof(uint32_t)), "sort_sample's working space");
+      sort_sample<KT, BLOCK>(src + sp[nd.seg] + nd.off, nd.len, keys, reinterpret_cast<uint32_t*>(keys + kRadix), bounds);
+      sample_bounds<Bits>(bounds);
+      bounds_of = ni;
+    }
     const uint32_t t0 = (g - nd.tile0) * (uint32_t)TILE;
     const uint32_t cnt = min((uint32_t)TILE, nd.len - t0);
     const bool full = cnt == (uint32_t)TILE;
@@ -797,19 +966,27 @@ __global__ __launch_bounds__(BLOCK, WAVES) void seg_scatter_kernel(
         static_for<IPT>([&](auto i) { v[i] = wb + i * kWave < cnt ? vin[wb + i * kWave] : VS(0); });
       }
     }
-    uint32_t r[IPT];
+    uint32_t r[IPT];  // digit << 16 | place among the wavefront's of this digit
+    static_assert(TILE <= 65536, "a place takes 16 bits");
     uint32_t* const ct = off[w];
+    if (by_sample) {
+      static_for<IPT>([&](auto i) {
+        r[i] = sample_digit<KT>(k[i], bounds);
+        if constexpr (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // (more searches at once spill)
+      });
+    } else {
+      static_for<IPT>([&](auto i) { r[i] = step_digit<KT>(k[i], st); });
+    }
     if (full) {
-      const uint32_t d0 = step_digit<KT>(k[0], st);
-      if (__popcll(ballot64(d0 == readfirstlane(d0))) >= 16) {
-        static_for<IPT>([&](auto i) { r[i] = rank_wave_atomic<true>(step_digit<KT>(k[i], st), ct); });
+      if (__popcll(ballot64(r[0] == readfirstlane(r[0]))) >= 16) {
+        static_for<IPT>([&](auto i) { r[i] = r[i] << 16 | rank_wave_atomic<true>(r[i], ct); });
       } else {
-        static_for<IPT>([&](auto i) { r[i] = rank_wave_atomic<false>(step_digit<KT>(k[i], st), ct); });
+        static_for<IPT>([&](auto i) { r[i] = r[i] << 16 | rank_wave_atomic<false>(r[i], ct); });
       }
     } else {
       static_for<IPT>([&](auto i) {
-        r[i] = 0;
-        if (wb + i * kWave < cnt) r[i] = rank_wave_atomic<true>(step_digit<KT>(k[i], st), ct);
+        if (wb + i * kWave < cnt) r[i] = r[i] << 16 | rank_wave_atomic<true>(r[i], ct);
+        else r[i] = 0;
       });
     }
     __syncthreads();
@@ -830,7 +1007,12 @@ __global__ __launch_bounds__(BLOCK, WAVES) void seg_scatter_kernel(
       gbase[tid] = row - excl;
     }
     __syncthreads();
-    static_for<IPT>([&](auto i) { r[i] += ct[step_digit<KT>(k[i], st)]; });
+    if (by_sample) {
+      static_for<IPT>([&](auto i) {
+        if (full || wb + i * kWave < cnt) dstage[(r[i] & 0xFFFFu) + ct[r[i] >> 16]] = (uint8_t)(r[i] >> 16);
+      });
+    }
+    static_for<IPT>([&](auto i) { r[i] = (r[i] & 0xFFFFu) + ct[r[i] >> 16]; });
     static_for<IPT>([&](auto i) {
       if (full || wb + i * kWave < cnt) {
         keys[r[i]] = k[i];
@@ -844,15 +1026,21 @@ __global__ __launch_bounds__(BLOCK, WAVES) void seg_scatter_kernel(
     Bits* const ko = dst + dp[nd.seg] + nd.off;
     V* vo = nullptr;
     if constexpr (HV) vo = vdst + dvp[nd.seg] + nd.off;
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) {
+    auto write = [&](int j, auto digit) {
       const uint32_t i = (uint32_t)(j * BLOCK + tid);
       if (full || i < cnt) {
         const Bits kk = keys[i];
-        const uint32_t o = min(gbase[step_digit<KT>(kk, st)] + i, top);
+        const uint32_t o = min(gbase[digit(kk, i)] + i, top);
         ko[o] = kk;
         if constexpr (HV) vo[o] = vstage[i];
       }
+    };
+    if (by_sample) {
+#pragma unroll 4
+      for (int j = 0; j < IPT; ++j) write(j, [&](Bits, uint32_t i) { return (uint32_t)dstage[i]; });
+    } else {
+#pragma unroll
+      for (int j = 0; j < IPT; ++j) write(j, [&](Bits x, uint32_t) { return step_digit<KT>(x, st); });
     }
     __syncthreads();
   }
@@ -975,11 +1163,10 @@ template <int KB, int VB>
 SegLayout seg_layout(size_t max_total, size_t nseg, size_t max_seg, int large_tile, bool wide_range) {
   constexpr size_t cap = SegCfg<KB, VB>::kCap;
   SegLayout L{};
-  // Levels of splitting: two reach the cap for segments up to 2^20 records
-  // unless their keys are skewed on more than two scales (the long kernel
-  // then takes what is left); longer ones get a third, and so do doubles from
-  // 2^15 on, whose encoded range around zero spans 2000 exponents (normal
-  // doubles, 2^20: 243 us with two levels and the long kernel).
+  // Levels of splitting: two reach the cap for segments up to 2^20 records;
+  // longer ones get a third, and so do doubles from 2^15 on: their encoded range
+  // around zero spans 2000 exponents, and equal steps may take a level
+  // to part these.
   L.levels = max_seg > (wide_range ? size_t(1) << 15 : size_t(1) << 20) ? 3 : 2;
   // a batch that a node's children form holds more than cap / 2 records on
   // average but for one per node and the breaks at children above cap / 2
@@ -1108,17 +1295,17 @@ int seg_typed(const void* kin, void* kout, const void* vin, void* vout, const ui
     const uint64_t* dvp = to_alt ? tab.alt : tab.vbegin;
     auto count = seg_count_kernel<KT>;
     count<<<std::min(L.tiles_ub[l], seg_resident(count, kCountBlock)), kCountBlock, 0, s>>>(
-        ks, tab, sp, nodes[l], rows, tile, ctl, l, l == 0 ? whole : 0u);
+        ks, tab, sp, nodes[l], rows, tile, C::kCap, ctl, l, L.levels - l, l == 0 ? whole : 0u);
     if (chunks != nullptr)
       seg_chunk_kernel<<<std::min(L.tiles_ub[l] / kChunk + 1, 2048u), kRadix, 0, s>>>(nodes[l], rows, chunks, ctl, l);
     const bool last = l + 1 == L.levels;
-    const uint32_t to = to_alt ? kSrcAlt : kSrcOut;
+    const uint32_t from = l == 0 ? kSrcIn : from_alt ? kSrcAlt : kSrcOut, to = to_alt ? kSrcAlt : kSrcOut;
     if (l == 0)
-      seg_scan_kernel<4><<<std::min(L.nodes_ub[l], 512u), 4 * kRadix, 0, s>>>(nodes[l], rows, chunks, tile, C::kCap, to, last ? 1 : 0,
+      seg_scan_kernel<4><<<std::min(L.nodes_ub[l], 512u), 4 * kRadix, 0, s>>>(nodes[l], rows, chunks, tile, C::kCap, from, to, last ? 1 : 0,
                                                                              last ? nullptr : nodes[l + 1], batches,
                                                                              longs, ctl, l);
     else
-      seg_scan_kernel<1><<<std::min(L.nodes_ub[l], 2048u), kRadix, 0, s>>>(nodes[l], rows, chunks, tile, C::kCap, to, last ? 1 : 0,
+      seg_scan_kernel<1><<<std::min(L.nodes_ub[l], 2048u), kRadix, 0, s>>>(nodes[l], rows, chunks, tile, C::kCap, from, to, last ? 1 : 0,
                                                                          last ? nullptr : nodes[l + 1], batches, longs,
                                                                          ctl, l);
     scatter<<<std::min(L.tiles_ub[l], seg_resident(scatter, block)), block, 0, s>>>(

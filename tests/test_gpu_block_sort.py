@@ -253,3 +253,122 @@ def test_doubles_take_splits(mg, dist):
     rng = np.random.default_rng(6)
     keys = random_keys(O.K_F64, (1 << 24) + 77, rng, dist)
     assert run_sort(mg, O.K_F64, None, keys, rng, inplace=True) == 4
+
+
+def skewed_keys(kt, n, rng, dist):
+    """Keys that even steps do not divide: log: every binary order of
+    magnitude equally often; zipf: small counts, 1 in 87% of the places (10%
+    in 4-byte keys); near: 1 - eps over 50 orders of eps; four: four values
+    2^-30, 2^-20 and 2^-10 apart; shares: 55% 0, 25% 1, 12% 2, the rest
+    spread; geometric: counts, halving; single: one value."""
+    bd = O.BITS_DTYPE[kt]
+    fd = np.float32 if bd == np.uint32 else np.float64
+    u = rng.random(n)
+    if dist == "log":
+        x = np.exp2(u * (31 if bd == np.uint32 else 63))
+    elif dist == "zipf":
+        x = np.minimum(np.maximum(u, 1e-9) ** (-5 if bd == np.uint64 else -2), 2.0**20)
+    elif dist == "near":
+        x = 1 - np.exp2(-50 * u)
+    elif dist == "four":
+        x = np.array([1, 1 + 2.0**-30, 1 + 2.0**-20, 1 + 2.0**-10])[rng.integers(0, 4, n)]
+    elif dist == "shares":
+        x = np.where(u < 0.55, 0, np.where(u < 0.8, 1, np.where(u < 0.92, 2, rng.random(n) * 1000)))
+    elif dist == "geometric":
+        x = np.floor(-np.log2(1 - u)) + 1
+    else:
+        x = np.full(n, 3.0)
+    return x.astype(fd).view(bd) if kt in (O.K_F32, O.K_F64) else x.astype(bd)
+
+
+def left_to_one_workgroup(temp):
+    """How many ranges the last level of splits left to a workgroup each (the
+    fourth word of the scratch)."""
+    return int(from_dev(temp[12:16], np.uint32)[0])
+
+
+STRAYS = 2  # a child that the sample puts below the longest sorted in LDS may be a little above it
+
+
+SKEWED = [(kt, vdt, d) for kt, vdt, ds in ((O.K_U64, None, "log zipf single"), (O.K_I32, np.uint32, "log zipf"),
+                                           (O.K_U64, np.uint64, "log zipf"), (O.K_F32, None, "near shares geometric"),
+                                           (O.K_F64, np.uint32, "near four shares geometric log single"))
+          for d in ds.split()]
+
+
+@pytest.mark.parametrize("kt,vdt,dist", SKEWED, ids=lambda v: str(v))
+@pytest.mark.parametrize("n", [200_003, 1 << 20, (1 << 23) - 1])
+def test_splits_divide_skewed_keys(mg, kt, vdt, dist, n):
+    """However the keys are distributed, the levels bring the children to what
+    one workgroup sorts in LDS: next to none is left to one that streams it."""
+    import torch
+    rng = np.random.default_rng(n + kt)
+    keys = skewed_keys(kt, n, rng, dist)
+    vals = None if vdt is None else random_vals(vdt, n, rng)
+    vt = mg.VAL_NONE if vdt is None else (mg.VAL_U32 if vdt == np.uint32 else mg.VAL_U64)
+    for inplace in (False, True):
+        temp = mg.temp_buffer(mg.lib.mgs_sort_temp_bytes(kt, vt, n), "cuda")
+        dk, dv = to_dev(keys), to_dev(vals)
+        ok = dk if inplace else torch.empty_like(dk)
+        ov = dv if inplace or dv is None else torch.empty_like(dv)
+        mg.sort(KEY_NAME[kt], dk, dv, keys_out=ok, vals_out=ov, temp=temp)
+        assert mg.lib.mgs_sort_path(kt, vt, n, mg._ptr(temp), temp.numel(), None) == 4
+        assert mg.temp_status(temp) == 0
+        assert left_to_one_workgroup(temp) <= STRAYS
+        ek, ev = O.sort(kt, keys, vals)
+        assert np.array_equal(from_dev(ok, keys.dtype), ek)
+        if vdt is not None:
+            assert np.array_equal(from_dev(ov, vdt), ev)
+
+
+@pytest.mark.parametrize("kt,vdt,dist", [v for v in SKEWED if v[1] != np.uint64], ids=lambda v: str(v))
+def test_segments_of_skewed_keys(mg, kt, vdt, dist):
+    """The same for segments of all lengths, each variant of the scatter."""
+    import torch
+    rng = np.random.default_rng(kt + 31)
+    lens = [0, 3, 300, 5119, 8193, 70_001, 300_002, 20_000, 1_100_003, 9000]
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint64)
+    keys = np.concatenate([skewed_keys(kt, n, rng, dist) for n in lens])
+    vals = None if vdt is None else random_vals(vdt, keys.size, rng)
+    vt = mg.VAL_NONE if vdt is None else mg.VAL_U32
+    ek, ev = O.segmented_sort(kt, keys, off, vals)
+    for variant in range(mg.lib.mgs_segmented_variant_count()):
+        dk, dv = to_dev(keys), to_dev(vals)
+        temp = mg.temp_buffer(mg.lib.mgs_segmented_sort_temp_bytes(kt, vt, keys.size, len(lens)) * 2, "cuda")
+        mg.segmented_sort(KEY_NAME[kt], dk, torch.from_numpy(off.view(np.int64)).cuda(), dv,
+                          tuning=mg.Tuning(variant, 0, 0, 0), temp=temp)
+        assert mg.temp_status(temp) == 0
+        assert left_to_one_workgroup(temp) <= STRAYS
+        assert np.array_equal(from_dev(dk, keys.dtype), ek)
+        if vdt is not None:
+            assert np.array_equal(from_dev(dv, vdt), ev)
+
+
+@pytest.mark.parametrize("vdt", [np.uint32, np.uint64], ids=str)
+@pytest.mark.parametrize("dist", ["uniform", "nested", "heavy"])
+def test_doubles_with_payloads_take_splits(mg, vdt, dist):
+    rng = np.random.default_rng(16)
+    n = (1 << 23) + 12_345
+    keys = scaled_keys(O.K_F64, n, rng, dist) if dist != "uniform" else random_keys(O.K_F64, n, rng)
+    assert run_sort(mg, O.K_F64, vdt, keys, rng, inplace=False) == 4
+
+
+@pytest.mark.parametrize("n,path", [(3584 * (254 * 254 // 8 * 7) - 1, 4), (3584 * (254 * 254 // 8 * 7), 2)], ids=str)
+def test_doubles_end_of_splits(mg, n, path):
+    """16-byte records on both sides of the longest that sorts by splits,
+    checked on the device: ascending, the payloads (places) with their keys, in
+    order where keys are equal."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    k = torch.floor(torch.randn(n, dtype=torch.float64, device="cuda", generator=g) * 2.0**20)
+    v = torch.arange(n, dtype=torch.int64, device="cuda")
+    temp = mg.temp_buffer(mg.lib.mgs_sort_temp_bytes(O.K_F64, mg.VAL_U64, n), "cuda")
+    ko, vo = torch.empty_like(k), torch.empty_like(v)
+    mg.sort("f64", k, v, keys_out=ko, vals_out=vo, temp=temp)
+    assert mg.lib.mgs_sort_path(O.K_F64, mg.VAL_U64, n, mg._ptr(temp), temp.numel(), None) == path
+    assert mg.temp_status(temp) == 0
+    assert path != 4 or left_to_one_workgroup(temp) <= STRAYS
+    same = ko[1:] == ko[:-1]
+    assert bool(((ko[1:] > ko[:-1]) | (same & (vo[1:] > vo[:-1]))).all())
+    assert torch.equal(k[vo], ko)
