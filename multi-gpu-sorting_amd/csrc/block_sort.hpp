@@ -37,8 +37,8 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_each(static_cast<F&&>(f), std::make_integer_sequence<int, N>{});
 }
 
-// Records that a thread puts in order on each side of the first one below its
-// predecessor.
+// Fewer records than this are put in order by one thread on each side of one
+// below its predecessor.
 constexpr uint32_t kTieReach = 16;
 // LDS counter rows of the 9-bit digits, one per wavefront.  The row stride
 // puts the two threads that scan one digit's 16 rows on different banks.
@@ -324,45 +324,51 @@ __device__ __forceinline__ void block_sort(BlockSortSmem<typename Codec<KT>::Bit
   auto stored = [] { __builtin_amdgcn_s_waitcnt(0); };
   stored();
   if (!__syncthreads_or(down != 0 ? 1 : 0)) return;
-  // Groups out of order: the thread that sees the first record of a group
-  // below its predecessor writes the whole group in order.  A group that
-  // reaches further than kTieReach from there is left to the passes.
-  bool slow = false;
+  // A group that reaches kTieReach from a record below its predecessor is left to
+  // the passes over all bits.  Every such record is asked before any group
+  // is mended: keys that crowd in the window (log-uniform ones: half of them)
+  // have many, and walking through their groups first took longer than the
+  // passes: 2000 u64 keys 75 us, now 21.
   const Bits lim = Bits(1) << low;
   auto image = [&](uint32_t p) { return Codec<KT>::enc(sm.keys[p]); };
-  while (down != 0) {
-    const uint32_t p = (uint32_t)__builtin_ctz(down) * BLOCK + tid;
-    down &= down - 1;
-    uint32_t l = p - 1, r = p;
-    Bits e = image(l);
-    bool first = true;
-    while (l > 0) {
-      const Bits x = image(l - 1);
-      if ((x ^ e) >= lim) break;
-      if (x > e) first = false;
-      if (!first || p - l > kTieReach) break;
-      e = x;
-      --l;
-    }
-    if (!first) continue;
-    while (r + 1 < m && (image(r + 1) ^ e) < lim && r - p <= kTieReach) ++r;
-    if (p - l > kTieReach || r - p > kTieReach) {
-      slow = true;
-      continue;
-    }
-    for (uint32_t q = l; q <= r; ++q) {
-      const Bits raw = sm.keys[q], x = Codec<KT>::enc(raw);
-      uint32_t to = l;
-      for (uint32_t t = l; t <= r; ++t) {
-        const Bits y = image(t);
-        to += (y < x || (y == x && t < q)) ? 1u : 0u;
-      }
-      store(to, raw);
-      if constexpr (HV) store_val(to, sm.vals[q]);
-    }
+  bool longer = false;
+  for (uint32_t rest = down; rest != 0; rest &= rest - 1) {
+    const uint32_t p = (uint32_t)__builtin_ctz(rest) * BLOCK + tid;
+    const Bits e = image(p);
+    longer |= p + kTieReach < m && (image(p + kTieReach) ^ e) < lim;
+    longer |= p > kTieReach && (image(p - 1 - kTieReach) ^ e) < lim;
   }
-  stored();
-  if (!__syncthreads_or(slow ? 1 : 0)) return;
+  if (!__syncthreads_or(longer ? 1 : 0)) {
+    // the thread that sees the first record of a group below its predecessor
+    // writes the whole group in order
+    while (down != 0) {
+      const uint32_t p = (uint32_t)__builtin_ctz(down) * BLOCK + tid;
+      down &= down - 1;
+      uint32_t l = p - 1, r = p;
+      Bits e = image(l);
+      bool first = true;
+      while (l > 0 && first) {
+        const Bits x = image(l - 1);
+        if ((x ^ e) >= lim) break;
+        first = x <= e;
+        e = x;
+        --l;
+      }
+      if (!first) continue;
+      while (r + 1 < m && (image(r + 1) ^ e) < lim) ++r;
+      for (uint32_t q = l; q <= r; ++q) {
+        const Bits raw = sm.keys[q], x = Codec<KT>::enc(raw);
+        uint32_t to = l;
+        for (uint32_t t = l; t <= r; ++t) {
+          const Bits y = image(t);
+          to += (y < x || (y == x && t < q)) ? 1u : 0u;
+        }
+        store(to, raw);
+        if constexpr (HV) store_val(to, sm.vals[q]);
+      }
+    }
+    return;
+  }
   // all differing bits, from the present order
   for (int shift = 0; shift < bits; shift += kBlockDigitBits) {
     reload();

@@ -372,3 +372,32 @@ def test_doubles_end_of_splits(mg, n, path):
     same = ko[1:] == ko[:-1]
     assert bool(((ko[1:] > ko[:-1]) | (same & (vo[1:] > vo[:-1]))).all())
     assert torch.equal(k[vo], ko)
+
+
+@pytest.mark.parametrize("kt,dist", [(O.K_U64, "log"), (O.K_U32, "log"), (O.K_F64, "near"), (O.K_U64, "zipf")],
+                         ids=lambda v: str(v))
+@pytest.mark.parametrize("n", [2000, 6999])
+def test_crowded_windows(mg, kt, dist, n):
+    """Keys of which many share a window value: right, and by the passes over
+    all bits (at most three times the window's, so five times a sort of uniform
+    keys leaves room for the clock) instead of walks through long groups."""
+    import torch
+    rng = np.random.default_rng(n + kt)
+    us = {}
+    for d in ("uniform", dist):
+        keys = random_keys(kt, n, rng) if d == "uniform" else skewed_keys(kt, n, rng, d)
+        dk = to_dev(keys)
+        ok = torch.empty_like(dk)
+        temp = mg.temp_buffer(mg.lib.mgs_sort_temp_bytes(kt, mg.VAL_NONE, n), "cuda")
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        best = float("inf")
+        for _ in range(8):
+            begin.record()
+            for _ in range(50):
+                mg.sort(KEY_NAME[kt], dk, keys_out=ok, temp=temp)
+            end.record()
+            end.synchronize()
+            best = min(best, begin.elapsed_time(end))
+        us[d] = best * 20
+        assert np.array_equal(from_dev(ok, keys.dtype), O.sort(kt, keys)[0])
+    assert us[dist] < 5 * us["uniform"], us
