@@ -522,13 +522,14 @@ __device__ __forceinline__ uint32_t sample_digit(typename Codec<KT>::Bits raw, c
 //   of them;
 // - before it, where one surely has more than the cap's share (two deviations;
 //   a step of uniform keys has one sample, the fullest of normal ones two), and
-//   either more than the later levels bring to the cap if each of them leaves a
-//   64th in its largest child, or the next level's steps, between the samples
-//   that share a step, would not part these: the exponents of floats fill a
-//   level's steps very unevenly, but the keys of one exponent are even.  The same
-//   value several times counts as not parted: its digit ends here.
-// Normal floats, 2^20: 85 us by steps, 114 with bounds from the sample on the first
-// level.
+//   one of: the samples' largest child still fits (an eighth of the samples); the
+//   step has more than the later levels bring to the cap if each of them leaves a
+//   64th in its largest child; or the next level's steps, between the samples
+//   that share a step, would not part these.  So a level of steps comes before
+//   another where that helps: the exponents of floats fill a level's steps very
+//   unevenly, but the keys of one exponent are even (normal floats, 2^20: 85 us
+//   by steps, 114 with bounds from the sample on the first level).  The same value
+//   several times counts as not parted: its digit ends here.
 // Sorted samples that share a step are neighbours, so a step has more than K of
 // them exactly if one shares it with the K-th after it: every wavefront looks at
 // all of them by itself, without a barrier.  sorted: the sample; key, low and high:
@@ -548,6 +549,7 @@ __device__ __forceinline__ bool crowded(const Bits* sorted, const Steps<Bits>& s
   auto step = [&](uint32_t i) { return step_of<Bits>(sorted[i], st); };
   if (left == 1) return more_than(may, step);
   if (!more_than(must, step)) return false;
+  if (share >= 8.0f) return true;
   if (more_than(max(must, (uint32_t)min((float)kSamples, share * (left == 2 ? 64.0f : 4096.0f))), step)) return true;
   const uint32_t d = t < kSamples ? step(t) : 0u;
   if (t < kSamples) {

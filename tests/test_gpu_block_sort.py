@@ -287,9 +287,6 @@ def left_to_one_workgroup(temp):
     return int(from_dev(temp[12:16], np.uint32)[0])
 
 
-STRAYS = 2  # a child that the sample puts below the longest sorted in LDS may be a little above it
-
-
 SKEWED = [(kt, vdt, d) for kt, vdt, ds in ((O.K_U64, None, "log zipf single"), (O.K_I32, np.uint32, "log zipf"),
                                            (O.K_U64, np.uint64, "log zipf"), (O.K_F32, None, "near shares geometric"),
                                            (O.K_F64, np.uint32, "near four shares geometric log single"))
@@ -300,7 +297,7 @@ SKEWED = [(kt, vdt, d) for kt, vdt, ds in ((O.K_U64, None, "log zipf single"), (
 @pytest.mark.parametrize("n", [200_003, 1 << 20, (1 << 23) - 1])
 def test_splits_divide_skewed_keys(mg, kt, vdt, dist, n):
     """However the keys are distributed, the levels bring the children to what
-    one workgroup sorts in LDS: next to none is left to one that streams it."""
+    one workgroup sorts in LDS: none is left to one that streams it."""
     import torch
     rng = np.random.default_rng(n + kt)
     keys = skewed_keys(kt, n, rng, dist)
@@ -314,7 +311,7 @@ def test_splits_divide_skewed_keys(mg, kt, vdt, dist, n):
         mg.sort(KEY_NAME[kt], dk, dv, keys_out=ok, vals_out=ov, temp=temp)
         assert mg.lib.mgs_sort_path(kt, vt, n, mg._ptr(temp), temp.numel(), None) == 4
         assert mg.temp_status(temp) == 0
-        assert left_to_one_workgroup(temp) <= STRAYS
+        assert left_to_one_workgroup(temp) == 0
         ek, ev = O.sort(kt, keys, vals)
         assert np.array_equal(from_dev(ok, keys.dtype), ek)
         if vdt is not None:
@@ -338,7 +335,7 @@ def test_segments_of_skewed_keys(mg, kt, vdt, dist):
         mg.segmented_sort(KEY_NAME[kt], dk, torch.from_numpy(off.view(np.int64)).cuda(), dv,
                           tuning=mg.Tuning(variant, 0, 0, 0), temp=temp)
         assert mg.temp_status(temp) == 0
-        assert left_to_one_workgroup(temp) <= STRAYS
+        assert left_to_one_workgroup(temp) == 0
         assert np.array_equal(from_dev(dk, keys.dtype), ek)
         if vdt is not None:
             assert np.array_equal(from_dev(dv, vdt), ev)
@@ -368,7 +365,7 @@ def test_doubles_end_of_splits(mg, n, path):
     mg.sort("f64", k, v, keys_out=ko, vals_out=vo, temp=temp)
     assert mg.lib.mgs_sort_path(O.K_F64, mg.VAL_U64, n, mg._ptr(temp), temp.numel(), None) == path
     assert mg.temp_status(temp) == 0
-    assert path != 4 or left_to_one_workgroup(temp) <= STRAYS
+    assert path != 4 or left_to_one_workgroup(temp) == 0
     same = ko[1:] == ko[:-1]
     assert bool(((ko[1:] > ko[:-1]) | (same & (vo[1:] > vo[:-1]))).all())
     assert torch.equal(k[vo], ko)
