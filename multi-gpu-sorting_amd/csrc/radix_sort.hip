@@ -836,6 +836,15 @@ bool mid_path(int kb, int vb, bool floats, size_t n) {
   static const char* const kForcing[] = {"MGS_MSD", "MGS_MSD_MIN", "MGS_RANK_PEERS", "MGS_SKEW_PAIR_MIN",
                                          "MGS_XCD_LOCAL", "MGS_DESC_BUDGET", "MGS_LB_SPIN_LIMIT"};
   if (n >= mid_max(kb, vb, floats)) return false;
+  // 4-byte integer keys with payloads, whose four passes move the least per
+  // record: splits lose between the sizes where one workgroup's neighbours are
+  // few and where they fill the device, and with u64 payloads as soon as they
+  // need a second level (microseconds, splits against LSD passes: u32 + u32,
+  // uniform, 2^15.6 51 / 54, 2^17 59 / 48, 2^18 58 / 51, 2^18.5 55 / 63, 2^20 53 / 86;
+  // row numbers 2^17 58 / 44; zipf 2^17 72 / 52; u32 + u64 2^20 57 / 91, 2^21 133 / 108,
+  // 2^22 177 / 158)
+  if (kb == 4 && vb > 0 && !floats && n >= (size_t(1) << 16) && n < (size_t(3) << 17)) return false;
+  if (kb == 4 && vb == 8 && !floats && n >= (size_t(9) << 17)) return false;
   for (const char* name : kForcing)
     if (std::getenv(name) != nullptr) return false;
   return true;
