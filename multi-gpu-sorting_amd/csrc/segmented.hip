@@ -629,9 +629,16 @@ __global__ __launch_bounds__(kCountBlock, 8) void seg_count_kernel(const typenam
       // distance further on both sides, or a thirty-second where the steps then
       // still reach the cap (a sixty-fourth leaves more than 0.7% of uniform keys
       // below or above in one array of ten, and 2^20 u64 keys a second level:
-      // 58 us -> 82); or a step per value around all samples where 254 cover them
-      Bits lo = bounds[0], hi = bounds[kSamples - 1], more = (253 - (hi - lo)) / 2;
-      if (hi - lo > 253) {
+      // 58 us -> 82); or a step per value around the samples where 254 values,
+      // one below and one above cover them (keys of one byte)
+      Bits lo = bounds[0], hi = bounds[kSamples - 1], more;
+      if (hi - lo > 253 && hi - lo <= 255) {
+        ++lo;
+        hi = lo + 253;
+        more = 0;
+      } else if (hi - lo <= 253) {
+        more = (253 - (hi - lo)) / 2;
+      } else {
         lo = bounds[2];
         hi = bounds[kSamples - 3];
         more = (hi - lo) / (len / 238 <= cap ? 32 : 64);
