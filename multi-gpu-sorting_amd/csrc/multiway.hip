@@ -158,6 +158,12 @@ __device__ __forceinline__ uint64_t bound_global(const Bits* r, uint64_t lo, uin
 // are searched over the whole runs, the others between those of their coarse
 // neighbours, about half the dependent loads and on shared cache lines.
 constexpr uint64_t kMwCoarse = 16;
+// Two levels pay for their second launch where there are searches enough that
+// their loads, and not the longest search, bound the split kernel: whole call, one
+// level against two, u32: 64 runs of 2^19 313 / 307 us, of 2^22 2005 / 1709;
+// 256 of 2^20 4804 / 3424; 32 of 2^21 425 / 432, of 2^22 745 / 730; 16 of 2^23 543 / 553;
+// and up to 8 runs at no size (8 of 2^19 126 / 136, of 2^26 1819 / 1836).
+inline bool two_levels(uint64_t pieces, size_t k) { return k > 8 && pieces * k > (uint64_t(1) << 19); }
 
 // Thread (b, j'): split of run j' at boundary b (1 <= b < pieces); boundary
 // 0 and `pieces` are the runs' ends.  COARSE: the boundaries that are
@@ -516,8 +522,7 @@ int mw_launch(const void* const* runs, const size_t* lens, size_t k, void* out, 
   rc = sort_dispatch((mgs_key)KT, MGS_VAL_U32, sk, sk2, sid, sid2, ns, t + L.sort_temp,
                      sort_temp_bytes((mgs_key)KT, MGS_VAL_U32, ns), s);
   if (rc != MGS_OK) return rc;
-  // (one level where the pieces are few: a launch costs more than it saves)
-  const uint64_t coarse = L.pieces > 2048 ? kMwCoarse : 1;
+  const uint64_t coarse = two_levels(L.pieces, k) ? kMwCoarse : 1;
   mw_split_kernel<KT, true, Bits><<<grid_of(((L.pieces + coarse - 1) / coarse + 1) * k, 256), 256, 0, s>>>(
       d_runs, d_lens, d_sbase, (uint32_t)k, S, sk2, sid2, L.pieces, piece_step(KB, k), coarse, splits);
   if (coarse > 1)

@@ -78,6 +78,25 @@ def test_one_or_two_runs(mg, lens, portions):
     assert np.array_equal(from_dev(out, np.uint32), expect)
 
 
+@pytest.mark.parametrize("kt,k,total", [(O.K_U32, 256, 12_500_000), (O.K_U32, 256, 12_900_000),
+                                        (O.K_U64, 200, 14_000_000), (O.K_F32, 8, 13_000_000)], ids=lambda v: str(v))
+@pytest.mark.parametrize("dist", ["uniform", "pairs"])
+def test_multiway_split_levels(mg, kt, k, total, dist):
+    """Around 2^19 searches for the pieces' bounds, from where these take two levels."""
+    import torch
+    rng = np.random.default_rng(total + kt)
+    cuts = np.sort(rng.integers(0, total + 1, size=k - 1))
+    cuts = np.concatenate([[0], cuts, [total]])
+    keys = tied_keys(kt, total, rng, dist)
+    runs = [O.sort(kt, np.ascontiguousarray(keys[a:b]))[0] for a, b in zip(cuts[:-1], cuts[1:])]
+    expect = O.sort(kt, np.concatenate(runs))[0]
+    out = torch.empty(total, dtype=to_dev(expect).dtype, device="cuda")
+    temp = mg.temp_buffer(mg.lib.mgs_multiway_merge_temp_bytes(kt, k, total), "cuda")
+    mg.multiway_merge(KEY_NAME[kt], [to_dev(r) for r in runs], out, temp=temp)
+    assert mg.temp_status(temp) == 0
+    assert np.array_equal(from_dev(out, expect.dtype), expect)
+
+
 @pytest.mark.parametrize("kt", [O.K_U32, O.K_F64], ids=str)
 @pytest.mark.parametrize("k", [1, 2, 3, 9])
 def test_empty_runs(mg, kt, k):
