@@ -117,9 +117,13 @@ int mgs_sort(mgs_key kt, mgs_val vt,
  * callers that cannot allocate device memory: code under HIP graph capture,
  * tight serving loops).  Same kernels as mgs_sort; the scratch is a 64 MiB
  * array in the library's device memory, one per GPU, held until the process
- * ends, so n is limited to mgs_sort_temp_bytes(kt, vt, n) <= 64 MiB (2^23 - 1
- * u32 keys, about 8.3M u64 keys or u32 pairs, 5.5M u64 keys with u32
- * payloads); larger n returns MGS_ERR_TOO_LARGE.  Allocates nothing.  All
+ * ends, so n is limited to what the LSD passes take in 64 MiB: 2^23 - 1 keys
+ * of 4 bytes, 8303488 of 8 bytes, and with payloads records of 4 + 4 bytes
+ * 8307584, 4 + 8 bytes 5530176, 8 + 4 bytes 5527456, 8 + 8 bytes 4145600
+ * (more than mgs_sort_temp_bytes(kt, vt, n) <= 64 MiB admits: that scratch has
+ * room for the splits and the three passes of wider records too, and a sort
+ * without it takes the LSD passes); larger n returns MGS_ERR_TOO_LARGE.
+ * Allocates nothing.  All
  * calls on one GPU share its array: calls that overlap on one GPU (on
  * different streams or host threads) race and must be ordered by the
  * caller. */

@@ -67,3 +67,24 @@ def test_noalloc_size_limit(mg):
     # the size check comes before any access to the (short) buffer
     assert mg.lib.mgs_sort_noalloc(mg.KEY_U32, mg.VAL_NONE, k.data_ptr(), k.data_ptr(), None, None, n,
                                    torch.cuda.current_stream().cuda_stream) == -5
+
+
+@pytest.mark.parametrize("kt,vdt,most", [(O.K_U32, None, (1 << 23) - 1), (O.K_I64, None, 8303488),
+                                         (O.K_U32, np.uint32, 8307584), (O.K_I32, np.uint64, 5530176),
+                                         (O.K_U64, np.uint32, 5527456), (O.K_F64, np.uint64, 4145600)],
+                         ids=lambda v: str(v))
+def test_noalloc_documented_limits(mg, kt, vdt, most):
+    """The longest arrays that mgsort.h names, whose mgs_sort scratch with all
+    its paths may be more than the static array, and one record more."""
+    vt = mg.VAL_NONE if vdt is None else (mg.VAL_U32 if vdt == np.uint32 else mg.VAL_U64)
+    rng = np.random.default_rng(91 + kt)
+    keys = random_keys(kt, most, rng)
+    vals = random_vals(vdt, most, rng)
+    k, v = to_dev(keys), to_dev(vals)
+    # the size check comes before any access to the buffers
+    assert noalloc(mg, kt, vt, k, v, most + 1) == -5
+    assert noalloc(mg, kt, vt, k, v, most) == 0
+    ek, ev = O.sort(kt, keys, vals)
+    assert np.array_equal(from_dev(k, keys.dtype), ek)
+    if vdt is not None:
+        assert np.array_equal(from_dev(v, vdt), ev)
