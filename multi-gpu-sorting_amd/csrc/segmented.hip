@@ -82,13 +82,11 @@ enum : uint32_t { kBySample = 64, kDone = 65 };
 enum : uint32_t { kSrcIn = 0, kSrcAlt = 1, kSrcOut = 2 };
 
 // Per-segment table written by classify: first key in the key array, first
-// payload in the payload array, first slot in the compact scratch buffer,
-// length.
+// payload in the payload array, first slot in the compact scratch buffer.
 struct SegTab {
   uint64_t* begin;
   uint64_t* vbegin;
   uint64_t* alt;
-  uint32_t* len;
 };
 
 constexpr int kClassifyBlock = 1024;
@@ -217,7 +215,6 @@ __global__ __launch_bounds__(kClassifyBlock) void seg_classify_kernel(const uint
       tab.begin[s] = b;
       tab.vbegin[s] = (RANGES && val_begin != nullptr) ? val_begin[s] : b;
       tab.alt[s] = alt;
-      tab.len[s] = len;
     }
     const uint32_t bad = (s < nseg && !ok) ? 1u : 0u;
     const uint32_t is_s = (s < nseg && len > 0 && len <= small_max) ? 1u : 0u;
@@ -593,7 +590,6 @@ __global__ __launch_bounds__(kCountBlock, 8) void seg_count_kernel(const typenam
     n_tiles = (uint32_t)ctl->alloc[level];
   } else if (blockIdx.x == 0 && threadIdx.x == 0) {
     tab.begin[0] = tab.vbegin[0] = tab.alt[0] = 0;
-    tab.len[0] = whole;
     nodes[0].seg = nodes[0].off = nodes[0].tile0 = 0;
     nodes[0].len = whole;
     ctl->status = ctl->skipped = ctl->n_batches = ctl->n_long = 0;
@@ -1108,7 +1104,7 @@ constexpr size_t kAlign = 256;
 inline size_t align_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
 
 struct SegLayout {
-  size_t ctl, alt_k, alt_v, tab_begin, tab_vbegin, tab_alt, tab_len, nodes[kMaxLevels], batches, longs, rows, chunks, total;
+  size_t ctl, alt_k, alt_v, tab_begin, tab_vbegin, tab_alt, nodes[kMaxLevels], batches, longs, rows, chunks, total;
   uint32_t nodes_ub[kMaxLevels], tiles_ub[kMaxLevels], batches_ub;
   int levels;
 };
@@ -1200,7 +1196,6 @@ SegLayout seg_layout(size_t max_total, size_t nseg, size_t max_seg, int large_ti
   L.tab_begin = take(nseg * 8);
   L.tab_vbegin = take(nseg * 8);
   L.tab_alt = take(nseg * 8);
-  L.tab_len = take(nseg * 4);
   uint32_t tiles = 0;
   for (int l = 0; l < L.levels; ++l) {
     L.nodes[l] = take((size_t)L.nodes_ub[l] * sizeof(Node));
@@ -1277,7 +1272,7 @@ int seg_typed(const void* kin, void* kout, const void* vin, void* vout, const ui
   Node* nodes[kMaxLevels];
   for (int l = 0; l < L.levels; ++l) nodes[l] = reinterpret_cast<Node*>(t + L.nodes[l]);
   const SegTab tab{reinterpret_cast<uint64_t*>(t + L.tab_begin), reinterpret_cast<uint64_t*>(t + L.tab_vbegin),
-                   reinterpret_cast<uint64_t*>(t + L.tab_alt), reinterpret_cast<uint32_t*>(t + L.tab_len)};
+                   reinterpret_cast<uint64_t*>(t + L.tab_alt)};
   const Bits* ki = static_cast<const Bits*>(kin);
   Bits* ko = static_cast<Bits*>(kout);
   const V* vi = static_cast<const V*>(vin);
