@@ -163,19 +163,6 @@ __device__ __forceinline__ void block_min_max(BlockSortSmem<typename Codec<KT>::
   mx = b;
 }
 
-// The padding key of block_sort: not below any key bounded by mx.  (No float
-// has the image just below +0.0's: -0.0 shares +0.0's, and dec() of it would
-// land above mx.)
-template <int KT>
-__device__ __forceinline__ typename Codec<KT>::Bits block_pad(typename Codec<KT>::Bits mx) {
-  using Bits = typename Codec<KT>::Bits;
-  if constexpr (KT == MGS_KEY_F32 || KT == MGS_KEY_F64) {
-    constexpr Bits zero = Bits(1) << (sizeof(Bits) * 8 - 1);  // enc(+0.0)
-    if (mx == zero - 1) mx = zero - 2;
-  }
-  return Codec<KT>::dec(mx);
-}
-
 // Items per thread in use for m records, and the position of a thread's item
 // 0: wavefront w holds the positions [64 nit w, 64 nit (w + 1)), item i of a
 // lane at block_first + 64 i.
@@ -189,8 +176,9 @@ __device__ __forceinline__ uint32_t block_first(uint32_t nit) {
 }
 
 // Sorts the block's m records (1 <= m <= BLOCK * IPT) stably by enc(key) and
-// writes them to kout[0, m) (and vout).  mn and mx bound every enc(key).
-// Item slots beyond the m records hold block_pad(mx) on entry: padding
+// writes them to kout[0, m) (and vout).  mn and mx bound every enc(key); mx is
+// the image of a key, or all ones.
+// Item slots beyond the m records hold dec(mx) on entry: padding
 // behind the last record and not below any, so every pass leaves it there
 // and the passes need no bounds checks.  The counter rows are clear on entry
 // and on return; the caller puts a barrier between two calls.

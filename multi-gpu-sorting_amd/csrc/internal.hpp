@@ -6,7 +6,10 @@
 #include <algorithm>
 #include <cstddef>
 #include <cstdint>
+#include <map>
+#include <mutex>
 #include <string>
+#include <utility>
 
 #include "../../include/mgsort.h"
 
@@ -32,6 +35,27 @@ struct Marks {
     ++used;
   }
 };
+
+// Workgroups of `kernel` resident on the current device at once (the grid of a
+// persistent kernel; one per CU of an MI355X if the queries fail).  Cached per
+// (kernel, device), so that calls made while a stream is being captured into a
+// graph issue no device queries.
+template <typename K>
+uint32_t resident_blocks(K kernel, int block) {
+  constexpr uint32_t kFallback = 256;
+  static std::mutex mu;
+  static std::map<std::pair<const void*, int>, uint32_t> cache;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return kFallback;
+  const auto key = std::make_pair(reinterpret_cast<const void*>(kernel), dev);
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = cache.find(key);
+  if (it != cache.end()) return it->second;
+  int cus = 0, per_cu = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return kFallback;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, 0) != hipSuccess) return kFallback;
+  return cache[key] = (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, cus);
+}
 
 // Checks the launch(es) just enqueued.
 inline int check_launch() { return record_hip(hipGetLastError()); }

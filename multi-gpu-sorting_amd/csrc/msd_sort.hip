@@ -42,8 +42,6 @@
 // Every kernel of the path checks the decision word first; when the path is
 // off, they return at once and the LSD sort, launched after them, runs.
 #include <cstdlib>
-#include <map>
-#include <mutex>
 
 #include "internal.hpp"
 #include "msd_pass.hpp"
@@ -540,30 +538,6 @@ uint32_t env_u32(const char* name, uint32_t dflt) {
   return dflt;
 }
 
-// Workgroups of one msd kernel resident on the device (one per CU for the
-// pass kernels); cached per (kernel, device) so that graph capture issues
-// no queries.
-template <typename K>
-uint32_t msd_resident(K kernel) {
-  static std::mutex mu;
-  static std::map<std::pair<const void*, int>, uint32_t> cache;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  const auto key = std::make_pair(reinterpret_cast<const void*>(kernel), dev);
-  {
-    std::lock_guard<std::mutex> lock(mu);
-    auto it = cache.find(key);
-    if (it != cache.end()) return it->second;
-  }
-  int cus = 0, per_cu = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kMsdBlock, 0) != hipSuccess) return 0;
-  const uint32_t r = (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, cus);
-  std::lock_guard<std::mutex> lock(mu);
-  cache[key] = r;
-  return r;
-}
-
 }  // namespace
 
 bool msd_enabled() { return env_u32("MGS_MSD", 1) != 0; }
@@ -653,8 +627,7 @@ int msd_launch(const void* kin, void* kout, void* alt, size_t n, char* t, const 
   constexpr uint32_t kRangesPerChain = MsdCfg::kMaxChains / kXcds;
   const uint32_t chains1 = (ranges + kRangesPerChain - 1) / kRangesPerChain;
   // workgroups of the passes and the local sort: as many as are resident
-  uint32_t grid = msd_resident(msd_pass_kernel<KT, NoVal, 1, kMsdBlock, kMsdIpt, 4>);
-  grid = grid ? grid : 256u;
+  const uint32_t grid = resident_blocks(msd_pass_kernel<KT, NoVal, 1, kMsdBlock, kMsdIpt, 4>, kMsdBlock);
 
   mark(s, "msd_upfront");
   if ((reinterpret_cast<uintptr_t>(ki) % 16) == 0)

@@ -2,8 +2,6 @@
 // (msd_wide.hpp); instantiated per key type by msd_wide_*.hip.
 #pragma once
 
-#include <map>
-#include <mutex>
 #include <type_traits>
 
 #include "block_sort.hpp"
@@ -255,7 +253,7 @@ __global__ __launch_bounds__(BLOCK, 4) void local_kernel(typename Codec<KT>::Bit
     if (m == 0) continue;
     const Bits mn = high | (Bits)bt.z << low;
     const Bits mx = high | (Bits)bt.w << low | ((Bits(1) << low) - 1);
-    const Bits pad = block_pad<KT>(mx);
+    const Bits pad = Codec<KT>::dec(mx);
     const uint32_t nit = block_items<BLOCK>(m), wb = block_first<BLOCK>(nit);
     Bits k[IPT];
     VS v[IPT];
@@ -276,24 +274,6 @@ __global__ __launch_bounds__(BLOCK, 4) void local_kernel(typename Codec<KT>::Bit
     block_sort<KT, V, BLOCK, IPT>(sm, k, v, m, mn, mx, keys + bt.x, vo);
     __syncthreads();
   }
-}
-
-// Workgroups of `kernel` resident on the device; cached per (kernel, device)
-// so that graph capture issues no queries.
-template <typename K>
-uint32_t resident(K kernel, int block) {
-  static std::mutex mu;
-  static std::map<std::pair<const void*, int>, uint32_t> cache;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  const auto key = std::make_pair(reinterpret_cast<const void*>(kernel), dev);
-  std::lock_guard<std::mutex> lock(mu);
-  auto it = cache.find(key);
-  if (it != cache.end()) return it->second;
-  int cus = 0, per_cu = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 256;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, 0) != hipSuccess) return 256;
-  return cache[key] = (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, cus);
 }
 
 }  // namespace wide
@@ -346,7 +326,7 @@ int wide_launch(const void* kin, void* kout, void* kalt, const void* vin, void* 
   a.counters = at(L.counters) + kRadix;
   a.parity = 0;
   // (every chain has a home workgroup when the chains are not XCD-local)
-  pass1<<<std::max(std::min(wide::resident(pass1, Cfg::kBlock), P.tiles), P.chains1), Cfg::kBlock, 0, s>>>(a);
+  pass1<<<std::max(std::min(resident_blocks(pass1, Cfg::kBlock), P.tiles), P.chains1), Cfg::kBlock, 0, s>>>(a);
   mark(s, "wide_pass2");
   a.src = static_cast<const Bits*>(kalt);
   a.dst = static_cast<Bits*>(kout);
@@ -360,11 +340,11 @@ int wide_launch(const void* kin, void* kout, void* kalt, const void* vin, void* 
   a.batch_cnt = at(L.batch_cnt);
   a.batch_base = at(L.batch_base);
   a.batches = reinterpret_cast<uint4*>(t + L.batches);
-  pass2<<<wide::resident(pass2, Cfg::kBlock), Cfg::kBlock, 0, s>>>(a);
+  pass2<<<resident_blocks(pass2, Cfg::kBlock), Cfg::kBlock, 0, s>>>(a);
   mark(s, "wide_local");
   constexpr int LB = 512, LI = Cfg::kLocalIpt;
   auto local = wide::local_kernel<KT, V, LB, LI>;
-  local<<<wide::resident(local, LB), LB, 0, s>>>(static_cast<Bits*>(kout), static_cast<V*>(vout), ctl,
+  local<<<resident_blocks(local, LB), LB, 0, s>>>(static_cast<Bits*>(kout), static_cast<V*>(vout), ctl,
                                                  reinterpret_cast<const uint4*>(t + L.batches), at(L.counters),
                                                  at(L.bucket_start), P.chains1, a.ranges_per_chain * P.range_keys, nn,
                                                  (uint32_t)Cfg::kTile, status);

@@ -412,7 +412,7 @@ __global__ __launch_bounds__(kMwBlock, MwCfg<Bits>::kWaves) void mw_piece_kernel
   const uint32_t cnt = readfirstlane(bnd[k]);
   if (cnt == 0) return;
   const uint32_t nit = block_items<kMwBlock>(cnt), wb = block_first<kMwBlock>(nit);
-  const Bits pad = block_pad<KT>(mx);
+  const Bits pad = Codec<KT>::dec(mx);
   Bits key[kIpt];
   uint32_t none[kIpt];
   // the slice of the thread's first slot (last j with bnd[j] <= wb), then on

@@ -18,34 +18,6 @@ constexpr uint32_t kLookbackSpinLimit = MGS_LB_SPIN_LIMIT;
 #define MGS_PASS_LB_WINDOW 2
 #endif
 
-// The segmented kernels rank and count with the uniform-digit path (the
-// lanes of a wavefront that share the first lane's digit take one atomic)
-// unless MGS_SEG_UNI=0: measured on 4096 arrays of u64 keys + u32 payload,
-// it costs 1.7% on uniform keys and saves 35% on keys with 1000 distinct
-// values.
-#ifndef MGS_SEG_UNI
-#define MGS_SEG_UNI 1
-#endif
-constexpr bool kSegUni = MGS_SEG_UNI != 0;
-// The segment histograms (every byte of every key counted once) count with
-// MGS_SEG_HIST_UNI = 0: one atomic per key; 1: lds_count<true> (digit
-// groups); 2: lds_count_wave (one atomic for a wavefront that shares one
-// counter).
-#ifndef MGS_SEG_HIST_UNI
-#define MGS_SEG_HIST_UNI 2
-#endif
-__device__ __forceinline__ void seg_hist_count(uint32_t* c, uint32_t i) {
-  if constexpr (MGS_SEG_HIST_UNI == 2)
-    lds_count_wave(c, i);
-  else
-    lds_count<MGS_SEG_HIST_UNI != 0>(c, i);
-}
-#ifdef MGS_RANK_PEERS
-#define MGS_SEG_RANK(d, peers, cnt) rank_wave((d), (peers), (cnt))
-#else
-#define MGS_SEG_RANK(d, peers, cnt) rank_wave_atomic<kSegUni>((d), (cnt))
-#endif
-
 constexpr int kPassWindow = MGS_PASS_LB_WINDOW;
 
 // Issues the loads of the descriptors of predecessor tiles t, t-1, ...,

@@ -1,8 +1,6 @@
 // Onesweep LSD radix sort kernels and their launch sequence (see
 // radix_sort.hpp for the algorithm outline).
 #include <cstdlib>
-#include <map>
-#include <mutex>
 #include <type_traits>
 #include <utility>
 
@@ -762,7 +760,7 @@ __global__ __launch_bounds__(BLOCK) void small_sort_kernel(const typename Codec<
   }
   Bits mn, mx;
   block_min_max<KT, V, BLOCK, IPT>(sm, k, wb, n, nit, mn, mx);
-  const Bits pad = block_pad<KT>(mx);
+  const Bits pad = Codec<KT>::dec(mx);
   static_for<IPT>([&](auto i) { k[i] = wb + i * kWave < n ? k[i] : pad; });
   block_sort<KT, V, BLOCK, IPT>(sm, k, v, n, mn, mx, k_out, v_out);
 }
@@ -931,30 +929,6 @@ size_t sort_bytes(size_t n, bool wide) {
   return b;
 }
 
-// Workgroups of `kernel` that fit on the current device at once (persistent
-// grid).  Cached per (kernel, device), so that calls made while a stream is
-// being captured into a graph issue no device queries.
-template <typename K>
-uint32_t resident_blocks(K kernel, int block, size_t dyn_lds) {
-  static std::mutex mu;
-  static std::map<std::pair<const void*, int>, uint32_t> cache;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  const auto key = std::make_pair(reinterpret_cast<const void*>(kernel), dev);
-  {
-    std::lock_guard<std::mutex> lock(mu);
-    auto it = cache.find(key);
-    if (it != cache.end()) return it->second;
-  }
-  int cus = 0, per_cu = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, dyn_lds) != hipSuccess) return 0;
-  const uint32_t r = (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, cus);
-  std::lock_guard<std::mutex> lock(mu);
-  cache[key] = r;
-  return r;
-}
-
 template <int KT, int VT, bool BIG>
 int sort_typed_cfg(const void* kin, void* kout, const void* vin, void* vout, size_t n, void* temp, size_t temp_bytes,
                    hipStream_t s, Marks& mark) {
@@ -1058,8 +1032,7 @@ int sort_typed_cfg(const void* kin, void* kout, const void* vin, void* vout, siz
   uint32_t* carry = reinterpret_cast<uint32_t*>(t + L.carry);
   PassRound rd{0, L.tpr, (int)L.rounds, nullptr, nullptr};
   auto launch_pass = [&](auto kernel, auto* dsc, int p) {
-    const uint32_t res = resident_blocks(kernel, Cfg::kBlock, 0);
-    uint32_t grid = std::min<uint32_t>(L.num_tiles, res ? res : L.num_tiles);
+    uint32_t grid = std::min<uint32_t>(L.num_tiles, resident_blocks(kernel, Cfg::kBlock));
     grid = std::max<uint32_t>(grid, cm.chains);  // every chain has a home workgroup
     kernel<<<grid, Cfg::kBlock, 0, s>>>(ki, ka, ko, vi, va, vo, (uint32_t)n, p, aliased, cm, red, hist, counters,
                                         dsc, status, spin_limit, gate, rd);

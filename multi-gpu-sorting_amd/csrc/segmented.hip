@@ -41,8 +41,6 @@
 // workgroup for each middle one: u64 + u32, 1024 segments of 2^8 to 2^22, 26.3
 // -> 12.3 ms; u32, 256 ranges of 2^10 to 2^18, 331 -> 166 us; f64, normal, 64
 // of 2^10 to 2^22, 2518 -> 752 us.
-#include <map>
-#include <mutex>
 #include <type_traits>
 
 #include "block_sort.hpp"
@@ -254,14 +252,7 @@ __device__ void medium_sort_block(const typename Codec<KT>::Bits* k_in, typename
   constexpr bool HV = kHasVal<V>;
   constexpr int P = (int)sizeof(Bits);
   using VS = typename std::conditional<HV, V, uint32_t>::type;
-  struct RankSmem {
-    uint64_t peers[W][kRadix];
-  };
-  union StageSmem {
-    RankSmem r;
-    Bits keys[TILE];
-  };
-  __shared__ StageSmem u;
+  __shared__ Bits keys[TILE];
   __shared__ VS vstage[HV ? TILE : 1];
   __shared__ uint32_t off[W][kRadix];
   __shared__ uint32_t hist[P][kRadix];
@@ -279,7 +270,7 @@ __device__ void medium_sort_block(const typename Codec<KT>::Bits* k_in, typename
   for (uint32_t i = tid; i < n; i += BLOCK) {
     const Bits k = k_in[i];
 #pragma unroll
-    for (int p = 0; p < P; ++p) seg_hist_count(&hist[0][0], p * kRadix + digit_of<KT>(k, 8 * p));
+    for (int p = 0; p < P; ++p) lds_count_wave(&hist[0][0], p * kRadix + digit_of<KT>(k, 8 * p));
   }
   __syncthreads();
   if (k_in == k_out) {  // one key in all places: in order
@@ -306,10 +297,7 @@ __device__ void medium_sort_block(const typename Codec<KT>::Bits* k_in, typename
       if (tid < kRadix) run[tid] = e;
     }
     for (uint32_t tb = 0; tb < n; tb += TILE) {
-      for (int i = tid; i < W * kRadix; i += BLOCK) {
-        (&u.r.peers[0][0])[i] = 0;
-        (&off[0][0])[i] = 0;
-      }
+      for (int i = tid; i < W * kRadix; i += BLOCK) (&off[0][0])[i] = 0;
       __syncthreads();
       const uint32_t tile_cnt = min((uint32_t)TILE, n - tb);
       Bits key[IPT];
@@ -325,7 +313,7 @@ __device__ void medium_sort_block(const typename Codec<KT>::Bits* k_in, typename
       }
 #pragma unroll
       for (int k = 0; k < IPT; ++k)
-        if (wb + k * kWave < n) rk[k] = MGS_SEG_RANK(dg[k], u.r.peers[w], off[w]);
+        if (wb + k * kWave < n) rk[k] = rank_wave_atomic<true>(dg[k], off[w]);
       __syncthreads();
       uint32_t total = 0;
       if (tid < kRadix) {
@@ -349,7 +337,7 @@ __device__ void medium_sort_block(const typename Codec<KT>::Bits* k_in, typename
       for (int k = 0; k < IPT; ++k) {
         const uint32_t pos = off[w][dg[k]] + rk[k];
         if (wb + k * kWave < n && pos < (uint32_t)TILE) {
-          u.keys[pos] = key[k];
+          keys[pos] = key[k];
           if constexpr (HV) vstage[pos] = val[k];
         }
       }
@@ -358,7 +346,7 @@ __device__ void medium_sort_block(const typename Codec<KT>::Bits* k_in, typename
       for (int j = 0; j < IPT; ++j) {
         const uint32_t i = (uint32_t)(j * BLOCK + tid);
         if (i < tile_cnt) {
-          const Bits kk = u.keys[i];
+          const Bits kk = keys[i];
           const uint32_t o = gbase[digit_of<KT>(kk, shift)] + i;
           if (o < n) {
             dst[o] = kk;
@@ -1093,7 +1081,7 @@ __global__ __launch_bounds__(BLOCK, WAVES) void seg_local_kernel(const typename 
     }
     Bits mn, mx;
     block_min_max<KT, V, BLOCK, IPT>(sm, k, wb, m, nit, mn, mx);
-    const Bits pad = block_pad<KT>(mx);
+    const Bits pad = Codec<KT>::dec(mx);
     static_for<IPT>([&](auto i) { k[i] = wb + i * kWave < m ? k[i] : pad; });
     block_sort<KT, V, BLOCK, IPT>(sm, k, v, m, mn, mx, k_out + ob, vo);
     __syncthreads();
@@ -1221,24 +1209,6 @@ inline size_t segment_bound(size_t max_total, const mgs_tuning* tuning) {
 
 inline int large_variant_of(const mgs_tuning* tuning) { return tuning != nullptr ? tuning->large_variant : 0; }
 
-// Workgroups of `kernel` resident on the device; cached per (kernel, device)
-// so that graph capture issues no queries.
-template <typename K>
-uint32_t seg_resident(K kernel, int block) {
-  static std::mutex mu;
-  static std::map<std::pair<const void*, int>, uint32_t> cache;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  const auto key = std::make_pair(reinterpret_cast<const void*>(kernel), dev);
-  std::lock_guard<std::mutex> lock(mu);
-  auto it = cache.find(key);
-  if (it != cache.end()) return it->second;
-  int cus = 0, per_cu = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 256;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, 0) != hipSuccess) return 256;
-  return cache[key] = (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, cus);
-}
-
 template <int KT, int VT>
 int seg_typed(const void* kin, void* kout, const void* vin, void* vout, const uint64_t* bounds, bool ranges,
               const uint64_t* val_begin, size_t nseg, size_t max_total, const mgs_tuning* tuning, void* temp, size_t temp_bytes, hipStream_t s) {
@@ -1298,7 +1268,7 @@ int seg_typed(const void* kin, void* kout, const void* vin, void* vout, const ui
     const uint64_t* dp = to_alt ? tab.alt : tab.begin;
     const uint64_t* dvp = to_alt ? tab.alt : tab.vbegin;
     auto count = seg_count_kernel<KT>;
-    count<<<std::min(L.tiles_ub[l], seg_resident(count, kCountBlock)), kCountBlock, 0, s>>>(
+    count<<<std::min(L.tiles_ub[l], resident_blocks(count, kCountBlock)), kCountBlock, 0, s>>>(
         ks, tab, sp, nodes[l], rows, tile, C::kCap, ctl, l, L.levels - l, l == 0 ? whole : 0u);
     if (chunks != nullptr)
       seg_chunk_kernel<<<std::min(L.tiles_ub[l] / kChunk + 1, 2048u), kRadix, 0, s>>>(nodes[l], rows, chunks, ctl, l);
@@ -1312,7 +1282,7 @@ int seg_typed(const void* kin, void* kout, const void* vin, void* vout, const ui
       seg_scan_kernel<1><<<std::min(L.nodes_ub[l], 2048u), kRadix, 0, s>>>(nodes[l], rows, chunks, tile, C::kCap, from, to, last ? 1 : 0,
                                                                          last ? nullptr : nodes[l + 1], batches, longs,
                                                                          ctl, l);
-    scatter<<<std::min(L.tiles_ub[l], seg_resident(scatter, block)), block, 0, s>>>(
+    scatter<<<std::min(L.tiles_ub[l], resident_blocks(scatter, block)), block, 0, s>>>(
         ks, vs, to_alt ? ka : ko, to_alt ? va : vo, sp, svp, dp, dvp, nodes[l], rows, chunks, ctl, l);
   };
   if (max_seg > small_max) {
@@ -1336,11 +1306,11 @@ int seg_typed(const void* kin, void* kout, const void* vin, void* vout, const ui
     }
     using MC = typename C::M;
     auto lng = seg_long_kernel<KT, V, MC::kBlock, MC::kIpt>;
-    lng<<<std::min<uint32_t>((uint32_t)(max_total / (C::kCap + 1) + 1), seg_resident(lng, MC::kBlock)), MC::kBlock, 0, s>>>(
+    lng<<<std::min<uint32_t>((uint32_t)(max_total / (C::kCap + 1) + 1), resident_blocks(lng, MC::kBlock)), MC::kBlock, 0, s>>>(
         ka, ko, va, vo, tab, longs, ctl);
   }
   auto local = seg_local_kernel<KT, V, C::kLocalBlock, C::kLocalIpt, C::kLocalWaves>;
-  local<<<std::min(L.batches_ub, seg_resident(local, C::kLocalBlock)), C::kLocalBlock, 0, s>>>(ki, ka, ko, vi, va, vo, tab,
+  local<<<std::min(L.batches_ub, resident_blocks(local, C::kLocalBlock)), C::kLocalBlock, 0, s>>>(ki, ka, ko, vi, va, vo, tab,
                                                                                            batches, ctl);
   return check_launch();
 }
