@@ -148,9 +148,11 @@ int mgs_sort_timed(mgs_key kt, mgs_val vt,
  * arguments and this temp buffer used (no reference counterpart): waits for
  * `stream` and returns MGS_PATH_SMALL (one workgroup in LDS), MGS_PATH_SPLIT
  * (the segmented sort's splits, for one array; below 2^23 records, 4-byte
- * integers alone below 2^22, doubles below 2^27.6 to 2^28.6),
- * MGS_PATH_LSD (onesweep LSD passes) or MGS_PATH_THREE_PASS (the MSD pass, the bucket pass and the LDS sort of
- * sub-buckets, tried for 4-byte keys alone of 2^23 to 3 * 2^24 keys and of
+ * integers alone below 2^22, with payloads not from 2^16 to 3 * 2^17 and with
+ * u64 payloads below 9 * 2^17, floats with payloads not from 13 * 2^15 to
+ * 5 * 2^18, doubles below 2^27.6 to 2^28.6),
+ * MGS_PATH_LSD (onesweep LSD passes) or MGS_PATH_THREE_PASS (the MSD pass,
+ * the bucket pass and the LDS sort of sub-buckets, tried for 4-byte keys alone of 2^23 to 3 * 2^24 keys and of
  * 2^29 keys and more, for 8-byte integer keys from 2^23 and 4-byte integer
  * keys with payloads from 2^24 records up to about 2^28; it hands over to the
  * LSD passes when the key distribution does not suit it), or a negative

@@ -843,6 +843,11 @@ bool mid_path(int kb, int vb, bool floats, size_t n) {
   // 2^22 177 / 158)
   if (kb == 4 && vb > 0 && !floats && n >= (size_t(1) << 16) && n < (size_t(3) << 17)) return false;
   if (kb == 4 && vb == 8 && !floats && n >= (size_t(9) << 17)) return false;
+  // 4-byte floats with payloads: their exponents take a second level from about
+  // 2^18.7 on, which pays off above 2^20.3 (f32 + u32 uniform 2^18.6 52 / 75,
+  // 2^19 86 / 66, 2^20 87 / 90, 2^21 115 / 168; normal 2^19 92 / 63, 2^20 104 / 85,
+  // 2^21 119 / 150; + u64 normal 2^19 94 / 66)
+  if (kb == 4 && vb > 0 && floats && n >= (size_t(13) << 15) && n < (size_t(5) << 18)) return false;
   for (const char* name : kForcing)
     if (std::getenv(name) != nullptr) return false;
   return true;

@@ -22,8 +22,8 @@ def mg():
 
 def tied_keys(kt, n, rng, dist):
     """uniform; pairs: every key about twice; clustered: 5 far apart values
-    plus small offsets, so that the top 18 differing bits leave long groups in
-    disorder; lone: clustered with one key at the bottom of the range."""
+    plus small offsets, so that in 8-byte keys the top 27 differing bits leave
+    long groups in disorder; lone: clustered with one key at the bottom of the range."""
     if dist == "uniform":
         return random_keys(kt, n, rng)
     bd = O.BITS_DTYPE[kt]
@@ -423,10 +423,12 @@ def test_crowded_windows(mg, kt, dist, n):
 @pytest.mark.parametrize("kt,vdt,n,path", [(O.K_U32, np.uint32, (1 << 16) - 1, 4), (O.K_I32, np.uint32, 1 << 16, 2),
                                            (O.K_I32, np.uint64, (3 << 17) - 1, 2), (O.K_U32, np.uint64, 3 << 17, 4),
                                            (O.K_U32, np.uint64, (9 << 17) - 1, 4), (O.K_I32, np.uint64, 9 << 17, 2),
-                                           (O.K_U32, np.uint32, 9 << 17, 4), (O.K_F32, np.uint32, 1 << 16, 4),
+                                           (O.K_U32, np.uint32, 9 << 17, 4), (O.K_F32, np.uint32, (13 << 15) - 1, 4),
+                                           (O.K_F32, np.uint64, 13 << 15, 2), (O.K_F32, np.uint32, (5 << 18) - 1, 2),
+                                           (O.K_F32, np.uint64, 5 << 18, 4),
                                            (O.K_U32, None, 1 << 16, 4)], ids=lambda v: str(v))
-def test_integer_pairs_between_splits(mg, kt, vdt, n, path):
-    """4-byte integer keys with payloads on both sides of the sizes that the LSD
-    passes sort faster than splits."""
+def test_pairs_between_splits(mg, kt, vdt, n, path):
+    """4-byte keys with payloads on both sides of the sizes that the LSD passes
+    sort faster than splits."""
     rng = np.random.default_rng(n)
     assert run_sort(mg, kt, vdt, random_keys(kt, n, rng), rng, inplace=False) == path
