@@ -12,9 +12,10 @@
 //            that one workgroup sorts
 //   pass 1   scatter by the window's high byte, 8 chains of tiles
 //   pass 2   scatter by its low byte inside each of the 256 buckets
-//   local    every batch is sorted in LDS by its bits below the window
-//            (block_sort.hpp: two passes over the top 18 of them and a
-//            look at the neighbours) and written back in place
+//   local    every batch is sorted in LDS by its bits below the window and
+//            those in which its sub-buckets differ (block_sort.hpp: up to three
+//            passes over the top 27 of them and a look at the neighbours) and
+//            written back in place
 //
 // A sub-bucket that does not fit a workgroup, a key outside the sample's
 // shared leading bits, a window counter that overflowed or one XCD's buckets

@@ -15,8 +15,8 @@
 //             for j' < j, lower bound for j' > j, exactly i for j' = j
 //   base      each boundary's output position (the sum of its splits)
 //   piece     one workgroup per piece: its slices of the k runs, laid end to
-//             end in run order, sorted stably in LDS (block_sort.hpp: two
-//             radix passes whatever k is), which is their stable merge; or,
+//             end in run order, sorted stably in LDS (block_sort.hpp: two or
+//             three radix passes whatever k is), which is their stable merge; or,
 //             for up to 8 runs of 8-byte keys, merged by a tree of LDS
 //             merge-path rounds (adjacent slices, earlier runs first on ties)
 //
@@ -40,13 +40,15 @@ namespace {
 
 // Pieces sorted by radix passes: 8192 4-byte keys in 49 KB of LDS, three
 // workgroups of 512 threads per CU; 6144 8-byte keys in 66 KB, two.  The
-// passes are bound by the LDS (61% of the cycles, 58% of these in bank
-// conflicts of the random counters and positions) and by how far other
+// passes are bound by the LDS (62% of the cycles, half of these in bank
+// conflicts of the random counters and positions), the vector instructions (74%:
+// profiles/counters_by_kernel.txt) and by how far other
 // workgroups fill the gaps between barriers: 1024-thread workgroups of as
 // many keys measured 1.25 times slower, as did 16384 keys per piece.
 // Measured, whole call, against the merge tree: u32, 8 runs of 2^26 2.81 ->
-// 1.85 ms, 16 x 2^24 2.02 -> 1.13 ms, 64 x 2^22 3.6 -> 1.7 ms, 256 x 2^20
-// 6.7 -> 3.2 ms.
+// 1.82 ms, 16 x 2^24 2.02 -> 1.13 ms, 64 x 2^22 3.6 -> 1.7 ms, 256 x 2^20
+// 6.7 -> 3.2 ms; small merges of few runs were faster by the tree (4 x 2^22 147
+// against 161 us).
 constexpr int kMwBlock = 512;
 template <typename Bits>
 struct MwCfg {

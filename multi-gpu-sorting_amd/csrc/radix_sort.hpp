@@ -165,17 +165,21 @@ template <int KB, int VB> struct SmallCfg {
 };
 
 // Arrays below this length sort by one workgroup or by splits (mid_path).
-// LSD passes against splits: u64 2^14 85 us against 47, 2^20 166 against 83,
-// 2^22 290 against 159; f64 + u32 just below 2^23 529 against 308; f32 there
-// 231 against 193; u32 + u32 246 against 228.  u32 alone, whose four passes
-// move the least: 2^20 104 against 79, 2^22 145 against 136, but 194 against
-// 204 just below 2^23.
+// LSD passes against splits, uniform keys: u64 2^15 87 us against 50, 2^20 155
+// against 58, 2^22 287 against 158; f64 + u32 just below 2^23 529 against 303; f32
+// there 229 against 195 (normal: 207 against 235); u32 + u32 246 against 227 (zipf
+// 318 against 231).  u32 alone, whose four passes move the least: 2^20 104 against 49,
+// 2^22 141 against 135, but 194 against 204 just below 2^23.  Integers of which the
+// passes skip bytes are slower by splits, which move them twice or three times
+// whatever they are: u64 of 16 bits 2^23 173 us against 227, row numbers 301
+// against 334.
 // Doubles, which the three-pass path does not take, sort by splits as long as
 // two levels leave the local sort an eighth of room (uniform keys; 2^28.6,
 // 2^28.1 and 2^27.6 records of 8, 12 and 16 bytes): f64 normal 2^24 780 us
-// against 617, 2^28 8.95 ms against 7.82, 2^28.7 14.1 against 14.4; f64 + u32
-// uniform 2^26 3.08 ms against 1.92, normal 2^28 11.7 against 11.0; f64 + u64
-// normal 2^27 7.6 ms against 6.1, 2^27.7 11.9 against 11.8.
+// against 595, 2^28 8.92 ms against 7.34, 2^28.5 12.3 against 10.7; f64 + u32
+// 2^28 11.7 against 9.6, f64 + u64 2^27.5 10.5 against 8.5; none of ten
+// distributions is slower there (1 - eps 2^28.5 14.9 against 9.8, counts 5.5
+// against 4.6, one value 1.87 against 1.85).
 inline size_t mid_max(int kb, int vb, bool floats) {
   if (kb == 8 && floats) return (size_t)split_local_cap(kb, vb) * (254 * 254 / 8 * 7);
   return size_t(1) << (kb + vb <= 4 && !floats ? 22 : 23);

@@ -32,11 +32,11 @@
 // a payload takes one to two levels and the local sort instead of eight LSD
 // passes.  Bounds from the sample divide keys of any distribution into children
 // of at most about a fortieth, so the levels bring them to what one workgroup
-// sorts in LDS up to chance: on 868 calls of 23 distributions one child in
-// thousands was left, a little above it.  (Inputs made against the sample's fixed
-// places may leave long ones: 6 to 9 ns a record of 8-byte keys each.)  With
-// equal steps alone, log-uniform u64 keys left 61% of 2^23 records to one
-// workgroup: 45.6 ms, now 0.30; 2^26 doubles 1 - eps 336 ms, now 1.9.
+// sorts in LDS up to chance: of 868 calls with 23 distributions one left children,
+// two (49 us).  (Inputs made against the sample's fixed places may leave long ones:
+// one workgroup takes 6 to 9 ns a record of 8-byte keys.)  With equal steps alone,
+// log-uniform u64 keys left 61% of 2^23 records to one workgroup: 45.6 ms, now 0.28;
+// 2^26 doubles 1 - eps 336 ms, now 1.55.
 // Against LSD passes over all long segments at once and one
 // workgroup for each middle one: u64 + u32, 1024 segments of 2^8 to 2^22, 26.3
 // -> 12.3 ms; u32, 256 ranges of 2^10 to 2^18, 331 -> 166 us; f64, normal, 64
