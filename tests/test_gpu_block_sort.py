@@ -279,10 +279,17 @@ def skewed_keys(kt, n, rng, dist):
     magnitude equally often; zipf: small counts, 1 in 87% of the places (10%
     in 4-byte keys); near: 1 - eps over 50 orders of eps; four: four values
     2^-30, 2^-20 and 2^-10 apart; shares: 55% 0, 25% 1, 12% 2, the rest
-    spread; geometric: counts, halving; single: one value."""
+    spread; geometric: counts, halving; single: one value; ends: 40% the lowest
+    and 30% the highest key that sorts, the rest log."""
     bd = O.BITS_DTYPE[kt]
     fd = np.float32 if bd == np.uint32 else np.float64
     u = rng.random(n)
+    if dist == "ends":
+        k = skewed_keys(kt, n, rng, "log")
+        top = bd(~bd(0)) if kt in (O.K_U32, O.K_U64) else bd(~bd(0)) >> bd(1)
+        k[u < 0.3] = top  # (of floats the NaN that sorts last)
+        k[u > 0.6] = ~top
+        return k
     if dist == "log":
         x = np.exp2(u * (31 if bd == np.uint32 else 63))
     elif dist == "zipf":
@@ -306,9 +313,9 @@ def left_to_one_workgroup(temp):
     return int(from_dev(temp[12:16], np.uint32)[0])
 
 
-SKEWED = [(kt, vdt, d) for kt, vdt, ds in ((O.K_U64, None, "log zipf single"), (O.K_I32, np.uint32, "log zipf"),
-                                           (O.K_U64, np.uint64, "log zipf"), (O.K_F32, None, "near shares geometric"),
-                                           (O.K_F64, np.uint32, "near four shares geometric log single"))
+SKEWED = [(kt, vdt, d) for kt, vdt, ds in ((O.K_U64, None, "log zipf single ends"), (O.K_I32, np.uint32, "log zipf ends"),
+                                           (O.K_U64, np.uint64, "log zipf"), (O.K_F32, None, "near shares geometric ends"),
+                                           (O.K_F64, np.uint32, "near four shares geometric log single ends"))
           for d in ds.split()]
 
 
