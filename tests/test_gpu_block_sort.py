@@ -439,3 +439,49 @@ def test_pairs_between_splits(mg, kt, vdt, n, path):
     sort faster than splits."""
     rng = np.random.default_rng(n)
     assert run_sort(mg, kt, vdt, random_keys(kt, n, rng), rng, inplace=False) == path
+
+
+def sample_places(n):
+    """Where a range of n records is sampled (sort_sample in segmented.hip)."""
+    m = np.uint64(0xFFFFFFFF)
+    t = np.arange(255, dtype=np.uint64)
+    a, b = np.uint64(n) * t // np.uint64(255), np.uint64(n) * (t + np.uint64(1)) // np.uint64(255)
+    h = ((t + np.uint64(1)) * np.uint64(0x9E3779B9) & m) ^ np.uint64(n)
+    h = (h ^ (h >> np.uint64(16))) * np.uint64(0x85EBCA6B) & m
+    h = (h ^ (h >> np.uint64(13))) * np.uint64(0xC2B2AE35) & m
+    return (a + ((h ^ (h >> np.uint64(16))) * (b - a) >> np.uint64(32))).astype(np.int64)
+
+
+@pytest.mark.parametrize("kt,vdt", [(O.K_U32, None), (O.K_I32, np.uint64), (O.K_U64, np.uint32), (O.K_I64, None),
+                                    (O.K_U64, np.uint64)], ids=lambda v: str(v))
+@pytest.mark.parametrize("values", [1, 2000])
+def test_long_children(mg, kt, vdt, values):
+    """Keys made against the sample: on both levels it sees evenly spread keys
+    only, and all others lie close together, so that one child (or two, across a
+    step) is left to a workgroup that streams it; of one value, or not."""
+    import torch
+    n, bd = 90_001, O.BITS_DTYPE[kt]
+    nbits = 32 if bd == np.uint32 else 64
+    rng = np.random.default_rng(kt + values)
+    mid = np.uint64(3 << (nbits - 3))
+    k = mid + rng.integers(0, values, size=n).astype(np.uint64)
+    first = sample_places(n)
+    rest = np.setdiff1d(np.arange(n), first)
+    # the second level's range is the first's fullest step: all but its sample
+    k[rest[sample_places(rest.size)]] = mid - np.uint64(1 << 20) + np.arange(255, dtype=np.uint64) * np.uint64(1 << 13)
+    spread = np.arange(255, dtype=np.uint64) * np.uint64((1 << nbits) // 255)
+    near = np.abs(spread.astype(np.float64) - float(mid)) < 2.0**nbits / 100  # (not in that step)
+    k[first] = np.where(near, np.uint64(7), spread)
+    keys = k.astype(bd) ^ (bd(1) << bd(nbits - 1) if kt in (O.K_I32, O.K_I64) else bd(0))
+    vals = None if vdt is None else random_vals(vdt, n, rng)
+    off = np.array([0, n], dtype=np.uint64)
+    ek, ev = O.segmented_sort(kt, keys, off, vals)
+    dk, dv = to_dev(keys), to_dev(vals)
+    vt = mg.VAL_NONE if vdt is None else (mg.VAL_U32 if vdt == np.uint32 else mg.VAL_U64)
+    temp = mg.temp_buffer(mg.lib.mgs_segmented_sort_temp_bytes(kt, vt, n, 1), "cuda")
+    mg.segmented_sort(KEY_NAME[kt], dk, torch.from_numpy(off.view(np.int64)).cuda(), dv, temp=temp)
+    assert mg.temp_status(temp) == 0
+    assert left_to_one_workgroup(temp) in (1, 2)
+    assert np.array_equal(from_dev(dk, bd), ek.view(bd))
+    if vdt is not None:
+        assert np.array_equal(from_dev(dv, vdt), ev)
